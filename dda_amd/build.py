@@ -12,7 +12,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "_lib", "libdda_hip.so")
-SOURCES = ["api.hip", "matvec.hip", "krylov.hip", "observe.hip", "server.cpp"]
+# plans.hip is compiled in eight parts (DDA_PLAN_PART)
+SOURCES = ["matvec.hip"] + ["plans.hip:%d" % p for p in range(8)] + ["api.hip", "krylov.hip", "observe.hip", "server.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -23,11 +24,13 @@ FLAGS = [
 
 
 def _compile(src):
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
+    src, _, part = src.partition(":")
+    obj = os.path.join(BUILD, os.path.splitext(src)[0] + part + ".o")
+    defs = ["-DDDA_PLAN_PART=" + part] if part else []
     if src.endswith(".cpp"):  # host-only C++
         cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-Wall", "-pthread", "-c", os.path.join(SRC, src), "-o", obj]
     else:
-        cmd = [HIPCC] + FLAGS + ["-c", os.path.join(SRC, src), "-o", obj]
+        cmd = [HIPCC] + FLAGS + defs + ["-c", os.path.join(SRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     out = "\n".join(l for l in (r.stdout + r.stderr).splitlines() if "packed-fp32-ops" not in l)
     if r.returncode != 0:
@@ -48,7 +51,7 @@ def build_adapter_check():
 def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
-    with concurrent.futures.ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 1)) as ex:
         results = list(ex.map(_compile, SOURCES))
     for _, out in results:
         if out.strip() and verbose:

@@ -3,15 +3,16 @@
 // A transform of length N = R0 * R1 * ... over a tile of T adjacent columns.
 // Every thread owns PPT points of one column in every stage (PPT divisible by
 // each radix), so a stage is PPT / R butterflies per thread: butterfly
-// j_i = t + i * TPC, TPC = N / PPT threads per column. The first stage takes its
+// j_i = t + i * TPC, TPC = N / PPT threads per column (general plans, below, let
+// the threads a stage has no butterfly for sit it out). The first stage takes its
 // inputs x[j + m N / R0] from registers the caller filled (straight from HBM),
 // the last stage leaves X[j + m N / R_last] in registers, and only the stages
 // in between pass through LDS. Running the inverse with the radices reversed
 // makes its first stage consume exactly the points the forward transform left
 // in a thread's registers, so FFT -> pointwise product -> inverse FFT needs no
 // exchange in the middle. Twiddles W_{Ns R}^{m k} come from the host's table
-// of N roots of unity (one load per butterfly, then powers); the constants of
-// the in-register DFTs are evaluated at compile time.
+// of N roots of unity; the constants of the in-register DFTs are evaluated at
+// compile time.
 #pragma once
 
 #include "common.hpp"
@@ -74,7 +75,11 @@ constexpr double cexpr_trig(long long t, long long n, int which) {
 // X[k1 + P k2] = sum_q W_Q^{q k2} W_R^{q k1} sum_p a[q + Q p] W_P^{p k1}.
 // ------------------------------------------------------------------------------------
 template <int R> struct SmallFactor {
-  static constexpr int value = (R % 4 == 0 && R > 4) ? 4 : (R % 2 == 0 && R > 2) ? 2 : (R % 3 == 0 && R > 3) ? 3 : R;
+  static constexpr int value = (R % 4 == 0 && R > 4)   ? 4
+                               : (R % 2 == 0 && R > 2) ? 2
+                               : (R % 3 == 0 && R > 3) ? 3
+                               : (R % 5 == 0 && R > 5) ? 5
+                                                       : R;
 };
 
 template <int R, bool INV, typename C> struct RDft;
@@ -161,8 +166,7 @@ template <bool INV, typename C> struct RDft<5, INV, C> : RDftOdd<5, INV, C> {};
 template <bool INV, typename C> struct RDft<7, INV, C> : RDftOdd<7, INV, C> {};
 
 template <int R, bool INV, typename C> struct RDft {
-  static_assert(R == 6 || R == 8 || R == 10 || R == 12 || R == 16 || R == 20 || R == 24 || R == 32,
-                "unsupported in-register DFT length");
+  static_assert(SmallFactor<R>::value < R, "unsupported in-register DFT length");
   static __device__ inline void run(C* a) {
     constexpr int P = SmallFactor<R>::value;
     constexpr int Q = R / P;
@@ -210,20 +214,57 @@ template <int R, bool INV, typename C> struct RDftHalfIn {
   }
 };
 
+// How a stage gets its butterfly's twiddles W^m, m = 1 .. R - 1 (W^m = tw[m s],
+// tw the table of N roots of unity, each correct to half a unit in the last place):
+//   TW_CHAIN  one load, then repeated multiplication: W^m carries m times its
+//             rounding. The plans with radices up to 16 of the powers of two, the
+//             long lengths: where every load shows.
+//   TW_SPLIT  powers 1, 2, 3 and the multiples of 4 loaded, the others one product
+//             of two of those
+//   TW_HELD   powers formed once by the caller for all its transforms
+// General plans take TW_SPLIT: their radices go up to 28, whose chained powers
+// made the FP64 product at 80^3 2.1e-16 and the FP32 one at 96 x 70 x 120 9.9e-8
+// from the exact one, against 1.6e-16 and 8.1e-8 with run-time planned radices up
+// to 8; with TW_SPLIT it is 1.7e-16 and 6.5e-8, over 22 boxes of 8 to 250 cells
+// a side 0.97 (FP64) and 0.87 (FP32) of the run-time planned kernels' error.
+// Loading every power (FP64) gave no smaller error and took 22% longer at
+// 180 x 144 x 120. TW_SPLIT in the plans of the powers of two halves the FP32
+// error at 512^3 but makes their products 2 to 9% slower.
+enum TwiddleMode { TW_CHAIN = 0, TW_SPLIT = 1, TW_HELD = 2 };
+
+template <int R, typename C> struct TwiddleRow {
+  C lo[4], hi[(R + 3) / 4];
+  __device__ __forceinline__ TwiddleRow(const C* __restrict__ tw, int s) {
+#pragma unroll
+    for (int m = 1; m < 4 && m < R; m++) lo[m] = tw[m * s];
+#pragma unroll
+    for (int m = 4; m < R; m += 4) hi[m / 4] = tw[m * s];
+  }
+  // W^m, r = m mod 4
+  __device__ __forceinline__ C power(int r, int m) const {
+    if (m < 4) return lo[m];
+    return r ? cmul(hi[m / 4], lo[r]) : hi[m / 4];
+  }
+};
+
 // ------------------------------------------------------------------------------------
 // Plans
 // ------------------------------------------------------------------------------------
 template <int... Rs> struct RadixList {};
 
-// StaticPlan<N, WIDE>: PPT and the forward radix order (Fwd). WIDE plans (used
+// StaticPlan<N, WIDE>: PPT, TPC, the radix order (Fwd) and that of the single inverse
+// transforms (Bwd). WIDE plans (used
 // for complex float) hold 16 points per thread and need one LDS exchange fewer;
 // narrow plans (complex double) hold 8 to keep three components in registers.
 template <int N, bool WIDE> struct StaticPlan { static constexpr bool exists = false; };
 #define DDA_PLAN(N, W, P, ...)                            \
   template <> struct StaticPlan<N, W> {                   \
-    static constexpr bool exists = true;                  \
+    static constexpr bool exists = true, general = false; \
     static constexpr int PPT = P;                         \
+    static constexpr int TPC = N / P;                     \
     typedef RadixList<__VA_ARGS__> Fwd;                   \
+    typedef Fwd Bwd;                                      \
+    template <typename R> static constexpr int twiddles = TW_CHAIN; \
   };
 DDA_PLAN(32, false, 8, 8, 4)
 DDA_PLAN(32, true, 16, 16, 2)
@@ -249,9 +290,12 @@ DDA_PLAN(1024, true, 16, 16, 16, 4)
 // pass's long-column variants: 1024 = 32 x 32 holds 32 points per thread and
 // needs a single LDS exchange per transform).
 template <int N, int P, typename L> struct PlanOf {
-  static constexpr bool exists = true;
+  static constexpr bool exists = true, general = false;
   static constexpr int PPT = P;
+  static constexpr int TPC = N / P;
   typedef L Fwd;
+  typedef L Bwd;
+  template <typename R> static constexpr int twiddles = TW_CHAIN;
 };
 
 template <typename L> struct Reverse;
@@ -262,25 +306,62 @@ template <int R, int... Rs> struct Reverse<RadixList<R, Rs...>> {
   typedef typename Append<typename Reverse<RadixList<Rs...>>::type, R>::type type;
 };
 
-// Stage helpers. v[i * R + m] is input m of butterfly j_i = t + i * TPC. The
-// twiddle W_{NS R}^k comes from the table of N roots of unity, its powers by
-// repeated multiplication. HALF (first stage only): inputs m >= R/2 are zero
+// Butterflies of radix R that a thread of a column with TPC threads owns:
+// j_i = t + i * TPC, i < per; the last may lie beyond the stage's N / R.
+template <int N, int TPC, int R> struct Butterflies {
+  static constexpr int count = N / R;
+  static constexpr int per = (count + TPC - 1) / TPC;
+  static constexpr bool exact = per * TPC == count;
+};
+
+// A plan of radices R0, Rs... (R0 even) whose threads hold one butterfly of each
+// stage where they have one: TPC = N / (smallest radix) threads per column, so
+// that lengths such as 80 = 10 * 8 or 294 = 6 * 7 * 7 run as two or three stages
+// of nearly equal radices; in a stage of radix R, threads t >= N / R idle.
+template <int N, int R0, int... Rs> struct GenPlan {
+  static constexpr int cmin(int a) { return a; }
+  template <typename... A> static constexpr int cmin(int a, int b, A... r) { return cmin(a < b ? a : b, r...); }
+  static constexpr int cmax(int a) { return a; }
+  template <typename... A> static constexpr int cmax(int a, int b, A... r) { return cmax(a > b ? a : b, r...); }
+  static constexpr int cprod(int a) { return a; }
+  template <typename... A> static constexpr int cprod(int a, int b, A... r) { return cprod(a * b, r...); }
+  static constexpr bool exists = true, general = true;
+  static constexpr int PPT = cmax(R0, Rs...);
+  static constexpr int TPC = N / cmin(R0, Rs...);
+  typedef RadixList<R0, Rs...> Fwd;
+  typedef typename Reverse<Fwd>::type Bwd;  // ends on R0: the cropped half is never formed
+  template <typename R> static constexpr int twiddles = TW_SPLIT;
+  static_assert(R0 % 2 == 0 && cprod(R0, Rs...) == N, "radices");
+};
+
+// Stage helpers. v[i * R + m] is input m of butterfly j_i = t + i * TPC, its
+// twiddle W_{NS R}^{k m} (TwiddleRow). HALF (first stage only): inputs m >= R/2 are zero
 // and not read.
-// PRE: tw holds the R - 1 twiddle powers of the thread's one butterfly of the
-// twiddled stage (formed once by the caller and shared by all its transforms).
-template <int N, int PPT, int R, int NS, bool INV, bool HALF, typename C, bool PRE = false>
+// TW_HELD: tw holds the R - 1 twiddle powers of the thread's one butterfly of
+// the twiddled stage. Idle butterflies are computed on whatever v holds and
+// never stored.
+template <int N, int TPC, int R, int NS, bool INV, bool HALF, typename C, int TW>
 __device__ inline void stage_compute(C* v, int t, const C* __restrict__ tw) {
-  constexpr int TPC = N / PPT;
 #pragma unroll
-  for (int i = 0; i < PPT / R; i++) {
+  for (int i = 0; i < Butterflies<N, TPC, R>::per; i++) {
     C* a = v + i * R;
-    if (NS > 1 && PRE) {
+    const int j = t + i * TPC;
+    const int k = j % NS;  // NS is a compile-time constant
+    constexpr int step = N / (NS * R);
+    if constexpr (NS > 1 && TW == TW_HELD) {
 #pragma unroll
       for (int m = 1; m < R; m++) a[m] = INV ? cmulc(a[m], tw[m - 1]) : cmul(a[m], tw[m - 1]);
-    } else if (NS > 1) {
-      const int j = t + i * TPC;
-      const int k = j % NS;  // NS is a compile-time constant
-      const C w1 = tw[k * (N / (NS * R))];
+    } else if constexpr (NS > 1 && TW == TW_SPLIT) {
+      TwiddleRow<R, C> w(tw, k * step);
+#pragma unroll
+      for (int r = 0; r < 4 && r < R; r++)
+#pragma unroll
+        for (int m = r ? r : 4; m < R; m += 4) {
+          const C wm = w.power(r, m);
+          a[m] = INV ? cmulc(a[m], wm) : cmul(a[m], wm);
+        }
+    } else if constexpr (NS > 1) {
+      const C w1 = tw[k * step];
       C w = w1;
 #pragma unroll
       for (int m = 1; m < R; m++) {
@@ -288,20 +369,32 @@ __device__ inline void stage_compute(C* v, int t, const C* __restrict__ tw) {
         if (m + 1 < R) w = cmul(w, w1);
       }
     }
-    if (HALF && NS == 1)
+    if constexpr (HALF && NS == 1)
       RDftHalfIn<R, INV, C>::run(a);
     else
       RDft<R, INV, C>::run(a);
   }
 }
 
-// Writes the stage outputs to the tile at their Stockham positions.
-template <int N, int PPT, int R, int NS, typename C>
-__device__ inline void stage_store(const C* v, int t, C* tile, int lp, int l) {
-  constexpr int TPC = N / PPT;
+// Forms v[0 .. K) here: the compiler does not defer it to a later use.
+template <int K, typename C> __device__ __forceinline__ void keep_here(C* v) {
 #pragma unroll
-  for (int i = 0; i < PPT / R; i++) {
+  for (int m = 0; m < K; m++) asm volatile("" : "+v"(v[m].x), "+v"(v[m].y));
+}
+
+// Writes the stage outputs to the tile at their Stockham positions.
+template <int N, int TPC, int R, int NS, typename C>
+__device__ inline void stage_store(C* v, int t, C* tile, int lp, int l) {
+  typedef Butterflies<N, TPC, R> B;
+#pragma unroll
+  for (int i = 0; i < B::per; i++) {
     const int j = t + i * TPC;
+    if constexpr (!B::exact) {
+      // (formed before the branch: the compiler would move into it all that
+      // leads to them)
+      keep_here<R>(v + i * R);
+      if (j >= B::count) continue;
+    }
     const int q = j / NS, k = j % NS;
     const int base = q * NS * R + k;
 #pragma unroll
@@ -309,13 +402,15 @@ __device__ inline void stage_store(const C* v, int t, C* tile, int lp, int l) {
   }
 }
 
-// Reads the inputs of a stage of radix R from the tile.
-template <int N, int PPT, int R, typename C>
+// Reads the inputs of a stage of radix R from the tile (an idle butterfly reads
+// butterfly 0's: no branch, which would keep v out of registers).
+template <int N, int TPC, int R, typename C>
 __device__ inline void stage_load(C* v, int t, const C* tile, int lp, int l) {
-  constexpr int TPC = N / PPT;
+  typedef Butterflies<N, TPC, R> B;
 #pragma unroll
-  for (int i = 0; i < PPT / R; i++) {
-    const int j = t + i * TPC;
+  for (int i = 0; i < B::per; i++) {
+    int j = t + i * TPC;
+    if (!B::exact) j = j < B::count ? j : 0;
 #pragma unroll
     for (int m = 0; m < R; m++) v[i * R + m] = tile[(j + m * (N / R)) * lp + l];
   }
@@ -327,56 +422,75 @@ __device__ inline void stage_load(C* v, int t, const C* tile, int lp, int l) {
 // any exchange happened, so the caller may reuse the tile. HALF: the upper half
 // of every first-stage butterfly's inputs is zero (a zero-padded transform of
 // at most N/2 points) and is neither read nor computed with.
-// PRE (two-stage plans with one butterfly per thread per stage, see
-// TwoStage): tw is the thread's R2 - 1 second-stage twiddle powers.
-template <int N, int PPT, bool INV, int NS, typename C, typename L, bool HALF = false, bool PRE = false>
+// TW: the twiddles' TwiddleMode; TW_HELD for two-stage plans with one butterfly
+// per thread per stage (TwoStage), tw the thread's second-stage powers.
+template <int N, int TPC, bool INV, int NS, typename C, typename L, bool HALF = false, int TW = TW_CHAIN>
 struct RunStages;
 
-template <int N, int PPT, bool INV, int NS, typename C, int R, bool HALF, bool PRE>
-struct RunStages<N, PPT, INV, NS, C, RadixList<R>, HALF, PRE> {
+template <int N, int TPC, bool INV, int NS, typename C, int R, bool HALF, int TW>
+struct RunStages<N, TPC, INV, NS, C, RadixList<R>, HALF, TW> {
   static __device__ inline void run(C* v, int t, C* tile, int lp, int l, const C* tw) {
-    stage_compute<N, PPT, R, NS, INV, HALF, C, PRE>(v, t, tw);
+    stage_compute<N, TPC, R, NS, INV, HALF, C, TW>(v, t, tw);
   }
 };
 
-template <int N, int PPT, bool INV, int NS, typename C, int R, int R2, int... Rs, bool HALF, bool PRE>
-struct RunStages<N, PPT, INV, NS, C, RadixList<R, R2, Rs...>, HALF, PRE> {
+template <int N, int TPC, bool INV, int NS, typename C, int R, int R2, int... Rs, bool HALF, int TW>
+struct RunStages<N, TPC, INV, NS, C, RadixList<R, R2, Rs...>, HALF, TW> {
   static __device__ inline void run(C* v, int t, C* tile, int lp, int l, const C* tw) {
-    stage_compute<N, PPT, R, NS, INV, HALF, C, PRE>(v, t, tw);
-    stage_store<N, PPT, R, NS>(v, t, tile, lp, l);
+    stage_compute<N, TPC, R, NS, INV, HALF, C, TW>(v, t, tw);
+    stage_store<N, TPC, R, NS>(v, t, tile, lp, l);
     __syncthreads();
-    stage_load<N, PPT, R2>(v, t, tile, lp, l);
+    stage_load<N, TPC, R2>(v, t, tile, lp, l);
     __syncthreads();
-    RunStages<N, PPT, INV, NS * R, C, RadixList<R2, Rs...>, false, PRE>::run(v, t, tile, lp, l, tw);
+    RunStages<N, TPC, INV, NS * R, C, RadixList<R2, Rs...>, false, TW>::run(v, t, tile, lp, l, tw);
   }
 };
 
-// Plans of two stages with PPT = R0 = R1 (a thread holds one butterfly of
-// each stage; its second-stage twiddles are W_N^(t m), m = 1 .. R1 - 1, the
-// same for the forward and the conjugated inverse transform).
-template <int N, int PPT, typename L> struct TwoStage { static constexpr bool value = false; };
-template <int N, int PPT, int R0, int R1> struct TwoStage<N, PPT, RadixList<R0, R1>> {
-  static constexpr bool value = PPT == R0 && PPT == R1 && R0 * R1 == N;
+// Plans of two stages with one butterfly of each per thread: the thread's
+// second-stage twiddles are W_N^(t m), m = 1 .. R1 - 1, in the forward transform
+// and, conjugated, W_N^(t m), m = 1 .. R0 - 1, in the inverse, whose radices run
+// the other way round.
+template <int N, int TPC, typename L> struct TwoStage { static constexpr bool value = false; };
+template <int N, int TPC, int R0, int R1> struct TwoStage<N, TPC, RadixList<R0, R1>> {
+  static constexpr bool value = R0 * R1 == N && TPC == (R0 > R1 ? R0 : R1);
 };
-template <int R, typename C>
+// W_N^(t m), m = 1 .. K (t < N), formed as MODE says
+template <int K, int MODE, typename C>
 __device__ inline void twiddle_powers(C* wp, int t, const C* __restrict__ tw) {
-  const C w1 = tw[t % R];
-  C w = w1;
+  if constexpr (MODE == TW_CHAIN) {
+    const C w1 = tw[t];
+    C w = w1;
 #pragma unroll
-  for (int m = 0; m < R - 1; m++) {
-    wp[m] = w;
-    if (m + 2 < R) w = cmul(w, w1);
+    for (int m = 0; m < K; m++) {
+      wp[m] = w;
+      if (m + 1 < K) w = cmul(w, w1);
+    }
+  } else {
+    TwiddleRow<K + 1, C> w(tw, t);
+#pragma unroll
+    for (int m = 1; m <= K; m++) wp[m - 1] = w.power(m % 4, m);
   }
 }
 
 template <typename L> struct FirstRadix;
 template <int R, int... Rs> struct FirstRadix<RadixList<R, Rs...>> { static constexpr int value = R; };
 
-// Point index held in v[e] for the first stage of plan L (e = i * R0 + m).
-template <int N, int PPT, typename L>
+// Registers v[0 .. first_count) that the first stage of plan L uses, and the
+// point index held in v[e] (e = i * R0 + m). With idle butterflies a thread's
+// point may not be its own: first_ok says whether it is.
+template <int N, int TPC, typename L>
+__device__ __forceinline__ constexpr int first_count() {
+  return Butterflies<N, TPC, FirstRadix<L>::value>::per * FirstRadix<L>::value;
+}
+template <int N, int TPC, typename L>
 __device__ inline int first_point(int t, int e) {
   constexpr int R0 = FirstRadix<L>::value;
-  return t + (e / R0) * (N / PPT) + (e % R0) * (N / R0);
+  return t + (e / R0) * TPC + (e % R0) * (N / R0);
+}
+template <int N, int TPC, typename L>
+__device__ __forceinline__ bool first_ok(int t, int e) {
+  typedef Butterflies<N, TPC, FirstRadix<L>::value> B;
+  return B::exact || t + (e / FirstRadix<L>::value) * TPC < B::count;
 }
 
 // Whether v[e] of that layout lies in the upper half of the transform (point

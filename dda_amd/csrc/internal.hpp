@@ -14,6 +14,8 @@
 
 namespace dda {
 
+struct AxisOps;
+
 void set_error(const std::string& msg);
 
 #define DDA_TRY_HIP(expr)                                                                   \
@@ -195,6 +197,7 @@ struct dda_op_s {
   void* obs_scratch = nullptr;  // observables' work space
   size_t obs_bytes = 0;  // dda_op_tune ran (an FP32 twin of a tuned operator is tuned too)
   bool static_x = false;  // X passes with a compile-time plan (Gx has one)
+  const dda::AxisOps* gen[3] = {nullptr, nullptr, nullptr};  // the axes whose length has a general plan
   int cap_rhs = 1;   // right-hand sides the grid buffers hold
   int cc_rhs = 0;    // right-hand sides with couple constants set
   bool static_z = false;  // pass 3 uses a compile-time planned kernel

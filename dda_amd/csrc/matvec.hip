@@ -30,8 +30,8 @@
 #include <mutex>
 #include <tuple>
 
-#include "fft_static.hpp"
 #include "internal.hpp"
+#include "passes.hpp"
 
 namespace dda {
 
@@ -39,7 +39,6 @@ namespace dda {
 // Kernels
 // ------------------------------------------------------------------------------------
 
-__device__ inline bool stopped(const RhsFlags& f, int rhs) { return f.done != nullptr && f.done[rhs * f.stride] != 0; }
 
 // Pass 1: rows r0 .. r0+Lr-1 of the (z, y) plane, all three components. Tile
 // line l = c * Lr + lr.
@@ -167,15 +166,6 @@ __global__ __launch_bounds__(256) void k_pass5(const typename CxT<R>::T* __restr
   }
 }
 
-// Strided column FFT over T adjacent columns. Column `col` of batch b, point p
-// lives at base[b * bstride + p * pstride + col]; inputs beyond in_len are zero,
-// only the first out_len points are stored.
-struct ColParams {
-  int ncols;
-  int in_len, out_len;
-  long long pstride_in, pstride_out;
-  long long bstride_in, bstride_out;
-};
 
 template <typename R, int PPT, bool INV>
 __global__ __launch_bounds__(256) void k_colfft(const typename CxT<R>::T* in, typename CxT<R>::T* out, ColParams cp,
@@ -327,394 +317,6 @@ __global__ __launch_bounds__(256) void k_pass3(typename CxT<R>::T* a2, const typ
 }
 
 
-// ------------------------------------------------------------------------------------
-// Compile-time planned variants of the column passes (fft_static.hpp). Thread
-// (l, t) = (tid mod T, tid / T) owns column c0 + l and the plan's points t + ...
-// ------------------------------------------------------------------------------------
-
-// Buffer resources (V#) for the Z pass: raw (stride 0) buffers whose range
-// check turns loads beyond `bytes` into zeros and drops such stores, so that
-// the zero padding and the cropping need neither branches nor 64-bit address
-// arithmetic per access (the offset is a 32-bit byte offset from a uniform
-// base). Word 3 selects 32-bit data format, as gfx9-family buffers require.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t zrsrc(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ float2 zload(__amdgpu_buffer_rsrc_t r, uint32_t off, float2*) {
-  return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-}
-__device__ __forceinline__ double2 zload(__amdgpu_buffer_rsrc_t r, uint32_t off, double2*) {
-  return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
-typedef int zi2 __attribute__((ext_vector_type(2)));
-typedef int zi4 __attribute__((ext_vector_type(4)));
-constexpr int kStoreNT = 2;  // buffer cache policy: nt
-// The Z pass's stores and those of the X-forward and Y-inverse passes are
-// non-temporal (nt): their outputs are read by the next pass only after this
-// kernel's end, and streaming them leaves little dirty data in the L2s to be
-// written back when the kernel ends (the gap before the next kernel).
-// Measured in a solve at 256^3: 591 -> 560 us per 2-RHS matvec; the Y-forward
-// pass keeps ordinary stores (non-temporal ones made it 5% slower).
-__device__ __forceinline__ void zstore(__amdgpu_buffer_rsrc_t r, uint32_t off, float2 v) {
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(zi2, v), r, off, 0, kStoreNT);
-}
-__device__ __forceinline__ void zstore(__amdgpu_buffer_rsrc_t r, uint32_t off, double2 v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(zi4, v), r, off, 0, kStoreNT);
-}
-template <bool NT> __device__ __forceinline__ void cstore(float2* p, float2 v) {
-  if constexpr (NT) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    __builtin_nontemporal_store(__builtin_bit_cast(f2, v), reinterpret_cast<f2*>(p));
-  } else {
-    *p = v;
-  }
-}
-template <bool NT> __device__ __forceinline__ void cstore(double2* p, double2 v) {
-  if constexpr (NT) {
-    typedef double d2 __attribute__((ext_vector_type(2)));
-    __builtin_nontemporal_store(__builtin_bit_cast(d2, v), reinterpret_cast<d2*>(p));
-  } else {
-    *p = v;
-  }
-}
-
-// Waves per SIMD the Z pass is compiled for, a register budget: FP32
-// 16-point plans at 3 (168 VGPRs: the tensor loads of several points stay in
-// flight), other FP32 plans at 4, FP64 left to the compiler. At 1024 points
-// the 16-point plan runs 1024-thread work-groups, which fit a CU only at 4
-// waves per SIMD (128 VGPRs, a few spilled).
-// 32-point plans (FP32) hold 192 VGPRs of data: 2 waves per SIMD (256).
-template <typename R, int N, int PPT> struct P3Waves {
-  static constexpr int value = sizeof(R) == 4 ? (PPT >= 32 ? 2 : PPT >= 16 && N < 1024 ? 3 : 4) : 1;
-};
-
-// Pass 3 with a static plan of length N = Gz (see k_pass3 for the mapping).
-// Thread (l, t) holds, of every component, the points z = t + K_e of the plan's
-// first stage (K_e a compile-time constant per register e), so one lane offset
-// t * Gy * Gx + l addresses all of them from per-(component, e) uniform bases;
-// each such buffer's range ends at z = Bz (points at and beyond it read as zero
-// and are not stored) and spans at most N / PPT planes (it stays below 4 GiB up
-// to 1024^3). The tensor is read through one buffer per component with a lane
-// offset per point.
-// PL is the plan (StaticPlan<N, W> or a PlanOf variant).
-template <typename R, int N, int T, typename PL>
-__global__ __launch_bounds__(T * (N / PL::PPT))
-__attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT>::value))) void k_pass3s(typename CxT<R>::T* a2,
-                                                                              const typename CxT<R>::T* __restrict__ dhat,
-                                                MvDims d, const typename CxT<R>::T* __restrict__ tw, int nwork,
-                                                int nper, int nrhs, RhsFlags fl) {
-  typedef typename CxT<R>::T C;
-  typedef PL P;
-  constexpr int PPT = P::PPT;
-  constexpr int TPC = N / PPT;
-  typedef typename P::Fwd F;
-  typedef typename Reverse<F>::type Inv;
-  const int ntx = (d.Gx + T - 1) / T;
-  const int ftn = (ntx + 1) / 2;
-  const int hx = d.Gx / 2, hy = d.Gy / 2, hz = N / 2;
-  const int w = (blockIdx.x & 7) * nper + (blockIdx.x >> 3);
-  if (w >= nwork) return;
-  const int sub = w & 3, q = w >> 2;
-  const int rhs = q % nrhs, grp = q / nrhs;
-  if (stopped(fl, rhs)) return;
-  a2 += (long long)rhs * 3 * d.Bz * d.Gy * d.Gx;
-  if (d.dhat_tab) dhat = (const typename CxT<R>::T*)d.dhat_tab[d.member[rhs]];
-  const int ft = grp % ftn, fyp = grp / ftn;
-  int ky = fyp, tile_x = ft;
-  if (sub & 2) {
-    if (fyp == 0 || fyp == hy) return;
-    ky = d.Gy - fyp;
-  }
-  if (sub & 1) {
-    tile_x = ntx - 1 - ft;
-    if (tile_x == ft) return;
-  }
-  extern __shared__ char smem[];
-  C* tile = reinterpret_cast<C*>(smem);
-  constexpr int lp = (T & 1) ? T : T + 1;
-  const int l = threadIdx.x % T, t = threadIdx.x / T;
-  const int kx = tile_x * T + l;
-  const bool colok = kx < d.Gx;
-  const long long cstride = (long long)d.Bz * d.Gy * d.Gx;
-  const uint32_t zstride = (uint32_t)d.Gy * d.Gx;
-  C* base = a2 + (long long)ky * d.Gx + (long long)tile_x * T;
-  // lanes of columns beyond Gx address past every range
-  const uint32_t voff = colok ? ((uint32_t)t * zstride + l) * (uint32_t)sizeof(C) : 0xfffffff0u;
-  auto range = [&](const C* b, int c, int e) {
-    const int z0 = first_point<N, PPT, F>(0, e);
-    const int nz = d.Bz - z0 < TPC ? d.Bz - z0 : TPC;
-    return zrsrc(b + c * cstride + (long long)z0 * zstride, nz > 0 ? (uint32_t)nz * zstride * sizeof(C) : 0u);
-  };
-  C reg[3][PPT];
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int e = 0; e < PPT; e++)
-      reg[c][e] = upper_half<F>(e) ? czero<C>() : zload(range(base, c, e), voff, (C*)nullptr);
-  // Bz <= N/2 (the grid holds at least twice the box): the forward transforms
-  // skip the zero upper half and the inverse ones never form it; two-stage
-  // plans form the second-stage twiddle powers once for all six transforms
-  // (FP64 and 32-point plans: no registers to spare)
-  constexpr bool PRE = TwoStage<N, PPT, F>::value && sizeof(R) == 4 && PPT <= 16;
-  C wp[PRE ? PPT - 1 : 1];
-  if constexpr (PRE) twiddle_powers<PPT>(wp, t, tw);
-  const C* twp = PRE ? wp : tw;
-#pragma unroll
-  for (int c = 0; c < 3; c++) RunStages<N, PPT, false, 1, C, F, true, PRE>::run(reg[c], t, tile, lp, l, twp);
-  const uint32_t plane = (uint32_t)(hy + 1) * (hx + 1);
-  const uint32_t oct = plane * (uint32_t)(hz + 1);
-  const int fy = ky <= hy ? ky : d.Gy - ky;
-  const R sy = ky <= hy ? (R)1 : (R)-1;
-  const int fx = kx <= hx ? kx : d.Gx - kx;
-  const R sx = kx <= hx ? (R)1 : (R)-1;
-  const uint32_t fyx = colok ? (uint32_t)fy * (hx + 1) + fx : 0u;
-  const R sxy = sx * sy;
-  // (issuing point e + 1's tensor loads before point e is formed was measured
-  // slower: 275 -> 310 us per 2-RHS FP32 launch at 256^3, 300 -> 347 us FP64)
-#pragma unroll
-  for (int e = 0; e < PPT; e++) {
-    const int kz = first_point<N, PPT, Inv>(t, e);
-    const int fz = kz <= hz ? kz : N - kz;
-    const R sz = kz <= hz ? (R)1 : (R)-1;
-    const uint32_t o = ((uint32_t)fz * plane + fyx) * (uint32_t)sizeof(C);
-    C dc[6];
-#pragma unroll
-    for (int c = 0; c < 6; c++) dc[c] = zload(zrsrc(dhat + (size_t)c * oct, oct * sizeof(C)), o, (C*)nullptr);
-    const C d0 = dc[0], d1 = cscale(dc[1], sxy), d2 = cscale(dc[2], sx * sz), d3 = dc[3], d4 = cscale(dc[4], sy * sz),
-            d5 = dc[5];
-    const C x0 = reg[0][e], x1 = reg[1][e], x2 = reg[2][e];
-    reg[0][e] = cdot3(d0, x0, d1, x1, d2, x2);
-    reg[1][e] = cdot3(d1, x0, d3, x1, d4, x2);
-    reg[2][e] = cdot3(d2, x0, d4, x1, d5, x2);
-  }
-  // the store resources are formed anew (an opaque copy of the base keeps the
-  // compiler from holding the load ones in scalar registers across the
-  // transforms)
-  C* sbase = base;
-  asm volatile("" : "+s"(sbase));
-#pragma unroll
-  for (int c = 0; c < 3; c++) {
-    RunStages<N, PPT, true, 1, C, Inv, false, PRE>::run(reg[c], t, tile, lp, l, twp);
-#pragma unroll
-    for (int e = 0; e < PPT; e++)
-      if (!upper_half<F>(e)) zstore(range(sbase, c, e), voff, reg[c][e]);
-  }
-}
-
-// Pass 1 with a static plan of length N = Gx. A work-group takes LN consecutive
-// lines g = c * nrows + row of the A1 layout (contiguous in A1); thread (l, t),
-// t = tid mod TPC along the line, scatters line l's dipoles into the LDS tile,
-// then runs the transform from its first-stage points (only x < N/2 can hold
-// dipoles: the upper half is never read) and stores its outputs, TPC
-// consecutive points per line, coalesced.
-template <typename R, int N, bool W, int BS = 256>
-__global__ __launch_bounds__(BS) void k_pass1s(const typename CxT<R>::T* __restrict__ x,
-                                                typename CxT<R>::T* __restrict__ a1,
-                                                const uint32_t* __restrict__ row_start,
-                                                const uint32_t* __restrict__ row_dip,
-                                                const uint32_t* __restrict__ row_meta,
-                                                const typename CxT<R>::T* __restrict__ ccs, MvDims d,
-                                                const typename CxT<R>::T* __restrict__ tw, int conj, RhsFlags fl) {
-  typedef typename CxT<R>::T C;
-  typedef StaticPlan<N, W> P;
-  constexpr int PPT = P::PPT;
-  constexpr int TPC = N / PPT;
-  constexpr int LN = BS / TPC;
-  constexpr int lp = (LN & 1) ? LN : LN + 1;
-  typedef typename P::Fwd F;
-  typedef typename Reverse<F>::type Out;
-  const int rhs = blockIdx.y;
-  if (stopped(fl, rhs)) return;
-  x += (long long)rhs * 3 * d.S;
-  a1 += (long long)rhs * 3 * d.nrows * d.Gx;
-  ccs += rhs * 3 * d.nmat;
-  if (d.member) row_meta += (size_t)d.member[rhs] * d.nv;
-  extern __shared__ char smem[];
-  C* tile = reinterpret_cast<C*>(smem);
-  const int t = threadIdx.x % TPC, l = threadIdx.x / TPC;
-  const int nlines = 3 * d.nrows;
-  const int g = blockIdx.x * LN + l;
-  for (int i = threadIdx.x; i < (N / 2) * lp; i += blockDim.x) tile[i] = czero<C>();
-  __syncthreads();
-  if (g < nlines) {
-    const int c = g / d.nrows, row = g - c * d.nrows;
-    const uint32_t s0 = row_start[row], s1 = row_start[row + 1];
-    for (uint32_t q = s0 + t; q < s1; q += TPC) {
-      const uint32_t i = d.sorted ? q : row_dip[q], meta = row_meta[q];
-      C v = x[(size_t)c * d.S + i];
-      if (conj) v = cconj(v);
-      tile[(meta & 0xffff) * lp + l] = cmul(ccs[3 * (meta >> 16) + c], v);
-    }
-  }
-  __syncthreads();
-  C v[PPT];
-#pragma unroll
-  for (int e = 0; e < PPT; e++) v[e] = upper_half<F>(e) ? czero<C>() : tile[first_point<N, PPT, F>(t, e) * lp + l];
-  __syncthreads();
-  RunStages<N, PPT, false, 1, C, F, true>::run(v, t, tile, lp, l, tw);
-  if (g < nlines) {
-    C* dst = a1 + (size_t)g * N;
-#pragma unroll
-    for (int e = 0; e < PPT; e++) cstore<true>(dst + first_point<N, PPT, Out>(t, e), v[e]);
-  }
-}
-
-// The sums a pass 5 work-group forms over the entries it writes, in double,
-// with x and y as stored: x.y (DOT_U: q0, q1), |y|^2 (DOT_NORM: q0) or |y|^2
-// and x.conj(y) (DOT_OM: q0, q1, q2). Block sums of them, in a fixed order,
-// are stored as a solver's partial sums:
-// quantity q of work-group b of the launch's right-hand side r at
-// dot[(r * 4 + q) * gridDim.x + b]. Every thread of the block calls it.
-template <int BS>
-__device__ inline void dot_partials(double* dot, int op, double q0, double q1, double q2) {
-  __shared__ double red[3][BS / 64];
-  for (int off = 32; off > 0; off >>= 1) {
-    q0 += __shfl_xor(q0, off, 64);
-    q1 += __shfl_xor(q1, off, 64);
-    q2 += __shfl_xor(q2, off, 64);
-  }
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    red[0][w] = q0;
-    red[1][w] = q1;
-    red[2][w] = q2;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int nq = op == DOT_U ? 2 : op == DOT_NORM ? 1 : 3;
-    double* p = dot + (long long)blockIdx.y * 4 * gridDim.x + blockIdx.x;
-    for (int q = 0; q < nq; q++) {
-      double t = 0;
-      for (int i = 0; i < BS / 64; i++) t += red[q][i];
-      p[(long long)q * gridDim.x] = t;
-    }
-  }
-}
-
-// Pass 5 with a static plan: lines g = c * n_list + slot over the non-empty
-// rows; inverse transform from A1 (loads coalesced), the kept half (x < N/2)
-// through the tile, then line l's dipoles gathered by its TPC threads.
-// dot_op != DOT_NONE: also the partial sums of x and y (dot_partials) into dot.
-template <typename R, int N, bool W, int BS = 256>
-__global__ __launch_bounds__(BS) void k_pass5s(const typename CxT<R>::T* __restrict__ a1,
-                                                const typename CxT<R>::T* __restrict__ x,
-                                                typename CxT<R>::T* __restrict__ y,
-                                                const uint32_t* __restrict__ row_list, int n_list,
-                                                const uint32_t* __restrict__ row_start,
-                                                const uint32_t* __restrict__ row_dip,
-                                                const uint32_t* __restrict__ row_meta,
-                                                const typename CxT<R>::T* __restrict__ ccs, MvDims d,
-                                                const typename CxT<R>::T* __restrict__ tw, int conj, RhsFlags fl,
-                                                double* __restrict__ dot, int dot_op) {
-  typedef typename CxT<R>::T C;
-  typedef StaticPlan<N, W> P;
-  constexpr int PPT = P::PPT;
-  constexpr int TPC = N / PPT;
-  constexpr int LN = BS / TPC;
-  constexpr int lp = (LN & 1) ? LN : LN + 1;
-  typedef typename P::Fwd F;
-  typedef typename Reverse<F>::type Out;
-  const int rhs = blockIdx.y;
-  if (stopped(fl, rhs)) return;
-  a1 += (long long)rhs * 3 * d.nrows * d.Gx;
-  x += (long long)rhs * 3 * d.S;
-  y += (long long)rhs * 3 * d.S;
-  ccs += rhs * 3 * d.nmat;
-  if (d.member) row_meta += (size_t)d.member[rhs] * d.nv;
-  extern __shared__ char smem[];
-  C* tile = reinterpret_cast<C*>(smem);
-  const int t = threadIdx.x % TPC, l = threadIdx.x / TPC;
-  const int g = blockIdx.x * LN + l;
-  const bool ok = g < 3 * n_list;
-  const int c = ok ? g / n_list : 0;
-  const int row = ok ? (int)row_list[g - c * n_list] : 0;
-  const C* src = a1 + ((size_t)c * d.nrows + row) * N;
-  C v[PPT];
-#pragma unroll
-  for (int e = 0; e < PPT; e++) v[e] = ok ? src[first_point<N, PPT, F>(t, e)] : czero<C>();
-  // the dipoles this thread gathers (a row holds at most N/2: the grid spans
-  // at least twice the box), their x entries and positions loaded before the
-  // transform so that those loads wait while it runs
-  constexpr int MAXD = (N / 2 + TPC - 1) / TPC;
-  const uint32_t s0 = ok ? row_start[row] : 0u, s1 = ok ? row_start[row + 1] : 0u;
-  uint32_t gi[MAXD], gm[MAXD];
-  C ga[MAXD];
-#pragma unroll
-  for (int k = 0; k < MAXD; k++) {
-    const uint32_t q = s0 + t + k * TPC;
-    gi[k] = q < s1 ? (d.sorted ? q : row_dip[q]) : 0u;
-    gm[k] = q < s1 ? row_meta[q] : 0u;
-    ga[k] = q < s1 ? x[(size_t)c * d.S + gi[k]] : czero<C>();
-  }
-  RunStages<N, PPT, true, 1, C, F>::run(v, t, tile, lp, l, tw);
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < PPT; e++)
-    if (!upper_half<Out>(e)) tile[first_point<N, PPT, Out>(t, e) * lp + l] = v[e];
-  __syncthreads();
-  double q0 = 0, q1 = 0, q2 = 0;
-#pragma unroll
-  for (int k = 0; k < MAXD; k++) {
-    if (s0 + t + k * TPC < s1) {
-      C a = ga[k];
-      if (conj) a = cconj(a);
-      C r = cadd(cmul(ccs[3 * (gm[k] >> 16) + c], tile[(gm[k] & 0xffff) * lp + l]), a);
-      if (conj) r = cconj(r);
-      y[(size_t)c * d.S + gi[k]] = r;
-      if (dot_op != DOT_NONE) {
-        const double xr = ga[k].x, xi = ga[k].y, yr = r.x, yi = r.y;
-        const bool du = dot_op == DOT_U;
-        q0 += du ? xr * yr - xi * yi : yr * yr + yi * yi;
-        q1 += du ? xr * yi + xi * yr : xr * yr + xi * yi;
-        q2 += xi * yr - xr * yi;
-      }
-    }
-  }
-  if (dot_op != DOT_NONE) dot_partials<BS>(dot, dot_op, q0, q1, q2);
-  if (blockIdx.x == 0) {
-    const int pad = d.S - d.nv;
-    for (int q = threadIdx.x; q < 3 * pad; q += blockDim.x) {
-      const int cc = q / pad;
-      y[(size_t)cc * d.S + d.nv + (q - cc * pad)] = czero<C>();
-    }
-  }
-}
-
-// Column FFT with a static plan (pass 2 / pass 4 and the tensor generation).
-// HIN: in_len <= N/2, the zero upper half of the input is skipped; HOUT:
-// out_len <= N/2, the upper half of the output is never formed.
-template <typename R, int N, int T, bool W, bool INV, bool HIN, bool HOUT>
-__global__ __launch_bounds__(T * (N / StaticPlan<N, W>::PPT)) void k_colfft_s(const typename CxT<R>::T* in,
-                                                                                typename CxT<R>::T* out, ColParams cp,
-                                                  const typename CxT<R>::T* __restrict__ tw, RhsFlags fl) {
-  typedef typename CxT<R>::T C;
-  typedef StaticPlan<N, W> P;
-  constexpr int PPT = P::PPT;
-  typedef typename P::Fwd F;
-  typedef typename Reverse<F>::type Out;
-  if (stopped(fl, blockIdx.y / fl.per)) return;
-  extern __shared__ char smem[];
-  C* tile = reinterpret_cast<C*>(smem);
-  constexpr int lp = (T & 1) ? T : T + 1;
-  const int l = threadIdx.x % T, t = threadIdx.x / T;
-  const int col = blockIdx.x * T + l;
-  const bool colok = col < cp.ncols;
-  const C* src = in + (long long)blockIdx.y * cp.bstride_in + col;
-  C* dst = out + (long long)blockIdx.y * cp.bstride_out + col;
-  C v[PPT];
-#pragma unroll
-  for (int e = 0; e < PPT; e++) {
-    const int p = first_point<N, PPT, F>(t, e);
-    v[e] = (!(HIN && upper_half<F>(e)) && colok && p < cp.in_len) ? src[p * cp.pstride_in] : czero<C>();
-  }
-  RunStages<N, PPT, INV, 1, C, F, HIN>::run(v, t, tile, lp, l, tw);
-#pragma unroll
-  for (int e = 0; e < PPT; e++) {
-    const int p = first_point<N, PPT, Out>(t, e);
-    if (!(HOUT && upper_half<Out>(e)) && colok && p < cp.out_len)
-      cstore<INV>(dst + p * cp.pstride_out, v[e]);
-  }
-}
 
 // Row FFT over contiguous lines (used for the X axis of the tensor generation).
 template <typename R, int PPT, bool INV>
@@ -867,12 +469,6 @@ inline int col_tile(int n, int pref) {
   return t;
 }
 
-template <typename K>
-dda_status set_lds(K kernel, size_t bytes) {
-  if (bytes > 64 * 1024) DDA_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-  return DDA_OK;
-}
 
 template <typename R, bool INV>
 dda_status launch_col(const void* in, void* out, const ColParams& cp, const FftPlan& p, int T, const void* tw,
@@ -928,240 +524,8 @@ dda_status launch_row(void* data, long long nlines, const FftPlan& p, const void
   return DDA_OK;
 }
 
-
-// Columns per work-group for a static plan: 128-byte row segments, at most 256
-// threads.
-// Long columns (512, 1024 points) keep 128-byte segments with larger
-// work-groups: up to 1024 threads for a single-component transform, 512 for
-// the Z pass, whose threads hold three components. PREF (if nonzero) asks for
-// that many columns instead.
-template <typename R, int N, bool W, int MAXT = 256, int PREF = 0>
-constexpr int static_cols() {
-  constexpr int pref = PREF ? PREF : sizeof(R) == 8 ? 8 : 16;
-  constexpr int tpc = N / StaticPlan<N, W>::PPT;
-  constexpr int cap = N >= 512 ? MAXT : 256;
-  // at least one full wavefront per work-group
-  constexpr int t = pref * tpc < 64 ? 64 / tpc : pref;
-  return t * tpc <= cap ? t : cap / tpc;
-}
-
-// Plan width of a static kernel: 1 = wide (16 points per thread where the plan
-// has them), 0 = narrow, -1 = the precision's default (wide for complex float).
-template <typename R>
-inline bool plan_wide(int w) {
-  return w < 0 ? sizeof(R) == 4 : w != 0;
-}
-
-// The other tile the tuner tries for the FP32 Y passes: twice the default
-// columns per work-group where that stays within 1024 threads, else half
-// (keeping at least one wavefront).
-template <int T, int TPC>
-constexpr int other_cols() {
-  return 2 * T * TPC <= 1024 ? 2 * T : (T / 2) * TPC >= 64 ? T / 2 : T;
-}
-// and the third: four times the default columns where that stays within 1024
-// threads and the LDS (FP32 tiles of N x (4T + 1) points), else the second
-template <int T, int TPC, int N>
-constexpr int third_cols() {
-  return 4 * T * TPC <= 1024 && (size_t)N * (4 * T + 1) * 8 <= 160 * 1024 ? 4 * T : other_cols<T, TPC>();
-}
-
-// ALT: 0 the default tile, 1 other_cols, 2 third_cols
-template <typename R, int N, bool W, bool INV, int ALT = 0>
-dda_status launch_col_static_w(const void* in, void* out, const ColParams& cp, const void* tw, int nbatch,
-                               hipStream_t st, RhsFlags done) {
-  typedef typename CxT<R>::T C;
-  constexpr int T0 = static_cols<R, N, W, 1024>();
-  constexpr int TPC0 = N / StaticPlan<N, W>::PPT;
-  constexpr int T = ALT == 0 ? T0 : ALT == 1 ? other_cols<T0, TPC0>() : third_cols<T0, TPC0, N>();
-  constexpr int threads = T * (N / StaticPlan<N, W>::PPT);
-  constexpr int lp = (T & 1) ? T : T + 1;
-  const size_t lds = (size_t)N * lp * sizeof(C);
-  // the matvec's forward pass reads at most N/2 points and its inverse pass
-  // keeps at most N/2; the tensor generation transforms full lengths
-  const bool hin = !INV && 2 * cp.in_len <= N, hout = INV && 2 * cp.out_len <= N;
-  void (*k)(const C*, C*, ColParams, const C*, RhsFlags);
-  if constexpr (ALT != 0) {
-    // the other tiles are matvec variants: full-length transforms keep the default
-    if (!hin && !hout) return launch_col_static_w<R, N, W, INV, 0>(in, out, cp, tw, nbatch, st, done);
-    k = INV ? k_colfft_s<R, N, T, W, INV, false, INV> : k_colfft_s<R, N, T, W, INV, !INV, false>;
-  } else {
-    k = hin ? k_colfft_s<R, N, T, W, INV, !INV, false>
-            : hout ? k_colfft_s<R, N, T, W, INV, false, INV> : k_colfft_s<R, N, T, W, INV, false, false>;
-  }
-  DDA_TRY(set_lds(k, lds));
-  hipLaunchKernelGGL(k, dim3((cp.ncols + T - 1) / T, nbatch), dim3(threads), lds, st, (const C*)in, (C*)out, cp,
-                     (const C*)tw, done);
-  DDA_TRY_HIP(hipGetLastError());
-  return DDA_OK;
-}
-
-// wide: -1 the precision's default plan, 0 narrow, 1 wide; FP32 also 2 and 3,
-// narrow and wide with the second tile (other_cols), and 4 and 5 with the
-// third (third_cols).
-template <typename R, int N, bool INV>
-dda_status launch_col_static(const void* in, void* out, const ColParams& cp, const void* tw, int nbatch, hipStream_t st,
-                             RhsFlags done, int wide) {
-  if constexpr (sizeof(R) == 4) {
-    if (wide >= 4)
-      return (wide & 1) ? launch_col_static_w<R, N, true, INV, 2>(in, out, cp, tw, nbatch, st, done)
-                        : launch_col_static_w<R, N, false, INV, 2>(in, out, cp, tw, nbatch, st, done);
-    if (wide >= 2)
-      return (wide & 1) ? launch_col_static_w<R, N, true, INV, 1>(in, out, cp, tw, nbatch, st, done)
-                        : launch_col_static_w<R, N, false, INV, 1>(in, out, cp, tw, nbatch, st, done);
-  }
-  return plan_wide<R>(wide >= 2 ? (wide & 1) : wide) ? launch_col_static_w<R, N, true, INV>(in, out, cp, tw, nbatch, st, done)
-                                                    : launch_col_static_w<R, N, false, INV>(in, out, cp, tw, nbatch, st, done);
-}
-
-// The buffers of right-hand sides r0 .. r0 + nrhs - 1 of an operator: what one
-// sequence of the five passes works on (the whole block, or one half of it
-// when the halves run on two streams).
-struct MvView {
-  void* a1;
-  void* a2;
-  const void* ccs;
-  MvDims d;  // member table shifted to r0
-};
-
-inline MvView view_of(const dda_op_s* op, int r0) {
-  const MvDims& d = op->dims;
-  const size_t csz = op->prec == 64 ? sizeof(double2) : sizeof(float2);
-  MvView v;
-  v.a1 = (char*)op->a1 + (size_t)r0 * 3 * d.Bz * d.By * d.Gx * csz;
-  v.a2 = (char*)op->a2 + (size_t)r0 * 3 * d.Bz * d.Gy * d.Gx * csz;
-  v.ccs = (const char*)op->ccs + (size_t)r0 * 3 * d.nmat * csz;
-  v.d = d;
-  if (d.member) v.d.member = d.member + r0;
-  return v;
-}
-
-template <typename R, int N, typename PL, int T>
-dda_status launch_pass3_plan(dda_op_s* op, const MvView& v, hipStream_t st, RhsFlags done, int nrhs) {
-  typedef typename CxT<R>::T C;
-  constexpr int threads = T * (N / PL::PPT);
-  constexpr int lp = (T & 1) ? T : T + 1;
-  const MvDims& d = v.d;
-  const size_t lds = (size_t)N * lp * sizeof(C);
-  const int ntx = (d.Gx + T - 1) / T;
-  const int nwork = (d.Gy / 2 + 1) * ((ntx + 1) / 2) * 4 * nrhs;
-  const int nper = (nwork + 7) / 8;
-  auto k = k_pass3s<R, N, T, PL>;
-  DDA_TRY(set_lds(k, lds));
-  hipLaunchKernelGGL(k, dim3(8 * nper), dim3(threads), lds, st, (C*)v.a2, (const C*)op->dhat, d,
-                     (const C*)op->tw[2], nwork, nper, nrhs, done);
-  DDA_TRY_HIP(hipGetLastError());
-  return DDA_OK;
-}
-
-// The other tile the tuner tries for the FP32 Z pass: 32 columns where the
-// default is 16 and 32 fit the work-group size the kernel's register budget
-// allows (MAXTH threads), else half the default.
-template <int T, int TPC, int MAXTH>
-constexpr int other_cols_z() {
-  return T != 32 && 32 * TPC <= MAXTH ? 32 : (T / 2) * TPC >= 64 ? T / 2 : T;
-}
-
-template <typename R, int N, bool W, bool ALT = false>
-dda_status launch_pass3_static_w(dda_op_s* op, const MvView& v, hipStream_t st, RhsFlags done, int nrhs) {
-  // FP32 1024-point columns: 16 columns (128-byte segments) in a 1024-thread
-  // work-group at 128 VGPRs, the CU's whole register file (17.5 ms at 1024^3,
-  // against 22.7 ms for two 512-thread work-groups of 8 columns)
-  // short FP32 columns (at most 64 points): 32 columns (256-byte segments)
-  // per work-group; measured on a 128-RHS block at a 64-point Z grid: 935 ->
-  // 781 us per launch
-  constexpr int T0 = static_cols<R, N, W, (N == 1024 && sizeof(R) == 4 && W) ? 1024 : 512,
-                                 (sizeof(R) == 4 && N <= 64) ? 32 : 0>();
-  constexpr int TPC = N / StaticPlan<N, W>::PPT;
-  constexpr int T = ALT ? other_cols_z<T0, TPC, 256 * P3Waves<R, N, StaticPlan<N, W>::PPT>::value>() : T0;
-  return launch_pass3_plan<R, N, StaticPlan<N, W>, T>(op, v, st, done, nrhs);
-}
-
-// Z-pass variants (Tune::p3_wide): -1 the precision's default, 0 narrow,
-// 1 wide; at 1024 points also 2 and 3, the 32 x 32 plan (32 points per
-// thread, one LDS exchange per transform, 2 waves per SIMD, FP32) over 16
-// columns (512 threads, 128-byte segments, one work-group per CU by LDS) or
-// 8 columns (256 threads, 64-byte segments, two work-groups per CU).
-// FP32 only: in FP64 the 32-point plan's data alone needs 384 VGPRs. The FP32
-// default at 1024 points is 2: measured at 1024^3 (sphere 512 across) 14.8 ms
-// against 17.8 ms (wide), 19.2 ms (variant 3) and 33.0 ms (narrow).
-// (Two further forms were measured and dropped. The wide plan without held
-// twiddle powers at 4 waves per SIMD, 128 VGPRs: 308.8 against 293.2 us per
-// 2-RHS FP32 launch at 256^3, and it spills at 32, 128 and 512 points. A
-// persistent kernel, resident work-groups looping over the tiles and loading
-// each component of the next tile into the registers its store frees:
-// 303.5 against 289.3 us (2-RHS FP32, 256^3), 315.0 against 291.4 us (FP64),
-// 15.1 against 14.6 ms (FP32, 1024^3); its loop costs 13% more VALU at 1024
-// points than the hidden loads save.)
-typedef PlanOf<1024, 32, RadixList<32, 32>> Plan1024x32;
-// FP32 below 1024 points: 2 and 3 are the narrow and wide plans with the
-// other tile (other_cols_z).
-inline int p3_variants(int n, int prec) { return prec == 32 ? 4 : 2; }
-
-template <typename R, int N>
-dda_status launch_pass3_static(dda_op_s* op, const MvView& v, hipStream_t st, RhsFlags done, int nrhs,
-                               const dda_op_s::Tune& tn) {
-  const int var = tn.p3_wide;
-  if constexpr (N == 1024 && sizeof(R) == 4) {
-    if (var == 2 || var < 0) return launch_pass3_plan<R, N, Plan1024x32, 16>(op, v, st, done, nrhs);
-    if (var == 3) return launch_pass3_plan<R, N, Plan1024x32, 8>(op, v, st, done, nrhs);
-  } else if constexpr (sizeof(R) == 4) {
-    if (var >= 2)
-      return (var & 1) ? launch_pass3_static_w<R, N, true, true>(op, v, st, done, nrhs)
-                       : launch_pass3_static_w<R, N, false, true>(op, v, st, done, nrhs);
-  }
-  return plan_wide<R>(var >= 2 ? (var & 1) : var) ? launch_pass3_static_w<R, N, true>(op, v, st, done, nrhs)
-                           : launch_pass3_static_w<R, N, false>(op, v, st, done, nrhs);
-}
-
-template <typename R, int N, bool W, int BS = 256>
-dda_status launch_x_static_w(dda_op_s* op, const MvView& v, bool inverse, const void* x, void* y, int conj,
-                             hipStream_t st, RhsFlags done, int nrhs, const PassDotReq& dr) {
-  typedef typename CxT<R>::T C;
-  constexpr int TPC = N / StaticPlan<N, W>::PPT;
-  constexpr int LN = BS / TPC;
-  constexpr int lp = (LN & 1) ? LN : LN + 1;
-  const MvDims& d = v.d;
-  const size_t lds = (size_t)N * lp * sizeof(C);
-  if (!inverse) {
-    auto k = k_pass1s<R, N, W, BS>;
-    DDA_TRY(set_lds(k, lds));
-    hipLaunchKernelGGL(k, dim3((3 * d.nrows + LN - 1) / LN, nrhs), dim3(LN * TPC), lds, st, (const C*)x, (C*)v.a1,
-                       op->row_start, op->row_dip, op->row_meta, (const C*)v.ccs, d, (const C*)op->tw[0], conj,
-                       done);
-  } else {
-    auto k = k_pass5s<R, N, W, BS>;
-    DDA_TRY(set_lds(k, lds));
-    const int nl = 3 * op->n_nonempty;
-    const int nbx = nl > 0 ? (nl + LN - 1) / LN : 1;
-    op->p5_blocks = nbx;
-    double* dot = dr.op != DOT_NONE ? dr.part + (size_t)dr.r0 * 4 * nbx : nullptr;
-    hipLaunchKernelGGL(k, dim3(nbx, nrhs), dim3(LN * TPC), lds, st, (const C*)v.a1, (const C*)x, (C*)y, op->row_list,
-                       op->n_nonempty, op->row_start, op->row_dip, op->row_meta, (const C*)v.ccs, d,
-                       (const C*)op->tw[0], conj, done, dot, dr.op);
-  }
-  DDA_TRY_HIP(hipGetLastError());
-  return DDA_OK;
-}
-
-template <typename R, int N>
-dda_status launch_x_static(dda_op_s* op, const MvView& v, bool inverse, const void* x, void* y, int conj,
-                           hipStream_t st, RhsFlags done, int nrhs, const dda_op_s::Tune& tn,
-                           const PassDotReq& dr = PassDotReq()) {
-  // default narrow for both precisions: half the LDS per wave, twice the waves
-  // per CU (measured 52 -> 39 us at 256^3 FP32); FP32 also 2 and 3, narrow
-  // and wide over 512-thread work-groups (twice the lines each)
-  const int var = tn.x_wide[inverse];
-  if constexpr (sizeof(R) == 4) {
-    if (var >= 2)
-      return (var & 1) ? launch_x_static_w<R, N, true, 512>(op, v, inverse, x, y, conj, st, done, nrhs, dr)
-                       : launch_x_static_w<R, N, false, 512>(op, v, inverse, x, y, conj, st, done, nrhs, dr);
-  }
-  return var >= 0 && (var & 1) ? launch_x_static_w<R, N, true>(op, v, inverse, x, y, conj, st, done, nrhs, dr)
-                               : launch_x_static_w<R, N, false>(op, v, inverse, x, y, conj, st, done, nrhs, dr);
-}
-
-// Lengths with a static plan; others use the run-time planned kernels.
+// Lengths with a static plan and tuned variants. Other lengths run the one plan
+// that plans.hip holds for them (axis_ops), or the run-time planned kernels.
 #define DDA_STATIC_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(512) X(1024)
 
 inline bool has_static_plan(int n) {
@@ -1181,11 +545,16 @@ inline bool has_static_plan(int n) {
 // Gz/8 planes of Gy*Gx elements (its plans have at least 8 points per
 // thread). Grids beyond that run the run-time planned Z pass, whose addressing
 // is 64-bit.
-inline bool static_z_fits(int Gx, int Gy, int Gz, size_t csz) {
+inline bool z_offsets_fit(int Gx, int Gy, int Gz, size_t csz) {
   const uint64_t lim = 1ull << 32;
   const uint64_t oct = (uint64_t)(Gx / 2 + 1) * (Gy / 2 + 1) * (Gz / 2 + 1);
-  const uint64_t span = (uint64_t)(Gz / 8 + 1) * Gy * Gx;
-  return has_static_plan(Gz) && oct * csz < lim && span * csz < lim;
+  // (a general plan of a short length holds fewer points, at most 28 threads
+  // or an eighth of the length per column)
+  const uint64_t span = (uint64_t)std::max(Gz / 8 + 1, std::min(Gz, 28)) * Gy * Gx;
+  return oct * csz < lim && span * csz < lim;
+}
+inline bool static_z_fits(int Gx, int Gy, int Gz, size_t csz) {
+  return has_static_plan(Gz) && z_offsets_fit(Gx, Gy, Gz, csz);
 }
 
 template <typename R, bool INV>
@@ -1203,6 +572,20 @@ dda_status launch_col_any(const void* in, void* out, const ColParams& cp, const 
 }
 
 }  // namespace
+
+#define DDA_PARTS(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7)
+#define X(P) const AxisOps* axis_ops_part##P(int n, int prec);
+DDA_PARTS(X)
+#undef X
+
+// The general plan's launchers for length n, or null.
+static const AxisOps* axis_ops(int n, int prec) {
+#define X(P) \
+  if (const AxisOps* o = axis_ops_part##P(n, prec)) return o;
+  DDA_PARTS(X)
+#undef X
+  return nullptr;
+}
 
 // Timing events of dda_op_profile, recycled between reads.
 static hipEvent_t pool_event(dda_op_s* op) {
@@ -1268,7 +651,9 @@ static dda_status launch_passes(dda_op_s* op, const void* xv, void* yv, int conj
   const FastDiv ldiv = make_fastdiv(L), ndiv = make_fastdiv(d.Gx);
   if (p0 <= 0 && 0 <= p1) {
     PassTimer pt(op, st, 0);
-    if (op->static_x) {
+    if (op->gen[0]) {
+      DDA_TRY(op->gen[0]->x(op, v, false, x, nullptr, conj, st, done, nrhs, PassDotReq()));
+    } else if (op->static_x) {
       switch (d.Gx) {
 #define X(N)                                                                         \
   case N:                                                                            \
@@ -1309,14 +694,21 @@ static dda_status launch_passes(dda_op_s* op, const void* xv, void* yv, int conj
       const long long nb0 = 3ll * d.Bz * q0;
       RhsFlags f = col_done;
       if (f.done) f.done += (long long)q0 * f.stride;
-      DDA_TRY((launch_col_any<R, false>(a1 + nb0 * cp.bstride_in, a2 + nb0 * cp.bstride_out, cp, op->plan[1],
-                                        op->col_t, op->tw[1], 3 * d.Bz * k, st, f, tn.col_wide[0])));
+      const C* in = a1 + nb0 * cp.bstride_in;
+      C* out = a2 + nb0 * cp.bstride_out;
+      if (op->gen[1])
+        DDA_TRY(op->gen[1]->col(false, in, out, cp, op->tw[1], 3 * d.Bz * k, st, f));
+      else
+        DDA_TRY((launch_col_any<R, false>(in, out, cp, op->plan[1], op->col_t, op->tw[1], 3 * d.Bz * k, st, f,
+                                          tn.col_wide[0])));
     }
   }
   // pass 3: Z forward, D multiply, Z inverse, in place on A2
   if (p0 <= 2 && 2 <= p1) {
     PassTimer pt(op, st, 2);
-    if (op->static_z) {
+    if (op->gen[2]) {
+      DDA_TRY(op->gen[2]->z(op, v, st, done, nrhs));
+    } else if (op->static_z) {
       switch (d.Gz) {
 #define X(N)                                                         \
   case N:                                                            \
@@ -1369,8 +761,13 @@ static dda_status launch_passes(dda_op_s* op, const void* xv, void* yv, int conj
       const long long nb0 = 3ll * d.Bz * q0;
       RhsFlags f = col_done;
       if (f.done) f.done += (long long)q0 * f.stride;
-      DDA_TRY((launch_col_any<R, true>(a2 + nb0 * cp.bstride_in, a1 + nb0 * cp.bstride_out, cp, op->plan[1],
-                                       op->col_t, op->tw[1], 3 * d.Bz * k, st, f, tn.col_wide[1])));
+      const C* in = a2 + nb0 * cp.bstride_in;
+      C* out = a1 + nb0 * cp.bstride_out;
+      if (op->gen[1])
+        DDA_TRY(op->gen[1]->col(true, in, out, cp, op->tw[1], 3 * d.Bz * k, st, f));
+      else
+        DDA_TRY((launch_col_any<R, true>(in, out, cp, op->plan[1], op->col_t, op->tw[1], 3 * d.Bz * k, st, f,
+                                         tn.col_wide[1])));
     }
   }
   // pass 5
@@ -1382,7 +779,9 @@ static dda_status launch_passes(dda_op_s* op, const void* xv, void* yv, int conj
       set_error("matvec: partial sums in pass 5 need a compile-time planned X pass");
       return DDA_NOT_SUPPORTED;
     }
-    if (op->static_x) {
+    if (op->gen[0]) {
+      DDA_TRY(op->gen[0]->x(op, v, true, x, y, conj, st, done, nrhs, dr));
+    } else if (op->static_x) {
       switch (d.Gx) {
 #define X(N)                                                                    \
   case N:                                                                       \
@@ -1891,8 +1290,12 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
   d.sorted = 1;  // the reference's (z, y, x) dipole order makes the row index the identity
   for (uint32_t k = 0; k < ds.nv && d.sorted; k++) d.sorted = row_dip[k] == k;
   const size_t csz = precision == 64 ? sizeof(double2) : sizeof(float2);
-  op->static_z = static_z_fits(d.Gx, d.Gy, d.Gz, csz) && !std::getenv("DDA_GENERIC_FFT");
-  op->static_x = has_static_plan(d.Gx) && !std::getenv("DDA_GENERIC_FFT");
+  if (!std::getenv("DDA_GENERIC_FFT")) {
+    for (int a = 0; a < 3; a++) op->gen[a] = axis_ops(grid[a], precision);
+    if (!z_offsets_fit(d.Gx, d.Gy, d.Gz, csz)) op->gen[2] = nullptr;
+    op->static_z = op->gen[2] || static_z_fits(d.Gx, d.Gy, d.Gz, csz);
+    op->static_x = op->gen[0] || has_static_plan(d.Gx);
+  }
   op->split_rhs = std::getenv("DDA_SPLIT") && std::atoi(std::getenv("DDA_SPLIT")) != 0;
 
   // Launch shapes: X passes hold ~2048 points per work-group; column passes
@@ -2538,7 +1941,8 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
     }
   }
   for (int pass = 0; pass < 5; pass++) {
-    const bool is_static = pass == 1 ? op->static_z : pass >= 3 ? op->static_x : has_static_plan(d.Gy);
+    const int axis = pass == 1 ? 2 : pass >= 3 ? 0 : 1;
+    const bool is_static = !op->gen[axis] && (pass == 1 ? op->static_z : pass >= 3 ? op->static_x : has_static_plan(d.Gy));
     if (!is_static) continue;
     // Z: p3_variants; FP32 X: narrow and wide, each with the other tile too;
     // FP32 Y: with the second and the third tile
