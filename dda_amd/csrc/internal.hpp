@@ -37,6 +37,8 @@ void set_error(const std::string& msg);
 struct MvDims {
   int Bx, By, Bz;
   int Gx, Gy, Gz;
+  int rs;  // elements from one row (x line) of A1 and A2 to the next: Gx up to whole 128-byte lines
+  int p2;  // elements from one (y, x) plane of A2 to the next: Gy * rs and one line more
   int nv;
   int S;       // vector stride
   int nrows;   // By * Bz

@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void k_pass1(const typename CxT<R>::T* __restr
   const int rhs = blockIdx.y;
   if (stopped(fl, rhs)) return;
   x += (long long)rhs * 3 * d.S;
-  a1 += (long long)rhs * 3 * d.nrows * d.Gx;
+  a1 += (long long)rhs * 3 * d.nrows * d.rs;
   ccs += rhs * 3 * d.nmat;
   if (d.member) row_meta += (size_t)d.member[rhs] * d.nv;
   extern __shared__ char smem[];
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void k_pass1(const typename CxT<R>::T* __restr
     const int c = l / lr_n;
     const int lr = l - c * lr_n;
     const int row = r0 + lr;
-    if (row < d.nrows) a1[((size_t)c * d.nrows + row) * N + p] = tile[p * lp + l];
+    if (row < d.nrows) a1[((size_t)c * d.nrows + row) * d.rs + p] = tile[p * lp + l];
   }
 }
 
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256) void k_pass5(const typename CxT<R>::T* __restr
   typedef typename CxT<R>::T C;
   const int rhs = blockIdx.y;
   if (stopped(fl, rhs)) return;
-  a1 += (long long)rhs * 3 * d.nrows * d.Gx;
+  a1 += (long long)rhs * 3 * d.nrows * d.rs;
   x += (long long)rhs * 3 * d.S;
   y += (long long)rhs * 3 * d.S;
   ccs += rhs * 3 * d.nmat;
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void k_pass5(const typename CxT<R>::T* __restr
     const int lr = l - c * lr_n;
     const int slot = s_base + lr;
     C v = czero<C>();
-    if (slot < n_list) v = a1[((size_t)c * d.nrows + row_list[slot]) * N + p];
+    if (slot < n_list) v = a1[((size_t)c * d.nrows + row_list[slot]) * d.rs + p];
     tile[p * lp + l] = v;
   }
   __syncthreads();
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void k_pass3(typename CxT<R>::T* a2, const typ
   const int sub = w & 3, q = w >> 2;
   const int rhs = q % nrhs, grp = q / nrhs;
   if (stopped(fl, rhs)) return;
-  a2 += (long long)rhs * 3 * d.Bz * d.Gy * d.Gx;
+  a2 += (long long)rhs * 3 * d.Bz * d.p2;
   if (d.dhat_tab) dhat = (const typename CxT<R>::T*)d.dhat_tab[d.member[rhs]];
   const int ft = grp % ftn, fyp = grp / ftn;
   int ky = fyp, tile_x = ft;
@@ -243,10 +243,10 @@ __global__ __launch_bounds__(256) void k_pass3(typename CxT<R>::T* a2, const typ
   const int lp = lds_stride(T);
   const int N = d.Gz;
   const int pts = N * T;
-  const long long cstride = (long long)d.Bz * d.Gy * d.Gx;
-  const long long zstride = (long long)d.Gy * d.Gx;
+  const long long cstride = (long long)d.Bz * d.p2;
+  const long long zstride = d.p2;
   const long long oct = (long long)(hx + 1) * (hy + 1) * (hz + 1);
-  C* base = a2 + (long long)ky * d.Gx;
+  C* base = a2 + (long long)ky * d.rs;
   C reg[3][PPT];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
@@ -456,6 +456,18 @@ namespace {
 
 inline int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
+// Rows of the grid buffers start on 128-byte lines, so that a column tile's row
+// segment is one line and not parts of two (8 elements off, the FP32 Y passes
+// at 256^3 take 10% longer, at 128 x 96 x 64 20%), and planes of A2 are one line
+// longer than their rows, so that a Z column's points, one per plane, do not
+// all lie a power of two apart and load a few HBM channels in turn. The line
+// took a product of the sphere 128 across (256^3) from 624 to 591 us (FP32, two
+// right-hand sides) and 645 to 610 us (FP64), of the ellipsoid 64 across
+// (128 x 96 x 64, FP64, 32 right-hand sides) from 927 to 825 us, of the sphere
+// 256 across (512^3, FP32) from 3.52 to 3.28 ms.
+inline int line_elems(int prec) { return prec == 64 ? 8 : 16; }
+inline int row_stride(int gx, int prec) { return round_up(gx, line_elems(prec)); }
+
 // Threads per block for a tile of `pts` points with PPT points per thread.
 inline int block_for(int pts, int ppt) {
   int b = round_up((pts + ppt - 1) / ppt, 64);
@@ -550,7 +562,7 @@ inline bool z_offsets_fit(int Gx, int Gy, int Gz, size_t csz) {
   const uint64_t oct = (uint64_t)(Gx / 2 + 1) * (Gy / 2 + 1) * (Gz / 2 + 1);
   // (a general plan of a short length holds fewer points, at most 28 threads
   // or an eighth of the length per column)
-  const uint64_t span = (uint64_t)std::max(Gz / 8 + 1, std::min(Gz, 28)) * Gy * Gx;
+  const uint64_t span = (uint64_t)std::max(Gz / 8 + 1, std::min(Gz, 28)) * (Gy + 1) * row_stride(Gx, csz == sizeof(double2) ? 64 : 32);
   return oct * csz < lim && span * csz < lim;
 }
 inline bool static_z_fits(int Gx, int Gy, int Gz, size_t csz) {
@@ -685,10 +697,10 @@ static dda_status launch_passes(dda_op_s* op, const void* xv, void* yv, int conj
     cp.ncols = d.Gx;
     cp.in_len = d.By;
     cp.out_len = d.Gy;
-    cp.pstride_in = d.Gx;
-    cp.pstride_out = d.Gx;
-    cp.bstride_in = (long long)d.By * d.Gx;
-    cp.bstride_out = (long long)d.Gy * d.Gx;
+    cp.pstride_in = d.rs;
+    cp.pstride_out = d.rs;
+    cp.bstride_in = (long long)d.By * d.rs;
+    cp.bstride_out = d.p2;
     for (int q0 = 0; q0 < nrhs; q0 += rhs_per_col_launch) {
       const int k = std::min(rhs_per_col_launch, nrhs - q0);
       const long long nb0 = 3ll * d.Bz * q0;
@@ -752,10 +764,10 @@ static dda_status launch_passes(dda_op_s* op, const void* xv, void* yv, int conj
     cp.ncols = d.Gx;
     cp.in_len = d.Gy;
     cp.out_len = d.By;
-    cp.pstride_in = d.Gx;
-    cp.pstride_out = d.Gx;
-    cp.bstride_in = (long long)d.Gy * d.Gx;
-    cp.bstride_out = (long long)d.By * d.Gx;
+    cp.pstride_in = d.rs;
+    cp.pstride_out = d.rs;
+    cp.bstride_in = d.p2;
+    cp.bstride_out = (long long)d.By * d.rs;
     for (int q0 = 0; q0 < nrhs; q0 += rhs_per_col_launch) {
       const int k = std::min(rhs_per_col_launch, nrhs - q0);
       const long long nb0 = 3ll * d.Bz * q0;
@@ -1247,6 +1259,8 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
   MvDims& d = op->dims;
   d.Bx = ds.box[0]; d.By = ds.box[1]; d.Bz = ds.box[2];
   d.Gx = grid[0]; d.Gy = grid[1]; d.Gz = grid[2];
+  d.rs = row_stride(d.Gx, precision);
+  d.p2 = d.Gy * d.rs + line_elems(precision);
   d.nv = ds.nv;
   d.S = S;
   d.nrows = d.By * d.Bz;
@@ -1318,8 +1332,8 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
     op->device_bytes += bytes;
     return DDA_OK;
   };
-  const size_t a1n = 3ull * d.Bz * d.By * d.Gx;
-  const size_t a2n = 3ull * d.Bz * d.Gy * d.Gx;
+  const size_t a1n = 3ull * d.Bz * d.By * d.rs;
+  const size_t a2n = 3ull * d.Bz * d.p2;
   const size_t dn = 6ull * (d.Gx / 2 + 1) * (d.Gy / 2 + 1) * (d.Gz / 2 + 1);
   dda_status rc = DDA_OK;
   if (rc == DDA_OK) rc = dmalloc((void**)&op->row_start, row_start.size() * 4);
@@ -1699,7 +1713,7 @@ static dda_status ensure_rhs_capacity(dda_op_s* op, int nrhs) {
   DDA_TRY_HIP(hipStreamSynchronize(op->ctx->stream));
   const MvDims& d = op->dims;
   const size_t csz = op->prec == 64 ? sizeof(double2) : sizeof(float2);
-  const size_t a1n = 3ull * d.Bz * d.By * d.Gx, a2n = 3ull * d.Bz * d.Gy * d.Gx;
+  const size_t a1n = 3ull * d.Bz * d.By * d.rs, a2n = 3ull * d.Bz * d.p2;
   void *a1 = nullptr, *a2 = nullptr, *ccs = nullptr;
   hipError_t e = hipMalloc(&a1, a1n * csz * nrhs);
   if (e == hipSuccess) e = hipMalloc(&a2, a2n * csz * nrhs);
@@ -1926,8 +1940,8 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
   hipStream_t st = op->ctx->stream;
   const size_t csz = sizeof(typename CxT<R>::T);
   // finite data in the grid buffers (their contents are scratch between matvecs)
-  DDA_TRY_HIP(hipMemsetAsync(op->a1, 0, 3ull * d.Bz * d.By * d.Gx * csz * nrhs, st));
-  DDA_TRY_HIP(hipMemsetAsync(op->a2, 0, 3ull * d.Bz * d.Gy * d.Gx * csz * nrhs, st));
+  DDA_TRY_HIP(hipMemsetAsync(op->a1, 0, 3ull * d.Bz * d.By * d.rs * csz * nrhs, st));
+  DDA_TRY_HIP(hipMemsetAsync(op->a2, 0, 3ull * d.Bz * d.p2 * csz * nrhs, st));
   const int reps = 5;
   char buf[160];
   dda_op_s::Tune best = op->tune;
@@ -1987,9 +2001,9 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
         cp.ncols = d.Gx;
         cp.in_len = inv ? d.Gy : d.By;
         cp.out_len = inv ? d.By : d.Gy;
-        cp.pstride_in = cp.pstride_out = d.Gx;
-        cp.bstride_in = (long long)(inv ? d.Gy : d.By) * d.Gx;
-        cp.bstride_out = (long long)(inv ? d.By : d.Gy) * d.Gx;
+        cp.pstride_in = cp.pstride_out = d.rs;
+        cp.bstride_in = inv ? d.p2 : (long long)d.By * d.rs;
+        cp.bstride_out = inv ? (long long)d.By * d.rs : d.p2;
         const void* in = inv ? op->a2 : op->a1;
         void* out = inv ? op->a1 : op->a2;
         // one launch's worth of column batches (a matvec splits larger blocks)

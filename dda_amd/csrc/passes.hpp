@@ -124,7 +124,7 @@ __attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT>::value))) void k_pass3
   const int sub = w & 3, q = w >> 2;
   const int rhs = q % nrhs, grp = q / nrhs;
   if (stopped(fl, rhs)) return;
-  a2 += (long long)rhs * 3 * d.Bz * d.Gy * d.Gx;
+  a2 += (long long)rhs * 3 * d.Bz * d.p2;
   if (d.dhat_tab) dhat = (const typename CxT<R>::T*)d.dhat_tab[d.member[rhs]];
   const int ft = grp % ftn, fyp = grp / ftn;
   int ky = fyp, tile_x = ft;
@@ -142,9 +142,9 @@ __attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT>::value))) void k_pass3
   const int l = threadIdx.x % T, t = threadIdx.x / T;
   const int kx = tile_x * T + l;
   const bool colok = kx < d.Gx;
-  const long long cstride = (long long)d.Bz * d.Gy * d.Gx;
-  const uint32_t zstride = (uint32_t)d.Gy * d.Gx;
-  C* base = a2 + (long long)ky * d.Gx + (long long)tile_x * T;
+  const long long cstride = (long long)d.Bz * d.p2;
+  const uint32_t zstride = (uint32_t)d.p2;
+  C* base = a2 + (long long)ky * d.rs + (long long)tile_x * T;
   // lanes of columns beyond Gx address past every range
   const uint32_t voff = colok ? ((uint32_t)t * zstride + l) * (uint32_t)sizeof(C) : 0xfffffff0u;
   auto range = [&](const C* b, int c, int e) {
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(BS) void k_pass1s(const typename CxT<R>::T* __restr
   const int rhs = blockIdx.y;
   if (stopped(fl, rhs)) return;
   x += (long long)rhs * 3 * d.S;
-  a1 += (long long)rhs * 3 * d.nrows * d.Gx;
+  a1 += (long long)rhs * 3 * d.nrows * d.rs;
   ccs += rhs * 3 * d.nmat;
   if (d.member) row_meta += (size_t)d.member[rhs] * d.nv;
   extern __shared__ char smem[];
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(BS) void k_pass1s(const typename CxT<R>::T* __restr
   __syncthreads();
   RunStages<N, TPC, false, 1, C, F, true, P::template twiddles<R>>::run(v, t, tile, lp, l, tw);
   if (g < nlines) {
-    C* dst = a1 + (size_t)g * N;
+    C* dst = a1 + (size_t)g * d.rs;
 #pragma unroll
     for (int e = 0; e < NO; e++)
       if (first_ok<N, TPC, Out>(t, e)) cstore<true>(dst + first_point<N, TPC, Out>(t, e), v[e]);
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(BS) void k_pass5s(const typename CxT<R>::T* __restr
   constexpr int NF = first_count<N, TPC, F>(), NO = first_count<N, TPC, Out>();
   const int rhs = blockIdx.y;
   if (stopped(fl, rhs)) return;
-  a1 += (long long)rhs * 3 * d.nrows * d.Gx;
+  a1 += (long long)rhs * 3 * d.nrows * d.rs;
   x += (long long)rhs * 3 * d.S;
   y += (long long)rhs * 3 * d.S;
   ccs += rhs * 3 * d.nmat;
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(BS) void k_pass5s(const typename CxT<R>::T* __restr
   const bool ok = l < LN && g < 3 * n_list;
   const int c = ok ? g / n_list : 0;
   const int row = ok ? (int)row_list[g - c * n_list] : 0;
-  const C* src = a1 + ((size_t)c * d.nrows + row) * N;
+  const C* src = a1 + ((size_t)c * d.nrows + row) * d.rs;
   C v[PPT];
 #pragma unroll
   for (int e = 0; e < NF; e++)
@@ -554,8 +554,8 @@ inline MvView view_of(const dda_op_s* op, int r0) {
   const MvDims& d = op->dims;
   const size_t csz = op->prec == 64 ? sizeof(double2) : sizeof(float2);
   MvView v;
-  v.a1 = (char*)op->a1 + (size_t)r0 * 3 * d.Bz * d.By * d.Gx * csz;
-  v.a2 = (char*)op->a2 + (size_t)r0 * 3 * d.Bz * d.Gy * d.Gx * csz;
+  v.a1 = (char*)op->a1 + (size_t)r0 * 3 * d.Bz * d.By * d.rs * csz;
+  v.a2 = (char*)op->a2 + (size_t)r0 * 3 * d.Bz * d.p2 * csz;
   v.ccs = (const char*)op->ccs + (size_t)r0 * 3 * d.nmat * csz;
   v.d = d;
   if (d.member) v.d.member = d.member + r0;
