@@ -12,8 +12,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "_lib", "libdda_hip.so")
-# plans.hip is compiled in eight parts (DDA_PLAN_PART)
-SOURCES = ["matvec.hip"] + ["plans.hip:%d" % p for p in range(8)] + ["api.hip", "krylov.hip", "observe.hip", "server.cpp"]
+# plans.hip is compiled in eight parts, tensor.hip in four (DDA_PLAN_PART)
+SOURCES = ["matvec.hip"] + ["plans.hip:%d" % p for p in range(8)] + ["tensor.hip:%d" % p for p in range(4)] + ["api.hip", "krylov.hip", "observe.hip", "server.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -32,6 +32,7 @@
 
 #include "internal.hpp"
 #include "passes.hpp"
+#include "plan_list.hpp"
 
 namespace dda {
 
@@ -536,10 +537,6 @@ dda_status launch_row(void* data, long long nlines, const FftPlan& p, const void
   return DDA_OK;
 }
 
-// Lengths with a static plan and tuned variants. Other lengths run the one plan
-// that plans.hip holds for them (axis_ops), or the run-time planned kernels.
-#define DDA_STATIC_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(512) X(1024)
-
 inline bool has_static_plan(int n) {
   switch (n) {
 #define X(N) case N:
@@ -595,6 +592,19 @@ static const AxisOps* axis_ops(int n, int prec) {
 #define X(P) \
   if (const AxisOps* o = axis_ops_part##P(n, prec)) return o;
   DDA_PARTS(X)
+#undef X
+  return nullptr;
+}
+
+#define X(P) const TensorOps* tensor_ops_part##P(int n);
+X(0) X(1) X(2) X(3)
+#undef X
+
+// The launchers of the tensor's passes for length n, or null.
+static const TensorOps* tensor_ops(int n) {
+#define X(P) \
+  if (const TensorOps* o = tensor_ops_part##P(n)) return o;
+  X(0) X(1) X(2) X(3)
 #undef X
   return nullptr;
 }
@@ -882,25 +892,46 @@ template dda_status launch_matvec<float>(dda_op_s*, const void*, void*, int, hip
 template dda_status launch_matvec<double>(dda_op_s*, const void*, void*, int, hipStream_t, const int*, int, int,
                                           double*, int);
 
-// Generate the octant of the FFT'd, d^3-scaled tensor on the device in FP64:
-// fill one component on the full grid, 3-D FFT (X rows, Y and Z columns), keep
-// the octant times -1/N, converted to the operator's precision.
-// clip: offsets with |offset| >= clip per axis are zero (the reference clips at
-// the box; a tensor clipped anywhere between the box and G/2 gives the same
-// products for every dipole inside the box). Writes the octant into dst in the
-// operator's precision.
+// The octant of the FFT'd, d^3-scaled tensor, generated on the device in FP64,
+// times -1/N and in the operator's precision, into dst. clip: offsets with
+// |offset| >= clip per axis are zero (the reference clips at the box; a tensor
+// clipped anywhere between the box and G/2 gives the same products for every
+// dipole inside the box).
 static dda_status generate_dhat(dda_op_s* op, int cx, int cy, int cz, void* dst) {
   const MvDims& d = op->dims;
   hipStream_t st = op->ctx->stream;
+  const int g[3] = {d.Gx, d.Gy, d.Gz};
+  // grids with a planned length on every axis by octants (tensor.hip), others
+  // whole, one component after the other, with the run-time planned transforms
+  const TensorOps* ops[3];
+  for (int a = 0; a < 3; a++) ops[a] = std::getenv("DDA_GENERIC_FFT") ? nullptr : tensor_ops(g[a]);
+  const bool oct = ops[0] && ops[1] && ops[2];
   const long long total = (long long)d.Gx * d.Gy * d.Gz;
-  double2* w = nullptr;
-  DDA_TRY_HIP(hipMalloc(&w, total * sizeof(double2)));
+  const long long hx = d.Gx / 2 + 1, plane = hx * (d.Gy / 2 + 1), octn = plane * (d.Gz / 2 + 1);
+  // the double-precision tensor is formed where it stays
+  double2* w = oct && op->prec == 64 ? (double2*)dst : nullptr;
+  const bool own = w == nullptr;
+  if (own) DDA_TRY_HIP(hipMalloc(&w, (oct ? 6 * cz * plane : total) * sizeof(double2)));
   void* tw64[3] = {nullptr, nullptr, nullptr};
   dda_status rc = DDA_OK;
-  for (int a = 0; a < 3 && rc == DDA_OK; a++) rc = make_twiddles(op->plan[a].n, 64, &tw64[a], st);
+  for (int a = 0; a < 3 && rc == DDA_OK; a++) {
+    if (op->prec == 64)
+      tw64[a] = op->tw[a];
+    else
+      rc = make_twiddles(g[a], 64, &tw64[a], st);
+  }
   const double kd = op->wave_num * op->grid_unit;
   const double scale = -1.0 / (double)total;
-  for (int comp = 0; comp < 6 && rc == DDA_OK; comp++) {
+  if (rc == DDA_OK && oct) {
+    const long long cs = own ? cz * plane : octn;
+    rc = ops[0]->rows(w, cx, cy, cz, kd, cs, plane, tw64[0], st);
+    // xx, xy, xz, yy, yz, zz: xy and yz are odd in y, xz and yz in z
+    TensorCols tc = {(int)hx, cy, cz, 0x12, hx, plane, cs, cs, 1.0};
+    if (rc == DDA_OK) rc = ops[1]->cols(w, w, 64, tc, tw64[1], st);
+    tc = {(int)plane, cz, 1, 0x14, plane, 0, cs, octn, scale};
+    if (rc == DDA_OK) rc = ops[2]->cols(w, dst, op->prec, tc, tw64[2], st);
+  }
+  for (int comp = 0; comp < 6 && rc == DDA_OK && !oct; comp++) {
     hipLaunchKernelGGL(k_green_fill, dim3(2048), dim3(256), 0, st, w, comp, d.Gx, d.Gy, d.Gz, cx, cy, cz, kd);
     rc = launch_row<double>(w, (long long)d.Gy * d.Gz, op->plan[0], tw64[0], st);
     if (rc != DDA_OK) break;
@@ -931,8 +962,8 @@ static dda_status generate_dhat(dda_op_s* op, int cx, int cy, int cz, void* dst)
   }
   hipError_t e = hipStreamSynchronize(st);
   for (int a = 0; a < 3; a++)
-    if (tw64[a]) (void)hipFree(tw64[a]);
-  (void)hipFree(w);
+    if (tw64[a] && tw64[a] != op->tw[a]) (void)hipFree(tw64[a]);
+  if (own) (void)hipFree(w);
   if (rc != DDA_OK) return rc;
   DDA_TRY_HIP(e);
   return DDA_OK;

@@ -746,4 +746,21 @@ struct AxisOps {
                   RhsFlags done, int nrhs, const PassDotReq& dr);
 };
 
+// The column passes of the interaction tensor's generation: nb batches of ncols
+// columns of each of the six components; offsets below clip are read, bit c of
+// odd is set for components that are odd in the axis.
+struct TensorCols {
+  int ncols, clip, nb;
+  unsigned odd;
+  long long pstride, bstride, cstride_in, cstride_out;
+  double scale;
+};
+
+// The launchers of those passes at one grid length (tensor.hip).
+struct TensorOps {
+  dda_status (*rows)(void* w, int cx, int cy, int cz, double kd, long long cstride, long long zstride, const void* tw,
+                     hipStream_t st);
+  dda_status (*cols)(const void* in, void* out, int out_prec, const TensorCols& tc, const void* tw, hipStream_t st);
+};
+
 }  // namespace dda
