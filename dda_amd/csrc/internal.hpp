@@ -196,6 +196,13 @@ struct dda_op_s {
     std::vector<int> member_host;
   } pack;
   void* pos_dev = nullptr;      // [nv][3] positions, uploaded on first use by the observables
+  // the positions as the far field of many directions takes them (observe.hip)
+  struct Far {
+    bool made = false;
+    int npos = 0, nchunk = 0;
+    const void *segs = nullptr, *wave_seg = nullptr;
+  } far;
+  void* far_dev = nullptr;
   void* obs_scratch = nullptr;  // observables' work space
   size_t obs_bytes = 0;  // dda_op_tune ran (an FP32 twin of a tuned operator is tuned too)
   bool static_x = false;  // X passes with a compile-time plan (Gx has one)

@@ -1240,7 +1240,8 @@ static void free_op(dda_op_s* op) {
   if (op->pack.dhat_tab) (void)hipFree(op->pack.dhat_tab);
   if (op->pack.member_dev) (void)hipFree(op->pack.member_dev);
   void* bufs[] = {op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->dhat, op->a1,
-                  op->a2, op->tw[0], op->tw[1], op->tw[2], op->stage_x, op->stage_y, op->pos_dev, op->obs_scratch};
+                  op->a2, op->tw[0], op->tw[1], op->tw[2], op->stage_x, op->stage_y, op->pos_dev, op->far_dev,
+                  op->obs_scratch};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   delete op;

@@ -6,9 +6,10 @@
 // (DDA/FarFieldCalc.cpp:119-174, EMSim/JonesCalculus.cpp:74-86). The reference
 // evaluates the far field one direction per launch with a host read-back
 // (DDA/GpuFieldCalculator.cpp:64-72); here all directions and right-hand sides
-// go through one two-stage reduction.
+// go through one two-stage reduction, many directions as a matrix product.
 #include <cmath>
 #include <complex>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -182,6 +183,274 @@ __global__ void k_far_final(const double* __restrict__ part, const double* __res
   }
 }
 
+// ------------------------------------------------------------------------------------
+// Many directions, on the matrix cores.
+//
+// On the grid exp(-i kd n . r) = ex[x] ey[y] ez[z], so a direction needs
+// Bx / 2 + By + Bz sincos and not one per dipole (k_far_tables), and a row's
+// sum over x is multiplied by ey ez once. With coordinates from the box's
+// centre, the dipoles p+ at x and p- at -x of a row make
+//   p+ e^-iu + p- e^iu = (p+ + p-) cos u - i (p+ - p-) sin u,
+// half the multiplications. What is left is a real product
+// [values of a row's positions] x [cos, sin of the positions for 64 directions],
+// in 16 x 16 x 4 FP64 matrix instructions: 16 rows for the real and imaginary
+// parts of up to six values (of them 12 are used), two positions, 16 directions.
+//
+// The sphere 40 across (33,552 dipoles, 5,551 directions, both solutions) takes
+// 148 us; its instructions alone take 80 at the 74 TFLOP/s that a large product
+// reaches. What is left is the rows' ey ez (a fifth of the FP64 work) and the
+// last round of work-groups. The same sums on the vector units, whole rows of
+// dipoles from scalar loads and 24 multiply-adds per dipole, took 264 us, a
+// sincos per dipole and direction (k_far_partial) 1,480.
+// ------------------------------------------------------------------------------------
+
+constexpr int kFarWaves = 8;
+
+// The angle grid of dda_jones: sin and cos of theta and phi, and the frame.
+struct FarGrid {
+  const double* trig;  // [ntheta][sin, cos], [nphi][sin, cos]
+  int ntheta, nphi, symmetric;
+  double prop[3], pol1[3], pol2[3];
+};
+// Where a slot's direction comes from: dirs ([slot][3]) or, where that is
+// null, the angle grid (slot = angle, or 2 * angle + evaluation where symmetric).
+struct FarDirs {
+  const double* dirs;
+  FarGrid g;
+  int count;  // slots in use
+};
+
+// Direction n, perpendicular pe and parallel pa of evaluation f at angle i.
+__device__ inline void jones_frame(const FarGrid& g, int i, int f, double n[3], double pe[3], double pa[3]) {
+  const double* th = g.trig + 2 * (i / g.nphi);
+  const double* ph = g.trig + 2 * (g.ntheta + i % g.nphi);
+  const double st = th[0], ct = th[1], sp = ph[0], cp = ph[1];
+  const bool rot = f == 1 && g.symmetric;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const double X = rot ? g.pol1[a] : g.pol2[a], Y = rot ? -g.pol2[a] : g.pol1[a];
+    n[a] = ct * g.prop[a] + st * (cp * X + sp * Y);
+    pe[a] = sp * X - cp * Y;
+    pa[a] = -st * g.prop[a] + ct * (cp * X + sp * Y);
+  }
+}
+__device__ inline void far_direction(const FarDirs& f, int slot, double n[3]) {
+  if (f.dirs) {
+    for (int a = 0; a < 3; a++) n[a] = f.dirs[3 * slot + a];
+  } else {
+    double pe[3], pa[3];
+    if (f.g.symmetric)
+      jones_frame(f.g, slot >> 1, slot & 1, n, pe, pa);
+    else
+      jones_frame(f.g, slot, 0, n, pe, pa);
+  }
+}
+
+// Part of a row: positions u0, u0 + 1, .. of its folded half (u = 0 at the
+// centre), two a step; its records and those of the next segment are back to back.
+struct FarSeg {
+  int u0, steps, y, z;
+};
+
+// Tables of slots slot0 .. slot0 + nslots - 1. cs: cos and sin of kd n_x u, u < nu,
+// as the matrix instructions read them, [slot / 64][u][slot / 16 % 4][cos, sin][16];
+// yz[entry][slot]: exp(-i kd n_y y), then those of z.
+__global__ __launch_bounds__(64) void k_far_tables(FarDirs f, int slot0, int nslots, int nu, double u_first, int By,
+                                                   int Bz, double kd, double* cs, double2* yz) {
+  const int s = blockIdx.x * 64 + threadIdx.x;
+  double n[3] = {0, 0, 0};
+  if (slot0 + s < f.count) far_direction(f, slot0 + s, n);
+  const int ne = nu + By + Bz;
+  for (int e = blockIdx.y; e < ne; e += gridDim.y) {
+    double si, co;
+    if (e < nu) {
+      sincos(kd * n[0] * (e + u_first), &si, &co);
+      double* c = cs + (((long long)blockIdx.x * nu + e) * 4 + (threadIdx.x >> 4)) * 32 + (threadIdx.x & 15);
+      c[0] = co;
+      c[16] = si;
+    } else {
+      const int i = e - nu;
+      const double r = i < By ? i - 0.5 * (By - 1) : i - By - 0.5 * (Bz - 1);
+      sincos(-kd * (i < By ? n[1] : n[2]) * r, &si, &co);
+      yz[(long long)i * nslots + s] = make_double2(co, si);
+    }
+  }
+}
+
+// Records of the positions (pair: the dipoles at +u and -u, -1 for none):
+// rec[position][cos, sin][16], the factors of cos u and sin u in the matrix
+// instruction's 16 rows. Lane l holds rows l / 16 + 4 v, v = 0 .. 3, of the
+// result: real and imaginary part of value l / 16 (v = 0, 1), of value
+// 4 + l / 16 (v = 2, 3). Right-hand sides NR * blockIdx.y on.
+template <int NR>
+__global__ __launch_bounds__(256) void k_far_pack(const double2* __restrict__ pol, const int2* __restrict__ pair,
+                                                  int npos, int S, double* __restrict__ rec) {
+  pol += (long long)blockIdx.y * 3 * NR * S;
+  rec += (long long)blockIdx.y * npos * 32;
+  for (long long k = blockIdx.x * 256ll + threadIdx.x; k < 16ll * npos; k += gridDim.x * 256ll) {
+    const int q = (int)(k >> 4), i = (int)(k & 15);
+    const int n = (i & 3) + (i >= 8 ? 4 : 0);
+    double c = 0, s = 0;
+    if (n < 3 * NR) {
+      const int2 d = pair[q];
+      const double2 a = d.x >= 0 ? pol[(long long)n * S + d.x] : make_double2(0, 0);
+      const double2 b = d.y >= 0 ? pol[(long long)n * S + d.y] : make_double2(0, 0);
+      c = (i & 4) ? a.y + b.y : a.x + b.x;
+      s = (i & 4) ? b.x - a.x : a.y - b.y;
+    }
+    rec[(long long)q * 32 + i] = c;
+    rec[(long long)q * 32 + 16 + i] = s;
+  }
+}
+
+typedef double far4 __attribute__((ext_vector_type(4)));
+
+// Sums of 64 directions over the segments of one chunk of waves:
+// part[(chunk * 6 NR + value) * nslots + slot]. Wave w of chunk b takes segments
+// wave_seg[w] .. wave_seg[w + 1], w = 8 b + wave; their records are a stream,
+// read three steps ahead. Four tiles of 16 directions share each record; their
+// cos and sin come from LDS (LDSX) or, for boxes too long for it, from L2.
+// Records: those of right-hand side rhs[tile] - r0, or (rhs null) of the only one.
+template <int NR, bool LDSX>
+__global__ __launch_bounds__(64 * kFarWaves) void k_far_rows(const double* __restrict__ rec, int npos,
+                                                             const FarSeg* __restrict__ segs,
+                                                             const int2* __restrict__ wave_seg,
+                                                             const double* __restrict__ cs,
+                                                             const double2* __restrict__ yz, int nu, int By, int nslots,
+                                                             const int* __restrict__ rhs, int r0,
+                                                             double* __restrict__ part) {
+  extern __shared__ __align__(16) char smem[];
+  const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const double* ct = cs + (long long)blockIdx.x * nu * 128;
+  if (LDSX) {
+    double2* t = reinterpret_cast<double2*>(smem);
+    for (int i = threadIdx.x; i < nu * 64; i += 64 * kFarWaves) t[i] = reinterpret_cast<const double2*>(ct)[i];
+    __syncthreads();
+    ct = reinterpret_cast<const double*>(smem);
+  }
+  // instruction operand k = g: position g / 2 of the step, cos or sin
+  ct += (g >> 1) * 128 + (g & 1) * 16 + j;
+  if (rhs) rec += (long long)(rhs[blockIdx.x] - r0) * npos * 32;
+  const int2 ws = wave_seg[blockIdx.y * kFarWaves + wave], we = wave_seg[blockIdx.y * kFarWaves + wave + 1];
+  const double* r = rec + (long long)ws.y * 32 + lane;
+  double acc_r[4][NR], acc_i[4][NR];
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int h = 0; h < NR; h++) acc_r[t][h] = acc_i[t][h] = 0;
+  double a0 = r[0], a1 = r[64], a2 = r[128];
+  for (int q = ws.x; q < we.x; q++) {
+    const FarSeg sg = segs[q];
+    const double* b = ct + sg.u0 * 128;
+    far4 T[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) T[t] = (far4)(0.0);
+    for (int s = 0; s < sg.steps; s++, b += 256) {
+      const double a = a0;
+      a0 = a1;
+      a1 = a2;
+      r += 64;
+      a2 = r[128];
+#pragma unroll
+      for (int t = 0; t < 4; t++) T[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b[t * 32], T[t], 0, 0, 0);
+    }
+    const double2* py = yz + (long long)sg.y * nslots + blockIdx.x * 64 + j;
+    const double2* pz = yz + (long long)(By + sg.z) * nslots + blockIdx.x * 64 + j;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const double2 w = cmul(py[t * 16], pz[t * 16]);
+#pragma unroll
+      for (int h = 0; h < NR; h++) {
+        acc_r[t][h] = ffma(T[t][2 * h], w.x, ffma(-T[t][2 * h + 1], w.y, acc_r[t][h]));
+        acc_i[t][h] = ffma(T[t][2 * h], w.y, ffma(T[t][2 * h + 1], w.x, acc_i[t][h]));
+      }
+    }
+  }
+  // the waves' sums, in their order
+  constexpr int NV = 6 * NR;
+  double* red = reinterpret_cast<double*>(smem);
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < NR; h++)
+    if (4 * h + g < 3 * NR)
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        double* d = red + (wave * NV + 2 * (4 * h + g)) * 64 + t * 16 + j;
+        d[0] = acc_r[t][h];
+        d[64] = acc_i[t][h];
+      }
+  __syncthreads();
+  for (int v = wave; v < NV; v += kFarWaves) {
+    double t = 0;
+    for (int w = 0; w < kFarWaves; w++) t += red[(w * NV + v) * 64 + lane];
+    part[((long long)blockIdx.y * NV + v) * nslots + blockIdx.x * 64 + lane] = t;
+  }
+}
+
+// Last stage, 64 slots per work-group of 64 * 6 NR threads: the chunks' sums in
+// their order, then E = i k^2 (S - n (n . S)) of each slot: to out[6 * query]
+// (query: the slots' places, -1 for none), or on the angle grid the Jones
+// matrices of the two evaluations of each angle, out[8 * angle].
+template <int NR>
+__global__ __launch_bounds__(384 * NR) void k_far_last(const double* __restrict__ part, FarDirs f, int slot0,
+                                                       int nslots, int nchunk, double k, const int* __restrict__ query,
+                                                       double* __restrict__ out) {
+  constexpr int NV = 6 * NR;
+  __shared__ double sh[NV][64];
+  const int lane = threadIdx.x & 63, v = threadIdx.x >> 6;
+  const int s = blockIdx.x * 64 + lane;
+  double t = 0;
+  for (int b = 0; b < nchunk; b++) t += part[((long long)b * NV + v) * nslots + s];
+  sh[v][lane] = t;
+  __syncthreads();
+  const int slot = slot0 + s;
+  if (v != 0 || slot >= f.count) return;
+  // field of right-hand side r of lane l in direction n
+  auto field = [&](int r, int l, const double n[3], double e[6]) {
+    double nr = 0, ni = 0;
+    for (int a = 0; a < 3; a++) {
+      nr += n[a] * sh[6 * r + 2 * a][l];
+      ni += n[a] * sh[6 * r + 2 * a + 1][l];
+    }
+    for (int a = 0; a < 3; a++) {
+      e[2 * a] = -k * k * (sh[6 * r + 2 * a + 1][l] - n[a] * ni);
+      e[2 * a + 1] = k * k * (sh[6 * r + 2 * a][l] - n[a] * nr);
+    }
+  };
+  double n[3], e[6];
+  if (f.dirs) {
+    if (query[slot] < 0) return;
+    far_direction(f, slot, n);
+    field(0, lane, n, e);
+    for (int a = 0; a < 6; a++) out[6ll * query[slot] + a] = e[a];
+    return;
+  }
+  if (f.g.symmetric && (lane & 1)) return;
+  const int i = f.g.symmetric ? slot >> 1 : slot;
+  double2 perp[2], par[2];
+  for (int q = 0; q < 2; q++) {
+    double pe[3], pa[3];
+    jones_frame(f.g, i, q, n, pe, pa);
+    field(NR == 2 ? q : 0, NR == 2 ? lane : lane + q, n, e);
+    perp[q] = par[q] = make_double2(0, 0);
+    for (int a = 0; a < 3; a++) {
+      perp[q].x += e[2 * a] * pe[a];
+      perp[q].y += e[2 * a + 1] * pe[a];
+      par[q].x += e[2 * a] * pa[a];
+      par[q].y += e[2 * a + 1] * pa[a];
+    }
+  }
+  const double sp = f.g.trig[2 * (f.g.ntheta + i % f.g.nphi)], cp = f.g.trig[2 * (f.g.ntheta + i % f.g.nphi) + 1];
+  const double2 J[4] = {cadd(cscale(par[1], cp), cscale(par[0], sp)), csub(cscale(par[1], sp), cscale(par[0], cp)),
+                        cadd(cscale(perp[1], cp), cscale(perp[0], sp)),
+                        csub(cscale(perp[1], sp), cscale(perp[0], cp))};
+  for (int j = 0; j < 4; j++) {
+    out[8ll * i + 2 * j] = J[j].x;
+    out[8ll * i + 2 * j + 1] = J[j].y;
+  }
+}
+
 Frame frame_of(const dda_op_s* op) {
   const MvDims& d = op->dims;
   Frame f;
@@ -218,6 +487,160 @@ dda_status obs_scratch(dda_op_s* op, size_t bytes, void** out) {
     op->device_bytes += bytes;
   }
   *out = op->obs_scratch;
+  return DDA_OK;
+}
+
+// The operator's positions as k_far_rows takes them, made on first use: the
+// folded halves of the occupied rows, each from its innermost to its outermost
+// dipole, in segments of at most 32 steps, dealt to the waves in equal numbers of
+// steps. far.npos stays 0 where the rows are mostly holes (four positions and
+// more per dipole) or two dipoles share a position: those go by k_far_partial.
+dda_status far_segments(dda_op_s* op) {
+  dda_op_s::Far& far = op->far;
+  if (far.made) return DDA_OK;
+  const MvDims& d = op->dims;
+  const int nrows = d.nrows, c2 = d.Bx - 1;  // twice the centre
+  auto fold = [&](int x) { return std::abs(2 * x - c2) / 2; };
+  std::vector<int> lo(nrows, d.Bx), hi(nrows, -1), first(nrows);
+  for (int i = 0; i < d.nv; i++) {
+    const uint32_t* p = &op->pos[3 * (size_t)i];
+    const int r = p[2] * d.By + p[1], u = fold(p[0]);
+    lo[r] = std::min(lo[r], u);
+    hi[r] = std::max(hi[r], u);
+  }
+  std::vector<FarSeg> segs;
+  long long npos = 0;
+  for (int r = 0; r < nrows; r++) {
+    first[r] = (int)std::min<long long>(npos, INT32_MAX);
+    for (int u = lo[r]; u <= hi[r]; u += 64) {
+      FarSeg sg = {u, std::min(32, (hi[r] - u + 2) / 2), r % d.By, r / d.By};
+      segs.push_back(sg);
+      npos += 2 * sg.steps;
+    }
+  }
+  far.made = true;
+  if (npos > 4ll * d.nv + 64 || npos > (1 << 26)) return DDA_OK;
+  std::vector<int2> pair(npos, make_int2(-1, -1));
+  for (int i = 0; i < d.nv; i++) {
+    const uint32_t* p = &op->pos[3 * (size_t)i];
+    const int r = p[2] * d.By + p[1], x = p[0];
+    int2& q = pair[first[r] + fold(x) - lo[r]];
+    int& at = 2 * x >= c2 ? q.x : q.y;
+    if (at >= 0) return DDA_OK;
+    at = i;
+  }
+  const long long steps = npos / 2;
+  // 64 steps a wave, at most 64 work-groups' worth of waves
+  far.nchunk = (int)std::min<long long>(64, (steps + 64 * kFarWaves - 1) / (64 * kFarWaves));
+  const int nw = far.nchunk * kFarWaves;
+  std::vector<int2> ws(nw + 1);
+  long long at = 0;
+  size_t q = 0;
+  for (int w = 0; w <= nw; w++) {
+    while (q < segs.size() && at < steps * w / nw) at += segs[q++].steps;
+    ws[w] = make_int2((int)q, (int)(2 * at));
+  }
+  // (records are read three steps ahead, from one position buffer per batch)
+  const size_t pb = (pair.size() * sizeof(int2) + 15) / 16 * 16, sb = segs.size() * sizeof(FarSeg);
+  const size_t wb = ws.size() * sizeof(int2);
+  DDA_TRY_HIP(hipMalloc(&op->far_dev, pb + sb + wb));
+  op->device_bytes += pb + sb + wb;
+  char* dev = (char*)op->far_dev;
+  hipStream_t st = op->ctx->stream;
+  DDA_TRY_HIP(hipMemcpyAsync(dev, pair.data(), pair.size() * sizeof(int2), hipMemcpyHostToDevice, st));
+  DDA_TRY_HIP(hipMemcpyAsync(dev + pb, segs.data(), sb, hipMemcpyHostToDevice, st));
+  DDA_TRY_HIP(hipMemcpyAsync(dev + pb + sb, ws.data(), wb, hipMemcpyHostToDevice, st));
+  DDA_TRY_HIP(hipStreamSynchronize(st));
+  far.segs = dev + pb;
+  far.wave_seg = dev + pb + sb;
+  far.npos = (int)npos;
+  return DDA_OK;
+}
+
+// Work space of far_batches: the batches' tables, partial sums and records,
+// each batch's tables and sums and its records below 256 MB where they can be.
+struct FarPlan {
+  int nu;         // positions of the folded x axis, one more for the step's second
+  int per_batch;  // slots per batch, a multiple of 64
+  int recs;       // right-hand sides (NR = 2: pairs) per batch
+  size_t cs, yz, parts, bytes;
+};
+FarPlan far_plan(const dda_op_s* op, int slots, int nr, int nrec) {
+  const MvDims& d = op->dims;
+  const size_t most = 256ull << 20;
+  FarPlan p;
+  p.nu = (d.Bx + 1) / 2 + 1;
+  const size_t cs = 16ull * p.nu, yz = 16ull * (d.By + d.Bz), part = 48ull * nr * op->far.nchunk;
+  const size_t rec = 256ull * op->far.npos;
+  p.per_batch = (int)std::min<size_t>(std::max<size_t>(1, most / (64 * (cs + yz + part))), (slots + 63) / 64) * 64;
+  p.recs = (int)std::min<size_t>(std::max<size_t>(1, most / rec), std::min(nrec, 65535));
+  p.cs = cs * p.per_batch;
+  p.yz = yz * p.per_batch;
+  p.parts = part * p.per_batch;
+  p.bytes = p.cs + p.yz + p.parts + rec * p.recs + 3 * 512;  // read ahead
+  return p;
+}
+
+// The sums and last stages of the slots of f, in batches. rhs: the right-hand
+// side of each 64 slots, ascending, on the host and on the device (null: all of
+// record 0); query (device, one per slot) as k_far_last takes it; out_dev on the
+// device.
+template <int NR>
+dda_status far_batches(dda_op_s* op, const double2* pol, const FarDirs& f, const FarPlan& p, const int* rhs_host,
+                       const int* rhs, const int* query, double* out_dev, void* work) {
+  const MvDims& d = op->dims;
+  const dda_op_s::Far& far = op->far;
+  hipStream_t st = op->ctx->stream;
+  double* cs = (double*)work;
+  double2* yz = (double2*)((char*)work + p.cs);
+  double* part = (double*)((char*)yz + p.yz);
+  double* rec = (double*)((char*)part + p.parts);
+  const size_t red = sizeof(double) * kFarWaves * 6 * NR * 64, xt = 1024ull * p.nu;
+  const bool ldsx = xt <= 150 * 1024;
+  const size_t lds = ldsx ? std::max(red, xt) : red;
+  auto k = ldsx ? k_far_rows<NR, true> : k_far_rows<NR, false>;
+  if (lds > 64 * 1024)
+    DDA_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)lds));
+  const int tiles = (f.count + 63) / 64;
+  int have0 = 0, have1 = 0;  // right-hand sides whose records are there
+  for (int t0 = 0, t1; t0 < tiles; t0 = t1) {
+    const int r0 = rhs_host ? rhs_host[t0] : 0;
+    for (t1 = t0; t1 < tiles && (t1 - t0) * 64 < p.per_batch && (rhs_host ? rhs_host[t1] : 0) < r0 + p.recs;) t1++;
+    const int r1 = (rhs_host ? rhs_host[t1 - 1] : 0) + 1;
+    if (r0 < have0 || r1 > have1) {
+      have0 = r0;
+      have1 = r1;
+      hipLaunchKernelGGL(k_far_pack<NR>, dim3(std::min(1024, (16 * far.npos + 255) / 256), r1 - r0), dim3(256), 0, st,
+                         pol + (size_t)r0 * 3 * NR * d.S, (const int2*)op->far_dev, far.npos, d.S, rec);
+    }
+    const int s0 = t0 * 64, ns = (t1 - t0) * 64;
+    hipLaunchKernelGGL(k_far_tables, dim3(t1 - t0, std::min(p.nu + d.By + d.Bz, 64)), dim3(64), 0, st, f, s0, ns, p.nu,
+                       d.Bx & 1 ? 0.0 : 0.5, d.By, d.Bz, op->wave_num * op->grid_unit, cs, yz);
+    hipLaunchKernelGGL(k, dim3(t1 - t0, far.nchunk), dim3(64 * kFarWaves), lds, st, rec, far.npos,
+                       (const FarSeg*)far.segs, (const int2*)far.wave_seg, cs, yz, p.nu, d.By, ns,
+                       rhs ? rhs + t0 : nullptr, have0, part);
+    hipLaunchKernelGGL(k_far_last<NR>, dim3(t1 - t0), dim3(384 * NR), 0, st, part, f, s0, ns, far.nchunk, op->wave_num,
+                       query, out_dev);
+    DDA_TRY_HIP(hipGetLastError());
+  }
+  return DDA_OK;
+}
+
+// Whether nq field evaluations, of `slots` 64-padded slots, go by k_far_rows. Its
+// launches and tables cost what some hundred evaluations by k_far_partial do: the
+// two meet at 64 evaluations of 217,160 dipoles (113 against 118 us), 128 of
+// 94,296 (92 and 93), about 200 of 33,552 (81) and 4,096 of 280 (77 and 78), so
+// the line lies at 8 million dipole phases. A work-group's 64 directions take the
+// time of ten by k_far_partial, however many of them are in use. (4,096 of
+// 217,160 dipoles: 582 against 3,434 us.) An angle grid's directions and Jones
+// matrices are formed on the device too, which pays from 1,000 evaluations on at
+// any size (11,102 of 280 dipoles: 70 against 434 us).
+dda_status many_directions(dda_op_s* op, bool angle_grid, long long nq, long long slots, bool* many) {
+  *many = ((double)nq * op->dims.nv >= 8e6 || (angle_grid && nq >= 1000)) && 6 * nq >= slots && slots < (1ll << 30);
+  if (!*many) return DDA_OK;
+  DDA_TRY(far_segments(op));
+  *many = op->far.npos > 0;
   return DDA_OK;
 }
 
@@ -455,6 +878,48 @@ extern "C" dda_status dda_far_field(dda_op_t op, const void* pol_dev, int nrhs, 
       set_error("dda_far_field: right-hand side index out of range");
       return DDA_INVALID_ARG;
     }
+  {
+    // many directions: slots by right-hand side, each's filled up to 64
+    std::vector<int> fill(nrhs + 1, 0);
+    for (int i = 0; i < nq; i++) fill[(rhs ? rhs[i] : 0) + 1]++;
+    long long slots = 0;
+    for (int r = 0; r < nrhs; r++) {
+      const int n = fill[r + 1];
+      fill[r] = (int)slots;
+      slots += (n + 63) / 64 * 64;
+    }
+    bool many = false;
+    DDA_TRY(many_directions(op, false, nq, slots, &many));
+    if (many) {
+      std::vector<double> hd(3 * slots, 0.0);
+      std::vector<int> hi(slots + slots / 64, -1);
+      for (int i = 0; i < nq; i++) {
+        const int r = rhs ? rhs[i] : 0, s = fill[r]++;
+        for (int a = 0; a < 3; a++) hd[3 * (size_t)s + a] = dirs[3 * (size_t)i + a];
+        hi[s] = i;
+        hi[slots + s / 64] = r;
+      }
+      for (long long t = 0; t < slots / 64; t++) hi[slots + t] = std::max(0, hi[slots + t]);
+      const FarPlan plan = far_plan(op, (int)slots, 1, nrhs);
+      const size_t dbytes = hd.size() * sizeof(double), ibytes = (hi.size() + 3) / 4 * 16;
+      void* buf = nullptr;
+      DDA_TRY(obs_scratch(op, plan.bytes + dbytes + ibytes + 6ull * nq * sizeof(double), &buf));
+      double* dd = (double*)((char*)buf + plan.bytes);
+      int* id = (int*)((char*)dd + dbytes);
+      double* od = (double*)((char*)id + ibytes);
+      hipStream_t st = op->ctx->stream;
+      DDA_TRY_HIP(hipMemcpyAsync(dd, hd.data(), dbytes, hipMemcpyHostToDevice, st));
+      DDA_TRY_HIP(hipMemcpyAsync(id, hi.data(), hi.size() * sizeof(int), hipMemcpyHostToDevice, st));
+      FarDirs f;
+      std::memset(&f, 0, sizeof f);
+      f.dirs = dd;
+      f.count = (int)slots;
+      DDA_TRY(far_batches<1>(op, (const double2*)pol_dev, f, plan, hi.data() + slots, id + slots, id, od, buf));
+      DDA_TRY_HIP(hipMemcpyAsync(out, od, 6ull * nq * sizeof(double), hipMemcpyDeviceToHost, st));
+      DDA_TRY_HIP(hipStreamSynchronize(st));
+      return DDA_OK;
+    }
+  }
   DDA_TRY(positions_on_device(op));
   const MvDims& d = op->dims;
   const int chunk = 4096;
@@ -493,6 +958,44 @@ extern "C" dda_status dda_jones(dda_op_t op, const void* pol_dev, int symmetric,
   }
   DDA_TRY(one_wave_number(op, "dda_jones"));
   const size_t count = (size_t)ntheta * nphi;
+  const size_t slots = symmetric ? 2 * count : count;
+  DDA_TRY(bind_device(op->ctx));
+  bool many = false;
+  DDA_TRY(many_directions(op, true, 2 * (long long)count, (long long)slots, &many));
+  if (many) {
+    std::vector<double> trig(2 * ((size_t)ntheta + nphi));
+    for (size_t i = 0; i < (size_t)ntheta + nphi; i++) {
+      const double a = i < ntheta ? theta0 + (double)i * dtheta : phi0 + (double)(i - ntheta) * dphi;
+      trig[2 * i] = std::sin(a);
+      trig[2 * i + 1] = std::cos(a);
+    }
+    const FarPlan plan = far_plan(op, (int)slots, symmetric ? 1 : 2, 1);
+    const size_t tbytes = trig.size() * sizeof(double);
+    void* buf = nullptr;
+    DDA_TRY(obs_scratch(op, plan.bytes + tbytes + 8 * count * sizeof(double), &buf));
+    double* td = (double*)((char*)buf + plan.bytes);
+    double* od = (double*)((char*)td + tbytes);
+    hipStream_t st = op->ctx->stream;
+    DDA_TRY_HIP(hipMemcpyAsync(td, trig.data(), tbytes, hipMemcpyHostToDevice, st));
+    FarDirs f;
+    std::memset(&f, 0, sizeof f);
+    f.g.trig = td;
+    f.g.ntheta = (int)ntheta;
+    f.g.nphi = (int)nphi;
+    f.g.symmetric = symmetric;
+    for (int a = 0; a < 3; a++) {
+      f.g.prop[a] = prop[a];
+      f.g.pol1[a] = pol1[a];
+      f.g.pol2[a] = pol2[a];
+    }
+    f.count = (int)slots;
+    const double2* pol = (const double2*)pol_dev;
+    DDA_TRY(symmetric ? far_batches<1>(op, pol, f, plan, nullptr, nullptr, nullptr, od, buf)
+                      : far_batches<2>(op, pol, f, plan, nullptr, nullptr, nullptr, od, buf));
+    DDA_TRY_HIP(hipMemcpyAsync(out, od, 8 * count * sizeof(double), hipMemcpyDeviceToHost, st));
+    DDA_TRY_HIP(hipStreamSynchronize(st));
+    return DDA_OK;
+  }
   // two field evaluations per angle: (p1; X = pol2, Y = pol1) and
   // (p2; X = pol2, Y = pol1) or, for a symmetric target, (p1; X = pol1, Y = -pol2)
   std::vector<double> dirs(6 * count), pe(12 * count), pa(12 * count);

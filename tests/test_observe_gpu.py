@@ -125,3 +125,53 @@ def test_anisotropic_material_solve_and_hdf5_output(ctx, tmp_path):
         np.testing.assert_array_equal(mats[0], g.materials[0])
     s.close()
     op.close()
+
+
+def _random_pol(ctx, op, k, seed):
+    rng = np.random.default_rng(seed)
+    p = rng.normal(size=(k, 3, op.vec_stride)) + 1j * rng.normal(size=(k, 3, op.vec_stride))
+    p[:, :, op.nv:] = 0
+    v = D.DeviceVector(ctx, k * op.vec_size, 64)
+    v.upload(p.reshape(-1))
+    return v
+
+
+# box, kept cells: even and odd x extents, rows on one side of the centre, rows with holes,
+# single cells, rows of more than one segment, x extents beyond the LDS table
+FAR_CASES = [((30, 20, 20), lambda x, y, z: x >= 0), ((31, 21, 19), lambda x, y, z: x >= 0),
+             ((33, 20, 30), lambda x, y, z: x > 20), ((40, 24, 30), lambda x, y, z: (x % 3 == y % 3) & (x < 33)),
+             ((1, 110, 90), lambda x, y, z: x >= 0), ((512, 6, 6), lambda x, y, z: (x + y) % 5 != 0),
+             ((301, 7, 5), lambda x, y, z: x >= 0), ((140, 9, 8), lambda x, y, z: x != 71)]
+
+
+@pytest.mark.parametrize("box,keep", FAR_CASES)
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_many_directions_match_few(ctx, box, keep, shuffled):
+    """Fields and Jones matrices of many directions (matrix instructions over
+    folded rows) against those of a few at a time (one sincos per dipole and
+    direction), for three right-hand sides. Both carry some roundings of phases
+    of up to 100 radians and of sums of 10^4 terms: 1e-12 of the largest field."""
+    print("box", box, "shuffled", shuffled, flush=True)
+    z, y, x = np.meshgrid(*(np.arange(b) for b in box[::-1]), indexing="ij")
+    pos = np.stack([a[keep(x, y, z)] for a in (x, y, z)], 1)
+    rng = np.random.default_rng(5)
+    if shuffled:
+        pos = pos[rng.permutation(len(pos))]
+    op = D.GpuMatVec(ctx, pos, None, box, 0.5e-6, 0.4 / 0.5e-6, nmat=1)
+    pol = _random_pol(ctx, op, 3, 1)
+    nq = 8_000_000 // len(pos) + 70
+    dirs = rng.normal(size=(nq, 3))
+    dirs /= np.linalg.norm(dirs, axis=1)[:, None]
+    rhs = rng.integers(0, 3, nq)
+    got = D.far_field(op, pol, 3, dirs, rhs)
+    ref = np.concatenate([D.far_field(op, pol, 3, dirs[i:i + 40], rhs[i:i + 40]) for i in range(0, nq, 40)])
+    tol = 1e-12 * np.abs(ref).max()
+    assert np.abs(got - ref).max() <= tol
+    prop, pol1, pol2 = P.beam_pols((0.3, -0.2, 0.8))
+    nt, nf = nq // 22 + 2, 11
+    for symmetric in (0, 1):
+        J = D.jones(op, pol, symmetric, prop, pol1, pol2, nt, 0.1, 0.03, nf, 0.2, 0.5)
+        for i in range(0, nt, 7):  # one theta at a time: few directions
+            Jr = D.jones(op, pol, symmetric, prop, pol1, pol2, 1, 0.1 + i * 0.03, 0.0, nf, 0.2, 0.5)
+            assert np.abs(J.reshape(nt, nf, 2, 2)[i] - Jr.reshape(nf, 2, 2)).max() <= 2 * tol
+    op.close()
