@@ -144,6 +144,7 @@ struct dda_op_s {
   uint32_t* row_start = nullptr;  // [nrows + 1]
   uint32_t* row_dip = nullptr;    // [nv] dipole index, grouped by row
   uint32_t* row_meta = nullptr;   // [nv] x | mat << 16
+  uint32_t* cell = nullptr;       // [Bz][By][Bx] dipole at each cell (compile-time planned X passes)
   uint32_t* row_list = nullptr;   // rows holding at least one dipole
   uint8_t* mat_dev = nullptr;     // [nv] material index per dipole
   int n_nonempty = 0;

@@ -1239,7 +1239,7 @@ static void free_op(dda_op_s* op) {
   }
   if (op->pack.dhat_tab) (void)hipFree(op->pack.dhat_tab);
   if (op->pack.member_dev) (void)hipFree(op->pack.member_dev);
-  void* bufs[] = {op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->dhat, op->a1,
+  void* bufs[] = {op->cell, op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->dhat, op->a1,
                   op->a2, op->tw[0], op->tw[1], op->tw[2], op->stage_x, op->stage_y, op->pos_dev, op->far_dev,
                   op->obs_scratch};
   for (void* b : bufs)
@@ -1342,6 +1342,20 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
     op->static_z = op->gen[2] || static_z_fits(d.Gx, d.Gy, d.Gz, csz);
     op->static_x = op->gen[0] || has_static_plan(d.Gx);
   }
+  // the cell map; dipoles that share a cell go by the rows' lists
+  std::vector<uint32_t> cell;
+  if (op->static_x) {
+    cell.assign((size_t)d.nrows * d.Bx, kNoDipole);
+    for (uint32_t i = 0; i < ds.nv && op->static_x; i++) {
+      const uint32_t* p = &op->pos[3 * (size_t)i];
+      uint32_t& at = cell[((size_t)p[2] * d.By + p[1]) * d.Bx + p[0]];
+      if (at != kNoDipole) {
+        op->static_x = false;
+        op->gen[0] = nullptr;
+      }
+      at = i;
+    }
+  }
   op->split_rhs = std::getenv("DDA_SPLIT") && std::atoi(std::getenv("DDA_SPLIT")) != 0;
 
   // Launch shapes: X passes hold ~2048 points per work-group; column passes
@@ -1373,6 +1387,7 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
   if (rc == DDA_OK) rc = dmalloc((void**)&op->row_meta, ds.nv * 4ull);
   if (rc == DDA_OK) rc = dmalloc((void**)&op->row_list, std::max<size_t>(1, row_list.size()) * 4);
   if (rc == DDA_OK) rc = dmalloc((void**)&op->mat_dev, ds.nv);
+  if (rc == DDA_OK && op->static_x) rc = dmalloc((void**)&op->cell, cell.size() * 4);
   if (rc == DDA_OK) rc = dmalloc(&op->ccs, 3ull * ds.nmat * csz);
   if (rc == DDA_OK && (ds.dmatrix || !cache)) rc = dmalloc(&op->dhat, dn * csz);
   if (rc == DDA_OK) rc = dmalloc(&op->a1, a1n * csz);
@@ -1387,6 +1402,7 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
   if (e == hipSuccess) e = copy_sync(op->row_start, row_start.data(), row_start.size() * 4, hipMemcpyHostToDevice, cst);
   if (e == hipSuccess) e = copy_sync(op->row_dip, row_dip.data(), ds.nv * 4ull, hipMemcpyHostToDevice, cst);
   if (e == hipSuccess) e = copy_sync(op->row_meta, row_meta.data(), ds.nv * 4ull, hipMemcpyHostToDevice, cst);
+  if (e == hipSuccess && op->static_x) e = copy_sync(op->cell, cell.data(), cell.size() * 4, hipMemcpyHostToDevice, cst);
   if (e == hipSuccess && !row_list.empty())
     e = copy_sync(op->row_list, row_list.data(), row_list.size() * 4, hipMemcpyHostToDevice, cst);
   if (e == hipSuccess) e = copy_sync(op->mat_dev, op->mat.data(), ds.nv, hipMemcpyHostToDevice, cst);

@@ -12,6 +12,9 @@ namespace dda {
 
 __device__ inline bool stopped(const RhsFlags& f, int rhs) { return f.done != nullptr && f.done[rhs * f.stride] != 0; }
 
+// A cell without a dipole in the cell map.
+constexpr uint32_t kNoDipole = 0xffffffffu;
+
 // The buffers of right-hand sides r0 .. r0 + nrhs - 1 of an operator: what one
 // sequence of the five passes works on (the whole block, or one half of it
 // when the halves run on two streams).
@@ -231,16 +234,16 @@ __attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT>::value))) void k_pass3
 
 // Pass 1 with a static plan of length N = Gx. A work-group takes LN consecutive
 // lines g = c * nrows + row of the A1 layout (contiguous in A1); thread (l, t),
-// t = tid mod TPC along the line, scatters line l's dipoles into the LDS tile,
-// then runs the transform from its first-stage points (only x < N/2 can hold
-// dipoles: the upper half is never read) and stores its outputs, TPC
-// consecutive points per line, coalesced.
+// t = tid mod TPC along the line, reads its first-stage points straight from the
+// vector through the cell map (only x < Bx <= N/2 can hold dipoles) and stores
+// its outputs, TPC consecutive points per line, coalesced.
+// (With the row's dipoles scattered into a zeroed LDS tile first, two barriers
+// and two LDS trips more: 70 us at 256^3, FP64 and two FP32 right-hand sides,
+// against 57; 282 against 250 at 512^3. What is left is writing A1.)
 template <typename R, int N, typename PL, int BS = 256>
 __global__ __launch_bounds__(BS) void k_pass1s(const typename CxT<R>::T* __restrict__ x,
                                                 typename CxT<R>::T* __restrict__ a1,
-                                                const uint32_t* __restrict__ row_start,
-                                                const uint32_t* __restrict__ row_dip,
-                                                const uint32_t* __restrict__ row_meta,
+                                                const uint32_t* __restrict__ cell, const uint8_t* __restrict__ mat,
                                                 const typename CxT<R>::T* __restrict__ ccs, MvDims d,
                                                 const typename CxT<R>::T* __restrict__ tw, int conj, RhsFlags fl) {
   typedef typename CxT<R>::T C;
@@ -260,32 +263,33 @@ __global__ __launch_bounds__(BS) void k_pass1s(const typename CxT<R>::T* __restr
   x += (long long)rhs * 3 * d.S;
   a1 += (long long)rhs * 3 * d.nrows * d.rs;
   ccs += rhs * 3 * d.nmat;
-  if (d.member) row_meta += (size_t)d.member[rhs] * d.nv;
+  if (d.member) mat += (size_t)d.member[rhs] * d.nv;
   extern __shared__ char smem[];
   C* tile = reinterpret_cast<C*>(smem);
   const int t = threadIdx.x % TPC, l = threadIdx.x / TPC;
   const int nlines = 3 * d.nrows;
   const int g = l < LN ? (int)blockIdx.x * LN + l : nlines;
-  for (int i = threadIdx.x; i < (N / 2) * lp; i += blockDim.x) tile[i] = czero<C>();
-  __syncthreads();
-  if (g < nlines) {
-    const int c = g / d.nrows, row = g - c * d.nrows;
-    const uint32_t s0 = row_start[row], s1 = row_start[row + 1];
-    for (uint32_t q = s0 + t; q < s1; q += TPC) {
-      const uint32_t i = d.sorted ? q : row_dip[q], meta = row_meta[q];
-      C v = x[(size_t)c * d.S + i];
-      if (conj) v = cconj(v);
-      tile[(meta & 0xffff) * lp + l] = cmul(ccs[3 * (meta >> 16) + c], v);
-    }
+  const bool ok = g < nlines;
+  const int c = ok ? g / d.nrows : 0, row = ok ? g - c * d.nrows : 0;
+  const uint32_t* cells = cell + (size_t)row * d.Bx;
+  x += (size_t)c * d.S;
+  uint32_t at[NF];
+#pragma unroll
+  for (int e = 0; e < NF; e++) {
+    const int p = first_point<N, TPC, F>(t, e);
+    at[e] = !upper_half<F>(e) && ok && p < d.Bx && first_ok<N, TPC, F>(t, e) ? cells[p] : kNoDipole;
   }
-  __syncthreads();
   C v[PPT];
 #pragma unroll
-  for (int e = 0; e < NF; e++)
-    v[e] = upper_half<F>(e) || !first_ok<N, TPC, F>(t, e) ? czero<C>() : tile[first_point<N, TPC, F>(t, e) * lp + l];
-  __syncthreads();
+  for (int e = 0; e < NF; e++) {
+    v[e] = czero<C>();
+    if (!upper_half<F>(e) && at[e] != kNoDipole) {
+      const C xv = x[at[e]];
+      v[e] = cmul(ccs[3 * (d.nmat > 1 ? mat[at[e]] : 0) + c], conj ? cconj(xv) : xv);
+    }
+  }
   RunStages<N, TPC, false, 1, C, F, true, P::template twiddles<R>>::run(v, t, tile, lp, l, tw);
-  if (g < nlines) {
+  if (ok) {
     C* dst = a1 + (size_t)g * d.rs;
 #pragma unroll
     for (int e = 0; e < NO; e++)
@@ -326,17 +330,19 @@ __device__ inline void dot_partials(double* dot, int op, double q0, double q1, d
 }
 
 // Pass 5 with a static plan: lines g = c * n_list + slot over the non-empty
-// rows; inverse transform from A1 (loads coalesced), the kept half (x < N/2)
-// through the tile, then line l's dipoles gathered by its TPC threads.
+// rows; inverse transform from A1 (loads coalesced), the kept half (x < Bx) goes
+// from the registers of the last stage to the dipoles that the cell map names.
+// (Through an LDS tile and the rows' dipole lists: 66 us at 256^3 (two FP32
+// right-hand sides) against 58, 231 against 218 at 512^3, 168 against 159 for 128
+// right-hand sides at 128 x 96 x 64; with the cells loaded after A1, whose loads
+// the entries of x then wait for, 68, 235 and 177.)
 // dot_op != DOT_NONE: also the partial sums of x and y (dot_partials) into dot.
 template <typename R, int N, typename PL, int BS = 256>
 __global__ __launch_bounds__(BS) void k_pass5s(const typename CxT<R>::T* __restrict__ a1,
                                                 const typename CxT<R>::T* __restrict__ x,
                                                 typename CxT<R>::T* __restrict__ y,
                                                 const uint32_t* __restrict__ row_list, int n_list,
-                                                const uint32_t* __restrict__ row_start,
-                                                const uint32_t* __restrict__ row_dip,
-                                                const uint32_t* __restrict__ row_meta,
+                                                const uint32_t* __restrict__ cell, const uint8_t* __restrict__ mat,
                                                 const typename CxT<R>::T* __restrict__ ccs, MvDims d,
                                                 const typename CxT<R>::T* __restrict__ tw, int conj, RhsFlags fl,
                                                 double* __restrict__ dot, int dot_op) {
@@ -356,7 +362,7 @@ __global__ __launch_bounds__(BS) void k_pass5s(const typename CxT<R>::T* __restr
   x += (long long)rhs * 3 * d.S;
   y += (long long)rhs * 3 * d.S;
   ccs += rhs * 3 * d.nmat;
-  if (d.member) row_meta += (size_t)d.member[rhs] * d.nv;
+  if (d.member) mat += (size_t)d.member[rhs] * d.nv;
   extern __shared__ char smem[];
   C* tile = reinterpret_cast<C*>(smem);
   const int t = threadIdx.x % TPC, l = threadIdx.x / TPC;
@@ -365,41 +371,36 @@ __global__ __launch_bounds__(BS) void k_pass5s(const typename CxT<R>::T* __restr
   const int c = ok ? g / n_list : 0;
   const int row = ok ? (int)row_list[g - c * n_list] : 0;
   const C* src = a1 + ((size_t)c * d.nrows + row) * d.rs;
+  // the dipoles of this thread's outputs come first (their x entries wait for
+  // them alone, and are there when the transform ends)
+  const uint32_t* cells = cell + (size_t)row * d.Bx;
+  x += (size_t)c * d.S;
+  uint32_t at[NO];
+#pragma unroll
+  for (int e = 0; e < NO; e++) {
+    const int p = first_point<N, TPC, Out>(t, e);
+    at[e] = !upper_half<Out>(e) && ok && p < d.Bx && first_ok<N, TPC, Out>(t, e) ? cells[p] : kNoDipole;
+  }
   C v[PPT];
 #pragma unroll
   for (int e = 0; e < NF; e++)
     v[e] = ok && first_ok<N, TPC, F>(t, e) ? src[first_point<N, TPC, F>(t, e)] : czero<C>();
-  // the dipoles this thread gathers (a row holds at most N/2: the grid spans
-  // at least twice the box), their x entries and positions loaded before the
-  // transform so that those loads wait while it runs
-  constexpr int MAXD = (N / 2 + TPC - 1) / TPC;
-  const uint32_t s0 = ok ? row_start[row] : 0u, s1 = ok ? row_start[row + 1] : 0u;
-  uint32_t gi[MAXD], gm[MAXD];
-  C ga[MAXD];
+  __builtin_amdgcn_sched_barrier(0);
+  C ga[NO];
 #pragma unroll
-  for (int k = 0; k < MAXD; k++) {
-    const uint32_t q = s0 + t + k * TPC;
-    gi[k] = q < s1 ? (d.sorted ? q : row_dip[q]) : 0u;
-    gm[k] = q < s1 ? row_meta[q] : 0u;
-    ga[k] = q < s1 ? x[(size_t)c * d.S + gi[k]] : czero<C>();
-  }
+  for (int e = 0; e < NO; e++) ga[e] = !upper_half<Out>(e) && at[e] != kNoDipole ? x[at[e]] : czero<C>();
   RunStages<N, TPC, true, 1, C, F, false, P::template twiddles<R>>::run(v, t, tile, lp, l, tw);
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < NO; e++)
-    if (!upper_half<Out>(e) && first_ok<N, TPC, Out>(t, e)) tile[first_point<N, TPC, Out>(t, e) * lp + l] = v[e];
-  __syncthreads();
   double q0 = 0, q1 = 0, q2 = 0;
 #pragma unroll
-  for (int k = 0; k < MAXD; k++) {
-    if (s0 + t + k * TPC < s1) {
-      C a = ga[k];
+  for (int e = 0; e < NO; e++) {
+    if (!upper_half<Out>(e) && at[e] != kNoDipole) {
+      C a = ga[e];
       if (conj) a = cconj(a);
-      C r = cadd(cmul(ccs[3 * (gm[k] >> 16) + c], tile[(gm[k] & 0xffff) * lp + l]), a);
+      C r = cadd(cmul(ccs[3 * (d.nmat > 1 ? mat[at[e]] : 0) + c], v[e]), a);
       if (conj) r = cconj(r);
-      y[(size_t)c * d.S + gi[k]] = r;
+      y[(size_t)c * d.S + at[e]] = r;
       if (dot_op != DOT_NONE) {
-        const double xr = ga[k].x, xi = ga[k].y, yr = r.x, yi = r.y;
+        const double xr = ga[e].x, xi = ga[e].y, yr = r.x, yi = r.y;
         const bool du = dot_op == DOT_U;
         q0 += du ? xr * yr - xi * yi : yr * yr + yi * yi;
         q1 += du ? xr * yi + xi * yr : xr * yr + xi * yi;
@@ -653,8 +654,7 @@ dda_status launch_x_plan(dda_op_s* op, const MvView& v, bool inverse, const void
     auto k = k_pass1s<R, N, PL, BS>;
     DDA_TRY(set_lds(k, lds));
     hipLaunchKernelGGL(k, dim3((3 * d.nrows + LN - 1) / LN, nrhs), dim3(BS), lds, st, (const C*)x, (C*)v.a1,
-                       op->row_start, op->row_dip, op->row_meta, (const C*)v.ccs, d, (const C*)op->tw[0], conj,
-                       done);
+                       op->cell, op->mat_dev, (const C*)v.ccs, d, (const C*)op->tw[0], conj, done);
   } else {
     auto k = k_pass5s<R, N, PL, BS>;
     DDA_TRY(set_lds(k, lds));
@@ -663,8 +663,8 @@ dda_status launch_x_plan(dda_op_s* op, const MvView& v, bool inverse, const void
     op->p5_blocks = nbx;
     double* dot = dr.op != DOT_NONE ? dr.part + (size_t)dr.r0 * 4 * nbx : nullptr;
     hipLaunchKernelGGL(k, dim3(nbx, nrhs), dim3(BS), lds, st, (const C*)v.a1, (const C*)x, (C*)y, op->row_list,
-                       op->n_nonempty, op->row_start, op->row_dip, op->row_meta, (const C*)v.ccs, d,
-                       (const C*)op->tw[0], conj, done, dot, dr.op);
+                       op->n_nonempty, op->cell, op->mat_dev, (const C*)v.ccs, d, (const C*)op->tw[0], conj, done, dot,
+                       dr.op);
   }
   DDA_TRY_HIP(hipGetLastError());
   return DDA_OK;

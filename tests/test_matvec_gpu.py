@@ -303,3 +303,26 @@ def test_invalid_arguments(ctx):
     op = D.GpuMatVec(ctx, g.pos, g.mat, g.box, g.grid_unit, params.wave_num)
     with pytest.raises(D.DDAError):
         D.MatVecGpu(op).apply(np.zeros(params.vec_size, complex))  # couple constants not set
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_dipoles_that_share_a_cell(ctx, precision):
+    """A list that names a cell twice is accepted: with equal entries at both,
+    each gets the product of the list that names it once."""
+    g, params, cc, cs, prop, pol = cases.build("ellipsoid_5_4_3")
+    x = P.random_dipole_vector(params, seed=31).reshape(3, -1)[:, :params.nv]
+    once = D.MatVecGpu(_ops(ctx, g, params, cs, precision))
+    pos = np.concatenate([g.pos, g.pos[7:9]])
+    twice = D.GpuMatVec(ctx, pos, None, g.box, g.grid_unit, params.wave_num, precision=precision, grid=params.grid,
+                        nmat=1)
+    twice.set_couple_constants(cs)
+
+    def apply(mv, op, v):
+        full = np.zeros((3, op.vec_stride), complex)
+        full[:, :op.nv] = v
+        return np.asarray(mv.apply(full.reshape(-1))).reshape(3, -1)[:, :op.nv]
+
+    y1 = apply(once, once.op, x)
+    y2 = apply(D.MatVecGpu(twice), twice, np.concatenate([x, x[:, 7:9]], 1))
+    tol = FP64_TOL if precision == 64 else FP32_TOL
+    assert cases.rel_err(y2, np.concatenate([y1, y1[:, 7:9]], 1)) <= tol
