@@ -289,13 +289,13 @@ DDA_PLAN(1024, true, 16, 16, 16, 4)
 // A plan given by its points per thread and radix order directly (the Z
 // pass's long-column variants: 1024 = 32 x 32 holds 32 points per thread and
 // needs a single LDS exchange per transform).
-template <int N, int P, typename L> struct PlanOf {
+template <int N, int P, typename L, int TW = TW_CHAIN> struct PlanOf {
   static constexpr bool exists = true, general = false;
   static constexpr int PPT = P;
   static constexpr int TPC = N / P;
   typedef L Fwd;
   typedef L Bwd;
-  template <typename R> static constexpr int twiddles = TW_CHAIN;
+  template <typename R> static constexpr int twiddles = TW;
 };
 
 template <typename L> struct Reverse;

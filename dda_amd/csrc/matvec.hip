@@ -2071,7 +2071,7 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
     // the precision's default unless another variant is faster by more than
     // 2% (closer timings change places between runs)
     // (the X passes default to the narrow plan in both precisions)
-    const int def = pass == 1 && d.Gz == 1024 && sizeof(R) == 4 ? 2 : pass < 3 && sizeof(R) == 4 ? 1 : 0;
+    const int def = pass == 1 && d.Gz >= 512 && sizeof(R) == 4 ? 2 : pass < 3 && sizeof(R) == 4 ? 1 : 0;
     int fastest = 0;
     for (int w = 1; w < nvar; w++)
       if (t[w] < t[fastest]) fastest = w;
@@ -2083,10 +2083,10 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
     else
       best.col_wide[pass == 2] = pick;
     static const char* names[5] = {"Y forward", "Z + tensor", "Y inverse", "X forward", "X inverse"};
-    static const char* vn1024[4] = {"narrow", "wide", "32x32/16 cols", "32x32/8 cols"};
+    static const char* vn32[4] = {"narrow", "wide", "32 points/16 cols", "32 points/8 cols"};
     static const char* vntile[6] = {"narrow", "wide", "narrow other tile", "wide other tile", "narrow third tile",
                                     "wide third tile"};
-    const char* const* vnames = pass == 1 && d.Gz == 1024 ? vn1024 : vntile;
+    const char* const* vnames = pass == 1 && d.Gz >= 512 ? vn32 : vntile;
     std::snprintf(buf, sizeof buf, "%s%s: narrow %.1f us, wide %.1f us", report->empty() ? "" : "; ", names[pass],
                   t[0], t[1]);
     *report += buf;

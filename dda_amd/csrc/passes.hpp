@@ -605,13 +605,17 @@ dda_status launch_pass3_static_w(dda_op_s* op, const MvView& v, hipStream_t st, 
 }
 
 // Z-pass variants (Tune::p3_wide): -1 the precision's default, 0 narrow,
-// 1 wide; at 1024 points also 2 and 3, the 32 x 32 plan (32 points per
-// thread, one LDS exchange per transform, 2 waves per SIMD, FP32) over 16
-// columns (512 threads, 128-byte segments, one work-group per CU by LDS) or
-// 8 columns (256 threads, 64-byte segments, two work-groups per CU).
+// 1 wide; at 512 and 1024 points also 2 and 3, plans of 32 points per thread
+// (32 x 16 and 32 x 32: one LDS exchange per transform, 2 waves per SIMD, FP32)
+// over 16 columns (128-byte segments; at 1024 points 512 threads, one work-group
+// per CU by LDS, at 512 points 256 threads, two work-groups) or 8 columns.
 // FP32 only: in FP64 the 32-point plan's data alone needs 384 VGPRs. The FP32
-// default at 1024 points is 2: measured at 1024^3 (sphere 512 across) 14.8 ms
-// against 17.8 ms (wide), 19.2 ms (variant 3) and 33.0 ms (narrow).
+// default is 2 there: at 1024^3 (sphere 512 across) 14.8 ms against 17.8 ms
+// (wide), 19.2 ms (variant 3) and 33.0 ms (narrow); at 512^3 1,608 us against
+// 1,842, 2,385 and 2,051 (the wide plan's 512 threads of 168 VGPRs leave one
+// work-group per CU, and a third stage of radix 2 costs it an LDS exchange more).
+// At 512 points with TW_SPLIT, the products' error is 1.5e-7 where the wide
+// plan's chained powers made it 2.0e-7.
 // (Two further forms were measured and dropped. The wide plan without held
 // twiddle powers at 4 waves per SIMD, 128 VGPRs: 308.8 against 293.2 us per
 // 2-RHS FP32 launch at 256^3, and it spills at 32, 128 and 512 points. A
@@ -620,7 +624,9 @@ dda_status launch_pass3_static_w(dda_op_s* op, const MvView& v, hipStream_t st, 
 // 303.5 against 289.3 us (2-RHS FP32, 256^3), 315.0 against 291.4 us (FP64),
 // 15.1 against 14.6 ms (FP32, 1024^3); its loop costs 13% more VALU at 1024
 // points than the hidden loads save.)
-typedef PlanOf<1024, 32, RadixList<32, 32>> Plan1024x32;
+template <int N> struct Plan32;
+template <> struct Plan32<1024> : PlanOf<1024, 32, RadixList<32, 32>> {};
+template <> struct Plan32<512> : PlanOf<512, 32, RadixList<32, 16>, TW_SPLIT> {};
 // FP32 below 1024 points: 2 and 3 are the narrow and wide plans with the
 // other tile (other_cols_z).
 inline int p3_variants(int n, int prec) { return prec == 32 ? 4 : 2; }
@@ -629,9 +635,9 @@ template <typename R, int N>
 dda_status launch_pass3_static(dda_op_s* op, const MvView& v, hipStream_t st, RhsFlags done, int nrhs,
                                const dda_op_s::Tune& tn) {
   const int var = tn.p3_wide;
-  if constexpr (N == 1024 && sizeof(R) == 4) {
-    if (var == 2 || var < 0) return launch_pass3_plan<R, N, Plan1024x32, 16>(op, v, st, done, nrhs);
-    if (var == 3) return launch_pass3_plan<R, N, Plan1024x32, 8>(op, v, st, done, nrhs);
+  if constexpr (N >= 512 && sizeof(R) == 4) {
+    if (var == 2 || var < 0) return launch_pass3_plan<R, N, Plan32<N>, 16>(op, v, st, done, nrhs);
+    if (var == 3) return launch_pass3_plan<R, N, Plan32<N>, 8>(op, v, st, done, nrhs);
   } else if constexpr (sizeof(R) == 4) {
     if (var >= 2)
       return (var & 1) ? launch_pass3_static_w<R, N, true, true>(op, v, st, done, nrhs)
