@@ -533,6 +533,21 @@ dda_status launch_col_static_w(const void* in, void* out, const ColParams& cp, c
   return DDA_OK;
 }
 
+// The FP32 variant of an untuned Y pass over ncols columns of nbatch batches.
+// Tiles of 64 columns (512-byte row segments) where they divide the rows and
+// leave 24 work-groups per CU: there the pass streams through HBM, and a 96-point
+// launch for 128 right-hand sides takes 318 us forward and 298 inverse against
+// 357 and 323 (whole products 1.5 to 3.4% less at 64 to 96 points); with fewer
+// work-groups 16 columns are as fast or faster, at 192 and 256 points always (by
+// up to 7%). At 512 points the narrow plan, which has three stages like the wide
+// one and half its registers: 442 and 418 us against 476 and 435 at 512^3.
+template <int N>
+inline int default_col_variant(int ncols, int nbatch) {
+  if (N == 512) return 0;
+  if (N > 128 || ncols % 64 || (long long)(ncols / 64) * nbatch < 6144) return 1;
+  return N >= 48 ? 5 : 3;
+}
+
 // wide: -1 the precision's default plan, 0 narrow, 1 wide; FP32 also 2 and 3,
 // narrow and wide with the second tile (other_cols), and 4 and 5 with the
 // third (third_cols).
@@ -540,6 +555,7 @@ template <typename R, int N, bool INV>
 dda_status launch_col_static(const void* in, void* out, const ColParams& cp, const void* tw, int nbatch, hipStream_t st,
                              RhsFlags done, int wide) {
   if constexpr (sizeof(R) == 4) {
+    if (wide < 0) wide = default_col_variant<N>(cp.ncols, nbatch);
     if (wide >= 4)
       return (wide & 1) ? launch_col_static_w<R, N, true, INV, 2>(in, out, cp, tw, nbatch, st, done)
                         : launch_col_static_w<R, N, false, INV, 2>(in, out, cp, tw, nbatch, st, done);
