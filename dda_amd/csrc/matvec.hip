@@ -2240,26 +2240,27 @@ extern "C" dda_status dda_op_profile_read(dda_op_t op, double ms[5], uint64_t co
   }
   // Launches of a device-side solve after some or all of its right-hand sides
   // have finished do less work or none (kernels return at entry for finished
-  // ones): launches shorter than 60% of their pass's median are counted in
-  // `skipped`, not in the times, so that ms / counts is the full launch.
+  // ones): the five launches of a matvec that takes less than 60% of the median
+  // matvec are counted in `skipped`, not in the times, so that ms / counts is the
+  // full launch. (A single short pass may take most of its time doing nothing.)
   uint64_t sk = 0;
-  std::vector<float> t(op->prof_recs.size());
-  std::vector<float> by_pass[5];
+  const size_t nmv = op->prof_recs.size() / 5;  // launch_passes records the five in order
+  std::vector<float> t(op->prof_recs.size()), total(nmv, 0.f);
   for (size_t i = 0; i < op->prof_recs.size(); i++) {
     auto& r = op->prof_recs[i];
     DDA_TRY_HIP(hipEventSynchronize(r.e));
     DDA_TRY_HIP(hipEventElapsedTime(&t[i], r.b, r.e));
-    by_pass[r.pass].push_back(t[i]);
+    if (i / 5 < nmv) total[i / 5] += t[i];
   }
-  float med[5] = {0, 0, 0, 0, 0};
-  for (int p = 0; p < 5; p++)
-    if (!by_pass[p].empty()) {
-      std::nth_element(by_pass[p].begin(), by_pass[p].begin() + by_pass[p].size() / 2, by_pass[p].end());
-      med[p] = by_pass[p][by_pass[p].size() / 2];
-    }
+  float med = 0;
+  if (nmv) {
+    std::vector<float> v(total);
+    std::nth_element(v.begin(), v.begin() + nmv / 2, v.end());
+    med = v[nmv / 2];
+  }
   for (size_t i = 0; i < op->prof_recs.size(); i++) {
     auto& r = op->prof_recs[i];
-    if (t[i] < 0.6f * med[r.pass] || t[i] < 0.002f) {
+    if (i / 5 >= nmv || total[i / 5] < 0.6f * med || total[i / 5] < 0.01f) {
       sk++;
     } else {
       ms[r.pass] += t[i];
