@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -43,7 +44,6 @@ struct MvDims {
   int S;       // vector stride
   int nrows;   // By * Bz
   int nmat;
-  int sorted;  // dipoles already in row order (row_dip is the identity)
   // Packs of several particles on one grid (nullptr otherwise): member[rhs]
   // selects the material map (row_meta / mat at member * nv) and the tensor
   // dhat_tab[member] of each right-hand side.
@@ -64,8 +64,12 @@ struct RhsFlags {
 // has a prime factor above 7.
 bool make_plan(int n, FftPlan* p);
 
-// Device twiddle table exp(-2 pi i t / n), t < n, computed in long double.
-dda_status make_twiddles(int n, int prec, void** out, hipStream_t st);
+// Device twiddle tables exp(-2 pi i t / n), t < n, of the three axes, computed in
+// long double: one allocation, at out[0].
+dda_status make_twiddles(const int n[3], int prec, void* out[3], hipStream_t st);
+
+// Fills op->pos where it is not there yet.
+dda_status host_positions(struct ::dda_op_s* op);
 
 // The FP32 twin of an FP64 operator: same geometry, tensor converted from the
 // FP64 one (or taken from the same cache).
@@ -111,6 +115,14 @@ struct dda_ctx_s {
   int device = 0;
   hipStream_t stream = nullptr;
   hipDeviceProp_t prop;
+  // Grid buffers and tensors of destroyed operators, oldest first, for the
+  // context's next ones (ctx_alloc, ctx_free).
+  struct Spare {
+    void* ptr;
+    size_t bytes;
+  };
+  std::mutex spare_mu;
+  std::vector<Spare> spare;
 };
 
 namespace dda {
@@ -127,6 +139,13 @@ inline dda_status bind_device(const dda_ctx_s* c) {
   }
   return DDA_OK;
 }
+
+// Large device buffers of a context's operators: a spare one of the size, else
+// hipMalloc (after giving the spare ones back where memory is short). *got is the
+// buffer's size, which ctx_free takes. ctx_free's caller has waited for all work
+// on the buffer but that on the context's stream.
+hipError_t ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, size_t* got);
+void ctx_free(dda_ctx_s* c, void* p, size_t bytes);
 }  // namespace dda
 
 struct dda_op_s {
@@ -136,11 +155,12 @@ struct dda_op_s {
   uint32_t nmat = 0;
   double grid_unit = 0, wave_num = 0;
   bool cc_set = false;
-  std::vector<uint32_t> pos;  // host copy [nv][3]
+  std::vector<uint32_t> pos;  // host copy [nv][3], see host_positions
   std::vector<uint8_t> mat;   // host copy [nv]
   std::vector<double> cc_sqrt_host;  // [nmat][3] complex, reference units
 
   // device
+  // (row_start, row_dip and row_meta: run-time planned X passes only)
   uint32_t* row_start = nullptr;  // [nrows + 1]
   uint32_t* row_dip = nullptr;    // [nv] dipole index, grouped by row
   uint32_t* row_meta = nullptr;   // [nv] x | mat << 16
@@ -152,6 +172,8 @@ struct dda_op_s {
   void* dhat = nullptr;           // octant [6][Gz/2+1][Gy/2+1][Gx/2+1] complex R, d^3 scaled
   void* a1 = nullptr;             // [3][Bz][By][Gx]
   void* a2 = nullptr;             // [3][Bz][Gy][Gx]
+  size_t a1_bytes = 0, a2_bytes = 0, dhat_bytes = 0;  // as ctx_alloc gave them
+  bool foreign = false;           // products were launched on streams other than the context's
   void* tw[3] = {nullptr, nullptr, nullptr};
   dda::FftPlan plan[3];
   void* stage_x = nullptr;        // host-apply staging vectors
@@ -196,7 +218,7 @@ struct dda_op_s {
     int* member_dev = nullptr;                 // [cap_rhs] member of each right-hand side
     std::vector<int> member_host;
   } pack;
-  void* pos_dev = nullptr;      // [nv][3] positions, uploaded on first use by the observables
+  void* pos_dev = nullptr;      // [nv][3] positions (run-time planned X passes: uploaded on first use by the observables)
   // the positions as the far field of many directions takes them (observe.hip)
   struct Far {
     bool made = false;

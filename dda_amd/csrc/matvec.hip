@@ -436,20 +436,29 @@ static hipError_t copy_sync(void* dst, const void* src, size_t bytes, hipMemcpyK
   return e == hipSuccess ? hipStreamSynchronize(st) : e;
 }
 
-dda_status make_twiddles(int n, int prec, void** out, hipStream_t st) {
+dda_status make_twiddles(const int n[3], int prec, void* out[3], hipStream_t st) {
   const long double pi = 3.1415926535897932384626433832795028L;
-  size_t esz = prec == 64 ? sizeof(double2) : sizeof(float2);
-  std::vector<char> h(esz * n);
-  for (int t = 0; t < n; t++) {
-    long double a = -2 * pi * (long double)t / (long double)n;
-    double c = (double)cosl(a), s = (double)sinl(a);
-    if (prec == 64)
-      reinterpret_cast<double2*>(h.data())[t] = make_double2(c, s);
-    else
-      reinterpret_cast<float2*>(h.data())[t] = make_float2((float)c, (float)s);
+  const size_t esz = prec == 64 ? sizeof(double2) : sizeof(float2);
+  size_t off[4] = {0, 0, 0, 0};
+  for (int a = 0; a < 3; a++) off[a + 1] = (off[a] + n[a] * esz + 127) / 128 * 128;
+  std::vector<char> h(off[3]);
+  for (int a = 0; a < 3; a++) {
+    auto set = [&](int t, double c, double s) {
+      if (prec == 64)
+        reinterpret_cast<double2*>(h.data() + off[a])[t] = make_double2(c, s);
+      else
+        reinterpret_cast<float2*>(h.data() + off[a])[t] = make_float2((float)c, (float)s);
+    };
+    for (int t = 0; 2 * t <= n[a]; t++) {  // root n - t is the conjugate of root t
+      long double s, c;
+      sincosl(-2 * pi * (long double)t / (long double)n[a], &s, &c);
+      set(t, (double)c, (double)s);
+      if (t) set(n[a] - t, (double)c, t * 2 == n[a] ? (double)s : -(double)s);
+    }
   }
-  DDA_TRY_HIP(hipMalloc(out, h.size()));
-  DDA_TRY_HIP(copy_sync(*out, h.data(), h.size(), hipMemcpyHostToDevice, st));
+  DDA_TRY_HIP(hipMalloc(&out[0], h.size()));
+  for (int a = 1; a < 3; a++) out[a] = (char*)out[0] + off[a];
+  DDA_TRY_HIP(copy_sync(out[0], h.data(), h.size(), hipMemcpyHostToDevice, st));
   return DDA_OK;
 }
 
@@ -914,12 +923,10 @@ static dda_status generate_dhat(dda_op_s* op, int cx, int cy, int cz, void* dst)
   if (own) DDA_TRY_HIP(hipMalloc(&w, (oct ? 6 * cz * plane : total) * sizeof(double2)));
   void* tw64[3] = {nullptr, nullptr, nullptr};
   dda_status rc = DDA_OK;
-  for (int a = 0; a < 3 && rc == DDA_OK; a++) {
-    if (op->prec == 64)
-      tw64[a] = op->tw[a];
-    else
-      rc = make_twiddles(g[a], 64, &tw64[a], st);
-  }
+  if (op->prec == 64)
+    for (int a = 0; a < 3; a++) tw64[a] = op->tw[a];
+  else
+    rc = make_twiddles(g, 64, tw64, st);
   const double kd = op->wave_num * op->grid_unit;
   const double scale = -1.0 / (double)total;
   if (rc == DDA_OK && oct) {
@@ -961,8 +968,7 @@ static dda_status generate_dhat(dda_op_s* op, int cx, int cy, int cz, void* dst)
     }
   }
   hipError_t e = hipStreamSynchronize(st);
-  for (int a = 0; a < 3; a++)
-    if (tw64[a] && tw64[a] != op->tw[a]) (void)hipFree(tw64[a]);
+  if (tw64[0] && tw64[0] != op->tw[0]) (void)hipFree(tw64[0]);
   if (own) (void)hipFree(w);
   if (rc != DDA_OK) return rc;
   DDA_TRY_HIP(e);
@@ -1211,6 +1217,27 @@ extern "C" uint32_t dda_fft_fit(uint32_t x, uint32_t override_, int support_non_
   }
 }
 
+static const char kBadDipole[] = "dda_op_create: dipole position outside the box or material index >= nmat";
+
+// The host's copy of the positions, made when something on the host needs it.
+dda_status dda::host_positions(dda_op_s* op) {
+  if (!op->pos.empty()) return DDA_OK;
+  op->pos.resize(3 * (size_t)op->dims.nv);
+  const hipError_t e = copy_sync(op->pos.data(), op->pos_dev, op->pos.size() * 4, hipMemcpyDeviceToHost, op->ctx->stream);
+  if (e != hipSuccess) op->pos.clear();
+  DDA_TRY_HIP(e);
+  return DDA_OK;
+}
+
+// Buffers that other streams may still use are freed, which waits for them.
+static void release_large(dda_op_s* op, void* p, size_t bytes) {
+  if (!p) return;
+  if (op->foreign)
+    (void)hipFree(p);
+  else
+    ctx_free(op->ctx, p, bytes);
+}
+
 static void free_op(dda_op_s* op) {
   if (op->split_stream) {
     (void)hipStreamSynchronize(op->split_stream);
@@ -1239,18 +1266,173 @@ static void free_op(dda_op_s* op) {
   }
   if (op->pack.dhat_tab) (void)hipFree(op->pack.dhat_tab);
   if (op->pack.member_dev) (void)hipFree(op->pack.member_dev);
-  void* bufs[] = {op->cell, op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->dhat, op->a1,
-                  op->a2, op->tw[0], op->tw[1], op->tw[2], op->stage_x, op->stage_y, op->pos_dev, op->far_dev,
+  void* bufs[] = {op->cell, op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->tw[0], op->stage_x, op->stage_y, op->pos_dev, op->far_dev,
                   op->obs_scratch};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
+  release_large(op, op->a1, op->a1_bytes);
+  release_large(op, op->a2, op->a2_bytes);
+  release_large(op, op->dhat, op->dhat_bytes);
   delete op;
 }
 
 void apply_cached_tuning(dda_op_s* op);
 
+// The index arrays of the compile-time planned X passes, formed on the device
+// from the positions: the cell map and the list of occupied rows. flags: bit 0 a
+// position outside the box, bit 1 two dipoles in one cell; then the rows' count.
+__global__ void k_cells_clear(uint32_t* cell, long long ncell, uint32_t* occupied, int nrows, int* flags) {
+  const long long i0 = blockIdx.x * (long long)blockDim.x + threadIdx.x, step = (long long)gridDim.x * blockDim.x;
+  for (long long i = i0; i < ncell; i += step) cell[i] = kNoDipole;
+  for (long long i = i0; i < nrows; i += step) occupied[i] = 0;
+  if (i0 < 2) flags[i0] = 0;
+}
+__global__ void k_cells(const uint32_t* __restrict__ pos, int nv, uint32_t Bx, uint32_t By, uint32_t Bz, uint32_t* cell,
+                        uint32_t* occupied, int* flags) {
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < nv; i += (long long)gridDim.x * blockDim.x) {
+    const uint32_t x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
+    if (x >= Bx || y >= By || z >= Bz) {
+      atomicOr(flags, 1);
+      continue;
+    }
+    const uint32_t row = z * By + y;
+    if (atomicExch(&cell[(size_t)row * Bx + x], (uint32_t)i) != kNoDipole) atomicOr(flags, 2);
+    occupied[row] = 1;
+  }
+}
+// One work-group: the occupied rows in order.
+__global__ __launch_bounds__(1024) void k_row_list(const uint32_t* __restrict__ occupied, int nrows,
+                                                   uint32_t* __restrict__ row_list, int* flags) {
+  __shared__ int sums[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int base = 0;
+  for (int r0 = 0; r0 < nrows; r0 += 1024) {
+    const int r = r0 + threadIdx.x;
+    const bool occ = r < nrows && occupied[r];
+    const unsigned long long m = __ballot(occ);
+    if (lane == 0) sums[wave] = __popcll(m);
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int w = 0; w < 16; w++) {
+      before += w < wave ? sums[w] : 0;
+      all += sums[w];
+    }
+    if (occ) row_list[base + before + __popcll(m & ((1ull << lane) - 1))] = r;
+    base += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) flags[1] = base;
+}
+
+// The rows of the (z, y) plane for the run-time planned X passes: counting sort
+// of the dipoles by row, stable, on the host.
+static dda_status build_rows(dda_op_s* op) {
+  MvDims& d = op->dims;
+  DDA_TRY(host_positions(op));
+  std::vector<uint32_t> row_start(d.nrows + 1, 0), row_dip(d.nv), row_meta(d.nv), row_list;
+  for (int i = 0; i < d.nv; i++) {
+    const uint32_t* p = &op->pos[3 * (size_t)i];
+    if ((int)p[0] >= d.Bx || (int)p[1] >= d.By || (int)p[2] >= d.Bz) {
+      set_error(kBadDipole);
+      return DDA_INVALID_ARG;
+    }
+    row_start[p[2] * d.By + p[1] + 1]++;
+  }
+  for (int r = 0; r < d.nrows; r++) {
+    if (row_start[r + 1]) row_list.push_back(r);
+    row_start[r + 1] += row_start[r];
+  }
+  std::vector<uint32_t> fill(row_start.begin(), row_start.end() - 1);
+  for (int i = 0; i < d.nv; i++) {
+    const uint32_t* p = &op->pos[3 * (size_t)i];
+    const uint32_t k = fill[p[2] * d.By + p[1]]++;
+    row_dip[k] = i;
+    row_meta[k] = p[0] | ((uint32_t)op->mat[i] << 16);
+  }
+  op->n_nonempty = (int)row_list.size();
+  hipStream_t st = op->ctx->stream;
+  auto upload = [&](uint32_t*& p, const std::vector<uint32_t>& v) -> dda_status {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    DDA_TRY_HIP(hipMalloc(&p, std::max<size_t>(1, v.size()) * 4));
+    op->device_bytes += v.size() * 4;
+    if (!v.empty()) DDA_TRY_HIP(copy_sync(p, v.data(), v.size() * 4, hipMemcpyHostToDevice, st));
+    return DDA_OK;
+  };
+  DDA_TRY(upload(op->row_start, row_start));
+  DDA_TRY(upload(op->row_dip, row_dip));
+  DDA_TRY(upload(op->row_meta, row_meta));
+  return upload(op->row_list, row_list);
+}
+
+// Positions, materials and index arrays of an operator whose other buffers are
+// there (A1 holds what is needed in between); from `like` (an operator on the
+// same dipoles) they are copied.
+static dda_status build_index(dda_op_s* op, const uint32_t* pos, const dda_op_s* like) {
+  MvDims& d = op->dims;
+  hipStream_t st = op->ctx->stream;
+  const size_t pb = 12ull * d.nv, ncell = (size_t)d.nrows * d.Bx;
+  auto dmalloc = [&](void* p, size_t bytes) -> dda_status {
+    DDA_TRY_HIP(hipMalloc((void**)p, bytes));
+    op->device_bytes += bytes;
+    return DDA_OK;
+  };
+  DDA_TRY(dmalloc(&op->mat_dev, d.nv));
+  if (!op->static_x) {
+    DDA_TRY_HIP(copy_sync(op->mat_dev, op->mat.data(), d.nv, hipMemcpyHostToDevice, st));
+    if (pos) {
+      op->pos.assign(pos, pos + 3 * (size_t)d.nv);
+    } else {
+      op->pos.resize(3 * (size_t)d.nv);
+      DDA_TRY_HIP(copy_sync(op->pos.data(), like->pos_dev, pb, hipMemcpyDeviceToHost, st));
+    }
+    return build_rows(op);
+  }
+  DDA_TRY(dmalloc(&op->pos_dev, pb));
+  DDA_TRY(dmalloc(&op->cell, ncell * 4));
+  DDA_TRY(dmalloc(&op->row_list, std::max(1, d.nrows) * 4ull));
+  if (like) {
+    op->n_nonempty = like->n_nonempty;
+    DDA_TRY_HIP(hipMemcpyAsync(op->pos_dev, like->pos_dev, pb, hipMemcpyDeviceToDevice, st));
+    DDA_TRY_HIP(hipMemcpyAsync(op->mat_dev, like->mat_dev, d.nv, hipMemcpyDeviceToDevice, st));
+    DDA_TRY_HIP(hipMemcpyAsync(op->cell, like->cell, ncell * 4, hipMemcpyDeviceToDevice, st));
+    DDA_TRY_HIP(hipMemcpyAsync(op->row_list, like->row_list, d.nrows * 4ull, hipMemcpyDeviceToDevice, st));
+    DDA_TRY_HIP(hipStreamSynchronize(st));
+    return DDA_OK;
+  }
+  DDA_TRY_HIP(hipMemcpyAsync(op->pos_dev, pos, pb, hipMemcpyHostToDevice, st));
+  if (op->nmat > 1)
+    DDA_TRY_HIP(hipMemcpyAsync(op->mat_dev, op->mat.data(), d.nv, hipMemcpyHostToDevice, st));
+  else
+    DDA_TRY_HIP(hipMemsetAsync(op->mat_dev, 0, d.nv, st));
+  int* flags = (int*)op->a1;
+  uint32_t* occupied = (uint32_t*)op->a1 + 64;
+  const int blocks = (int)std::min<size_t>(2048, (std::max<size_t>(ncell, d.nv) + 255) / 256);
+  hipLaunchKernelGGL(k_cells_clear, dim3(blocks), dim3(256), 0, st, op->cell, (long long)ncell, occupied, d.nrows, flags);
+  hipLaunchKernelGGL(k_cells, dim3(blocks), dim3(256), 0, st, (const uint32_t*)op->pos_dev, d.nv, d.Bx, d.By, d.Bz,
+                     op->cell, occupied, flags);
+  hipLaunchKernelGGL(k_row_list, dim3(1), dim3(1024), 0, st, occupied, d.nrows, op->row_list, flags);
+  DDA_TRY_HIP(hipGetLastError());
+  int h[2] = {0, 0};
+  DDA_TRY_HIP(copy_sync(h, flags, sizeof h, hipMemcpyDeviceToHost, st));
+  if (h[0] & 1) {
+    set_error(kBadDipole);
+    return DDA_INVALID_ARG;
+  }
+  op->n_nonempty = h[1];
+  if (h[0] & 2) {  // dipoles that share a cell go by the rows' lists
+    op->static_x = false;
+    op->gen[0] = nullptr;
+    (void)hipFree(op->cell);
+    op->cell = nullptr;
+    return build_rows(op);
+  }
+  return DDA_OK;
+}
+
 // The tensor comes from desc->dmatrix, else from `cache`, else from the FP64
 // operator `narrow_from` of the same shape (converted), else it is generated.
+// With narrow_from, positions may be null: they are its.
 static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precision, dda_dhat_cache_s* cache,
                             const dda_op_s* narrow_from, dda_op_t* out) {
   if (!ctx || !desc || !out || (precision != 32 && precision != 64)) {
@@ -1260,7 +1442,8 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
   DDA_TRY(bind_device(ctx));
   *out = nullptr;
   const dda_op_desc& ds = *desc;
-  if (ds.nv == 0 || !ds.pos || ds.nmat == 0 || ds.nmat > 256 || !(ds.grid_unit > 0) || !(ds.wave_num > 0)) {
+  const dda_op_s* like = narrow_from && narrow_from->cell ? narrow_from : nullptr;
+  if (ds.nv == 0 || (!ds.pos && !like) || ds.nmat == 0 || ds.nmat > 256 || !(ds.grid_unit > 0) || !(ds.wave_num > 0)) {
     set_error("dda_op_create: need nv > 0, positions, 1..256 materials, grid_unit > 0, wave_num > 0");
     return DDA_INVALID_ARG;
   }
@@ -1303,58 +1486,23 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
       free_op(op);
       return DDA_NOT_SUPPORTED;
     }
-  op->pos.assign(ds.pos, ds.pos + 3 * (size_t)ds.nv);
-  op->mat.assign(ds.nv, 0);
-  if (ds.mat) op->mat.assign(ds.mat, ds.mat + ds.nv);
-
-  // Rows of the (z, y) plane: counting sort of the dipoles by row, stable.
-  std::vector<uint32_t> row_start(d.nrows + 1, 0), row_dip(ds.nv), row_meta(ds.nv), row_list;
-  for (uint32_t i = 0; i < ds.nv; i++) {
-    const uint32_t* p = &op->pos[3 * i];
-    if ((int)p[0] >= d.Bx || (int)p[1] >= d.By || (int)p[2] >= d.Bz || op->mat[i] >= ds.nmat) {
-      set_error("dda_op_create: dipole position outside the box or material index >= nmat");
-      free_op(op);
-      return DDA_INVALID_ARG;
-    }
-    row_start[p[2] * d.By + p[1] + 1]++;
+  if (ds.mat)
+    op->mat.assign(ds.mat, ds.mat + ds.nv);
+  else
+    op->mat.assign(ds.nv, 0);
+  uint8_t top = 0;  // (a loop that the compiler turns into vector instructions)
+  for (uint8_t m : op->mat) top = m > top ? m : top;
+  if (top >= ds.nmat) {
+    set_error(kBadDipole);
+    free_op(op);
+    return DDA_INVALID_ARG;
   }
-  for (int r = 0; r < d.nrows; r++) {
-    if (row_start[r + 1]) row_list.push_back(r);
-    row_start[r + 1] += row_start[r];
-  }
-  {
-    std::vector<uint32_t> fill(row_start.begin(), row_start.end() - 1);
-    for (uint32_t i = 0; i < ds.nv; i++) {
-      const uint32_t* p = &op->pos[3 * i];
-      const uint32_t r = p[2] * d.By + p[1];
-      const uint32_t k = fill[r]++;
-      row_dip[k] = i;
-      row_meta[k] = p[0] | ((uint32_t)op->mat[i] << 16);
-    }
-  }
-  op->n_nonempty = (int)row_list.size();
-  d.sorted = 1;  // the reference's (z, y, x) dipole order makes the row index the identity
-  for (uint32_t k = 0; k < ds.nv && d.sorted; k++) d.sorted = row_dip[k] == k;
   const size_t csz = precision == 64 ? sizeof(double2) : sizeof(float2);
   if (!std::getenv("DDA_GENERIC_FFT")) {
     for (int a = 0; a < 3; a++) op->gen[a] = axis_ops(grid[a], precision);
     if (!z_offsets_fit(d.Gx, d.Gy, d.Gz, csz)) op->gen[2] = nullptr;
     op->static_z = op->gen[2] || static_z_fits(d.Gx, d.Gy, d.Gz, csz);
     op->static_x = op->gen[0] || has_static_plan(d.Gx);
-  }
-  // the cell map; dipoles that share a cell go by the rows' lists
-  std::vector<uint32_t> cell;
-  if (op->static_x) {
-    cell.assign((size_t)d.nrows * d.Bx, kNoDipole);
-    for (uint32_t i = 0; i < ds.nv && op->static_x; i++) {
-      const uint32_t* p = &op->pos[3 * (size_t)i];
-      uint32_t& at = cell[((size_t)p[2] * d.By + p[1]) * d.Bx + p[0]];
-      if (at != kNoDipole) {
-        op->static_x = false;
-        op->gen[0] = nullptr;
-      }
-      at = i;
-    }
   }
   op->split_rhs = std::getenv("DDA_SPLIT") && std::atoi(std::getenv("DDA_SPLIT")) != 0;
 
@@ -1378,40 +1526,40 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
     op->device_bytes += bytes;
     return DDA_OK;
   };
+  auto large = [&](void** p, size_t bytes, size_t* got) -> dda_status {
+    const hipError_t e = ctx_alloc(ctx, p, bytes, got);
+    if (e != hipSuccess) {
+      set_error(std::string("dda_op_create: hipMalloc failed: ") + hipGetErrorString(e));
+      return e == hipErrorOutOfMemory ? DDA_OUT_OF_MEMORY : DDA_HIP_ERROR;
+    }
+    op->device_bytes += bytes;
+    return DDA_OK;
+  };
   const size_t a1n = 3ull * d.Bz * d.By * d.rs;
   const size_t a2n = 3ull * d.Bz * d.p2;
   const size_t dn = 6ull * (d.Gx / 2 + 1) * (d.Gy / 2 + 1) * (d.Gz / 2 + 1);
   dda_status rc = DDA_OK;
-  if (rc == DDA_OK) rc = dmalloc((void**)&op->row_start, row_start.size() * 4);
-  if (rc == DDA_OK) rc = dmalloc((void**)&op->row_dip, ds.nv * 4ull);
-  if (rc == DDA_OK) rc = dmalloc((void**)&op->row_meta, ds.nv * 4ull);
-  if (rc == DDA_OK) rc = dmalloc((void**)&op->row_list, std::max<size_t>(1, row_list.size()) * 4);
-  if (rc == DDA_OK) rc = dmalloc((void**)&op->mat_dev, ds.nv);
-  if (rc == DDA_OK && op->static_x) rc = dmalloc((void**)&op->cell, cell.size() * 4);
   if (rc == DDA_OK) rc = dmalloc(&op->ccs, 3ull * ds.nmat * csz);
-  if (rc == DDA_OK && (ds.dmatrix || !cache)) rc = dmalloc(&op->dhat, dn * csz);
-  if (rc == DDA_OK) rc = dmalloc(&op->a1, a1n * csz);
-  if (rc == DDA_OK) rc = dmalloc(&op->a2, a2n * csz);
-  for (int a = 0; a < 3 && rc == DDA_OK; a++) rc = make_twiddles(grid[a], precision, &op->tw[a], ctx->stream);
+  if (rc == DDA_OK && (ds.dmatrix || !cache)) rc = large(&op->dhat, dn * csz, &op->dhat_bytes);
+  if (rc == DDA_OK) rc = large(&op->a1, a1n * csz, &op->a1_bytes);
+  if (rc == DDA_OK) rc = large(&op->a2, a2n * csz, &op->a2_bytes);
+  if (rc == DDA_OK) {
+    const int n[3] = {d.Gx, d.Gy, d.Gz};
+    rc = make_twiddles(n, precision, op->tw, ctx->stream);
+  }
+  if (rc == DDA_OK) rc = build_index(op, ds.pos, like);
+  hipError_t e = hipSuccess;
+  if (rc == DDA_OK) {
+    e = hipMemsetAsync(op->ccs, 0, 3ull * ds.nmat * csz, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess) {
+      set_error(std::string("dda_op_create: ") + hipGetErrorString(e));
+      rc = DDA_HIP_ERROR;
+    }
+  }
   if (rc != DDA_OK) {
     free_op(op);
     return rc;
-  }
-  hipError_t e = hipSuccess;
-  hipStream_t cst = ctx->stream;
-  if (e == hipSuccess) e = copy_sync(op->row_start, row_start.data(), row_start.size() * 4, hipMemcpyHostToDevice, cst);
-  if (e == hipSuccess) e = copy_sync(op->row_dip, row_dip.data(), ds.nv * 4ull, hipMemcpyHostToDevice, cst);
-  if (e == hipSuccess) e = copy_sync(op->row_meta, row_meta.data(), ds.nv * 4ull, hipMemcpyHostToDevice, cst);
-  if (e == hipSuccess && op->static_x) e = copy_sync(op->cell, cell.data(), cell.size() * 4, hipMemcpyHostToDevice, cst);
-  if (e == hipSuccess && !row_list.empty())
-    e = copy_sync(op->row_list, row_list.data(), row_list.size() * 4, hipMemcpyHostToDevice, cst);
-  if (e == hipSuccess) e = copy_sync(op->mat_dev, op->mat.data(), ds.nv, hipMemcpyHostToDevice, cst);
-  if (e == hipSuccess) e = hipMemsetAsync(op->ccs, 0, 3ull * ds.nmat * csz, cst);
-  if (e == hipSuccess) e = hipStreamSynchronize(cst);
-  if (e != hipSuccess) {
-    set_error(std::string("dda_op_create: upload failed: ") + hipGetErrorString(e));
-    free_op(op);
-    return DDA_HIP_ERROR;
   }
 
   if (ds.dmatrix) {
@@ -1537,25 +1685,26 @@ static dda_status pack_extend(dda_op_s* op, const std::vector<uint8_t>& mats, co
     op->wave_num = w0;
     DDA_TRY(rc);
   }
-  // materials and row metadata of every member ([nm][nv]); the union is in
-  // (z, y, x) order, so row k holds dipole k
-  std::vector<uint32_t> meta((size_t)nm * d.nv);
-  for (int m = 0; m < nm; m++)
-    for (int k = 0; k < d.nv; k++)
-      meta[(size_t)m * d.nv + k] = op->pos[3 * (size_t)k] | ((uint32_t)mats[(size_t)m * d.nv + k] << 16);
-  uint32_t* row_meta = nullptr;
+  // materials of every member ([nm][nv]) and, for the run-time planned X passes,
+  // row metadata; the union is in (z, y, x) order, so row k holds dipole k
   uint8_t* mat_dev = nullptr;
-  DDA_TRY_HIP(hipMalloc(&row_meta, meta.size() * 4));
-  hipError_t e = hipMalloc(&mat_dev, mats.size());
-  if (e != hipSuccess) (void)hipFree(row_meta);
-  DDA_TRY_HIP(e);
-  (void)hipFree(op->row_meta);
+  DDA_TRY_HIP(hipMalloc(&mat_dev, mats.size()));
   (void)hipFree(op->mat_dev);
-  op->row_meta = row_meta;
   op->mat_dev = mat_dev;
-  op->device_bytes += (size_t)(nm - 1) * d.nv * 5;
-  DDA_TRY_HIP(copy_sync(row_meta, meta.data(), meta.size() * 4, hipMemcpyHostToDevice, st));
+  op->device_bytes += (size_t)(nm - 1) * d.nv;
   DDA_TRY_HIP(copy_sync(mat_dev, mats.data(), mats.size(), hipMemcpyHostToDevice, st));
+  if (op->row_meta) {
+    std::vector<uint32_t> meta((size_t)nm * d.nv);
+    for (int m = 0; m < nm; m++)
+      for (int k = 0; k < d.nv; k++)
+        meta[(size_t)m * d.nv + k] = op->pos[3 * (size_t)k] | ((uint32_t)mats[(size_t)m * d.nv + k] << 16);
+    uint32_t* row_meta = nullptr;
+    DDA_TRY_HIP(hipMalloc(&row_meta, meta.size() * 4));
+    (void)hipFree(op->row_meta);
+    op->row_meta = row_meta;
+    op->device_bytes += (size_t)(nm - 1) * d.nv * 4;
+    DDA_TRY_HIP(copy_sync(row_meta, meta.data(), meta.size() * 4, hipMemcpyHostToDevice, st));
+  }
   DDA_TRY_HIP(hipMalloc(&op->pack.dhat_tab, nm * sizeof(void*)));
   DDA_TRY_HIP(copy_sync(op->pack.dhat_tab, op->pack.dhat.data(), nm * sizeof(void*), hipMemcpyHostToDevice, st));
   op->pack.member_host.assign(op->cap_rhs, 0);
@@ -1716,7 +1865,7 @@ dda_status dda::create_twin32(const dda_op_s* op, dda_op_t* out) {
   desc.grid[2] = d.Gz;
   desc.nv = d.nv;
   desc.vec_stride = d.S;
-  desc.pos = op->pos.data();
+  desc.pos = op->pos.empty() ? nullptr : op->pos.data();
   desc.mat = op->mat.data();
   desc.nmat = op->nmat;
   desc.grid_unit = op->grid_unit;
@@ -1763,24 +1912,27 @@ static dda_status ensure_rhs_capacity(dda_op_s* op, int nrhs) {
   const size_t csz = op->prec == 64 ? sizeof(double2) : sizeof(float2);
   const size_t a1n = 3ull * d.Bz * d.By * d.rs, a2n = 3ull * d.Bz * d.p2;
   void *a1 = nullptr, *a2 = nullptr, *ccs = nullptr;
-  hipError_t e = hipMalloc(&a1, a1n * csz * nrhs);
-  if (e == hipSuccess) e = hipMalloc(&a2, a2n * csz * nrhs);
+  size_t b1 = 0, b2 = 0;
+  hipError_t e = ctx_alloc(op->ctx, &a1, a1n * csz * nrhs, &b1);
+  if (e == hipSuccess) e = ctx_alloc(op->ctx, &a2, a2n * csz * nrhs, &b2);
   if (e == hipSuccess) e = hipMalloc(&ccs, 3ull * d.nmat * csz * nrhs);
   if (e == hipSuccess)
     e = copy_sync(ccs, op->ccs, 3ull * d.nmat * csz * op->cap_rhs, hipMemcpyDeviceToDevice, op->ctx->stream);
   if (e != hipSuccess) {
-    if (a1) (void)hipFree(a1);
-    if (a2) (void)hipFree(a2);
+    if (a1) ctx_free(op->ctx, a1, b1);
+    if (a2) ctx_free(op->ctx, a2, b2);
     if (ccs) (void)hipFree(ccs);
     set_error(std::string("grid buffers for a batch: ") + hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? DDA_OUT_OF_MEMORY : DDA_HIP_ERROR;
   }
   op->device_bytes += (a1n + a2n + 3ull * d.nmat) * csz * (nrhs - op->cap_rhs);
-  (void)hipFree(op->a1);
-  (void)hipFree(op->a2);
+  release_large(op, op->a1, op->a1_bytes);
+  release_large(op, op->a2, op->a2_bytes);
   (void)hipFree(op->ccs);
   op->a1 = a1;
   op->a2 = a2;
+  op->a1_bytes = b1;
+  op->a2_bytes = b2;
   op->ccs = ccs;
   if (op->pack.nmember) {
     int* mem = nullptr;
@@ -1865,6 +2017,7 @@ extern "C" dda_status dda_op_apply_batch(dda_op_t op, const void* x_dev, void* y
     return DDA_INVALID_ARG;
   }
   hipStream_t st = stream ? (hipStream_t)stream : op->ctx->stream;
+  if (st != op->ctx->stream) op->foreign = true;
   if (op->prec == 64) return launch_matvec<double>(op, x_dev, y_dev, conj, st, nullptr, nrhs, 0);
   return launch_matvec<float>(op, x_dev, y_dev, conj, st, nullptr, nrhs, 0);
 }

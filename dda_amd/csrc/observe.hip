@@ -501,6 +501,7 @@ dda_status obs_scratch(dda_op_s* op, size_t bytes, void** out) {
 dda_status far_segments(dda_op_s* op) {
   dda_op_s::Far& far = op->far;
   if (far.made) return DDA_OK;
+  DDA_TRY(host_positions(op));
   const MvDims& d = op->dims;
   const int nrows = d.nrows, c2 = d.Bx - 1;  // twice the centre
   auto fold = [&](int x) { return std::abs(2 * x - c2) / 2; };
