@@ -93,8 +93,12 @@ template <bool NT> __device__ __forceinline__ void cstore(double2* p, double2 v)
 // waves per SIMD (128 VGPRs, a few spilled).
 // 32-point plans (FP32) hold 192 VGPRs of data: 2 waves per SIMD (256), as
 // general plans above 20 points are.
-template <typename R, int N, int PPT> struct P3Waves {
-  static constexpr int value = sizeof(R) == 4 ? (PPT > 20 ? 2 : PPT > 12 && N < 1024 ? 3 : 4) : 1;
+// 64 columns of 8-point threads are 512-thread work-groups: 6 waves per SIMD (80
+// VGPRs, without held twiddle powers) fit three of them to a CU, 5 only two (128
+// right-hand sides at 128 x 96 x 64: 739 us with two, 695 with three).
+template <typename R, int N, int PPT, int T> struct P3Waves {
+  static constexpr bool many = sizeof(R) == 4 && PPT <= 8 && T == 64;
+  static constexpr int value = sizeof(R) == 4 ? (PPT > 20 ? 2 : PPT > 12 && N < 1024 ? 3 : many ? 6 : 4) : 1;
 };
 
 // Pass 3 with a static plan of length N = Gz (see k_pass3 for the mapping).
@@ -109,7 +113,7 @@ template <typename R, int N, int PPT> struct P3Waves {
 // threads the ranges and, for the tensor, first_ok leave out).
 template <typename R, int N, int T, typename PL>
 __global__ __launch_bounds__(T * PL::TPC)
-__attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT>::value))) void k_pass3s(typename CxT<R>::T* a2,
+__attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT, T>::value))) void k_pass3s(typename CxT<R>::T* a2,
                                                                               const typename CxT<R>::T* __restrict__ dhat,
                                                 MvDims d, const typename CxT<R>::T* __restrict__ tw, int nwork,
                                                 int nper, int nrhs, RhsFlags fl) {
@@ -169,7 +173,7 @@ __attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT>::value))) void k_pass3
   // skip the zero upper half and the inverse ones never form it; two-stage
   // plans form the second-stage twiddle powers once for all six transforms
   // (FP64 and 32-point plans: no registers to spare)
-  constexpr bool PRE = TwoStage<N, TPC, F>::value && sizeof(R) == 4 && PPT <= 16;
+  constexpr bool PRE = TwoStage<N, TPC, F>::value && sizeof(R) == 4 && PPT <= 16 && !P3Waves<R, N, PPT, T>::many;
   C wp[PRE ? PPT - 1 : 1];
   if constexpr (PRE) twiddle_powers<PPT - 1, P::template twiddles<R>>(wp, t, tw);
   const C* twp = PRE ? wp : tw;
@@ -597,12 +601,21 @@ dda_status launch_pass3_plan(dda_op_s* op, const MvView& v, hipStream_t st, RhsF
   return DDA_OK;
 }
 
-// The other tile the tuner tries for the FP32 Z pass: 32 columns where the
-// default is 16 and 32 fit the work-group size the kernel's register budget
-// allows (MAXTH threads), else half the default.
+// The other tile of the FP32 Z pass: 64 columns where the default is 32 (at most
+// 64 points), 32 where it is 16 and 32 fit the work-group size the kernel's
+// register budget allows (MAXTH threads), else half the default.
 template <int T, int TPC, int MAXTH>
 constexpr int other_cols_z() {
-  return T != 32 && 32 * TPC <= MAXTH ? 32 : (T / 2) * TPC >= 64 ? T / 2 : T;
+  return T == 32 ? 64 : 32 * TPC <= MAXTH ? 32 : (T / 2) * TPC >= 64 ? T / 2 : T;
+}
+// Whether an untuned FP32 Z pass of at most 64 points takes the 64-column tile:
+// where tiles pair with their x mirrors (the tensor is read once for both) and
+// there are 24 work-groups per CU. 128 right-hand sides at 128 x 96 x 64: 695
+// against 756 us, at 128 x 96 x 48 536 against 567, x 32 378 against 381; 32 at
+// x 64 2.7% less for the whole product, 8 3% more; 64 x 64 x 64, where one tile
+// is its own mirror, 188 against 121 us.
+inline bool wide_z_tile(const MvDims& d, int nrhs) {
+  return d.Gx % 128 == 0 && (long long)(d.Gx / 64) * d.Gy * nrhs >= 6144;
 }
 
 template <typename R, int N, bool W, bool ALT = false>
@@ -616,7 +629,7 @@ dda_status launch_pass3_static_w(dda_op_s* op, const MvView& v, hipStream_t st, 
   constexpr int T0 = static_cols<R, N, W, (N == 1024 && sizeof(R) == 4 && W) ? 1024 : 512,
                                  (sizeof(R) == 4 && N <= 64) ? 32 : 0>();
   constexpr int TPC = N / StaticPlan<N, W>::PPT;
-  constexpr int T = ALT ? other_cols_z<T0, TPC, 256 * P3Waves<R, N, StaticPlan<N, W>::PPT>::value>() : T0;
+  constexpr int T = ALT ? other_cols_z<T0, TPC, 256 * P3Waves<R, N, StaticPlan<N, W>::PPT, T0>::value>() : T0;
   return launch_pass3_plan<R, N, StaticPlan<N, W>, T>(op, v, st, done, nrhs);
 }
 
@@ -655,7 +668,7 @@ dda_status launch_pass3_static(dda_op_s* op, const MvView& v, hipStream_t st, Rh
     if (var == 2 || var < 0) return launch_pass3_plan<R, N, Plan32<N>, 16>(op, v, st, done, nrhs);
     if (var == 3) return launch_pass3_plan<R, N, Plan32<N>, 8>(op, v, st, done, nrhs);
   } else if constexpr (sizeof(R) == 4) {
-    if (var >= 2)
+    if (var >= 2 || (N <= 64 && var < 0 && wide_z_tile(v.d, nrhs)))
       return (var & 1) ? launch_pass3_static_w<R, N, true, true>(op, v, st, done, nrhs)
                        : launch_pass3_static_w<R, N, false, true>(op, v, st, done, nrhs);
   }
