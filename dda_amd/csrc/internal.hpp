@@ -166,6 +166,11 @@ struct dda_op_s {
   uint32_t* row_meta = nullptr;   // [nv] x | mat << 16
   uint32_t* cell = nullptr;       // [Bz][By][Bx] dipole at each cell (compile-time planned X passes)
   uint32_t* row_list = nullptr;   // rows holding at least one dipole
+  // compile-time planned X passes: the rows that pass 1 transforms, and (with a
+  // planned Y pass; else null and all rows) each plane's occupied range [first, last + 1)
+  uint32_t* active_list = nullptr;
+  int2* yrange = nullptr;         // [Bz]
+  int n_active = 0;
   uint8_t* mat_dev = nullptr;     // [nv] material index per dipole
   int n_nonempty = 0;
   void* ccs = nullptr;            // [nmat][3] complex R, d^(-3/2) scaled

@@ -720,6 +720,8 @@ static dda_status launch_passes(dda_op_s* op, const void* xv, void* yv, int conj
     cp.pstride_out = d.rs;
     cp.bstride_in = (long long)d.By * d.rs;
     cp.bstride_out = d.p2;
+    cp.yr = use_ranges(op, nrhs) ? op->yrange : nullptr;
+    cp.nz = make_fastdiv(d.Bz);
     for (int q0 = 0; q0 < nrhs; q0 += rhs_per_col_launch) {
       const int k = std::min(rhs_per_col_launch, nrhs - q0);
       const long long nb0 = 3ll * d.Bz * q0;
@@ -787,6 +789,8 @@ static dda_status launch_passes(dda_op_s* op, const void* xv, void* yv, int conj
     cp.pstride_out = d.rs;
     cp.bstride_in = d.p2;
     cp.bstride_out = (long long)d.By * d.rs;
+    cp.yr = use_ranges(op, nrhs) ? op->yrange : nullptr;
+    cp.nz = make_fastdiv(d.Bz);
     for (int q0 = 0; q0 < nrhs; q0 += rhs_per_col_launch) {
       const int k = std::min(rhs_per_col_launch, nrhs - q0);
       const long long nb0 = 3ll * d.Bz * q0;
@@ -1266,7 +1270,7 @@ static void free_op(dda_op_s* op) {
   }
   if (op->pack.dhat_tab) (void)hipFree(op->pack.dhat_tab);
   if (op->pack.member_dev) (void)hipFree(op->pack.member_dev);
-  void* bufs[] = {op->cell, op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->tw[0], op->stage_x, op->stage_y, op->pos_dev, op->far_dev,
+  void* bufs[] = {op->cell, op->active_list, op->yrange, op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->tw[0], op->stage_x, op->stage_y, op->pos_dev, op->far_dev,
                   op->obs_scratch};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -1280,12 +1284,13 @@ void apply_cached_tuning(dda_op_s* op);
 
 // The index arrays of the compile-time planned X passes, formed on the device
 // from the positions: the cell map and the list of occupied rows. flags: bit 0 a
-// position outside the box, bit 1 two dipoles in one cell; then the rows' count.
+// position outside the box, bit 1 two dipoles in one cell; then the counts of the
+// occupied rows and of the active ones.
 __global__ void k_cells_clear(uint32_t* cell, long long ncell, uint32_t* occupied, int nrows, int* flags) {
   const long long i0 = blockIdx.x * (long long)blockDim.x + threadIdx.x, step = (long long)gridDim.x * blockDim.x;
   for (long long i = i0; i < ncell; i += step) cell[i] = kNoDipole;
   for (long long i = i0; i < nrows; i += step) occupied[i] = 0;
-  if (i0 < 2) flags[i0] = 0;
+  if (i0 < 3) flags[i0] = 0;
 }
 __global__ void k_cells(const uint32_t* __restrict__ pos, int nv, uint32_t Bx, uint32_t By, uint32_t Bz, uint32_t* cell,
                         uint32_t* occupied, int* flags) {
@@ -1300,9 +1305,26 @@ __global__ void k_cells(const uint32_t* __restrict__ pos, int nv, uint32_t Bx, u
     occupied[row] = 1;
   }
 }
-// One work-group: the occupied rows in order.
+// One wave per plane: its occupied range, and the rows in it (all: every row).
+__global__ __launch_bounds__(64) void k_row_ranges(const uint32_t* __restrict__ occupied, int By, int all, int2* yrange,
+                                                   uint32_t* __restrict__ active) {
+  const int z = blockIdx.x;
+  int lo = By, hi = 0;
+  for (int y = threadIdx.x; y < By; y += 64)
+    if (occupied[z * By + y]) {
+      lo = min(lo, y);
+      hi = max(hi, y + 1);
+    }
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o, 64));
+    hi = max(hi, __shfl_xor(hi, o, 64));
+  }
+  if (threadIdx.x == 0 && yrange) yrange[z] = make_int2(lo, hi);
+  for (int y = threadIdx.x; y < By; y += 64) active[z * By + y] = all || (y >= lo && y < hi);
+}
+// One work-group: the rows set in `occupied`, in order, and their count.
 __global__ __launch_bounds__(1024) void k_row_list(const uint32_t* __restrict__ occupied, int nrows,
-                                                   uint32_t* __restrict__ row_list, int* flags) {
+                                                   uint32_t* __restrict__ row_list, int* count) {
   __shared__ int sums[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int base = 0;
@@ -1321,7 +1343,7 @@ __global__ __launch_bounds__(1024) void k_row_list(const uint32_t* __restrict__ 
     base += all;
     __syncthreads();
   }
-  if (threadIdx.x == 0) flags[1] = base;
+  if (threadIdx.x == 0) *count = base;
 }
 
 // The rows of the (z, y) plane for the run-time planned X passes: counting sort
@@ -1390,9 +1412,17 @@ static dda_status build_index(dda_op_s* op, const uint32_t* pos, const dda_op_s*
   }
   DDA_TRY(dmalloc(&op->pos_dev, pb));
   DDA_TRY(dmalloc(&op->cell, ncell * 4));
-  DDA_TRY(dmalloc(&op->row_list, std::max(1, d.nrows) * 4ull));
-  if (like) {
+  DDA_TRY(dmalloc(&op->row_list, d.nrows * 4ull));
+  DDA_TRY(dmalloc(&op->active_list, d.nrows * 4ull));
+  // the run-time planned Y passes read and store every row
+  const bool ranges = op->gen[1] || has_static_plan(d.Gy);
+  if (ranges) DDA_TRY(dmalloc(&op->yrange, d.Bz * sizeof(int2)));
+  if (like && (like->yrange != nullptr) == ranges) {
     op->n_nonempty = like->n_nonempty;
+    op->n_active = like->n_active;
+    DDA_TRY_HIP(hipMemcpyAsync(op->active_list, like->active_list, d.nrows * 4ull, hipMemcpyDeviceToDevice, st));
+    if (ranges)
+      DDA_TRY_HIP(hipMemcpyAsync(op->yrange, like->yrange, d.Bz * sizeof(int2), hipMemcpyDeviceToDevice, st));
     DDA_TRY_HIP(hipMemcpyAsync(op->pos_dev, like->pos_dev, pb, hipMemcpyDeviceToDevice, st));
     DDA_TRY_HIP(hipMemcpyAsync(op->mat_dev, like->mat_dev, d.nv, hipMemcpyDeviceToDevice, st));
     DDA_TRY_HIP(hipMemcpyAsync(op->cell, like->cell, ncell * 4, hipMemcpyDeviceToDevice, st));
@@ -1400,26 +1430,33 @@ static dda_status build_index(dda_op_s* op, const uint32_t* pos, const dda_op_s*
     DDA_TRY_HIP(hipStreamSynchronize(st));
     return DDA_OK;
   }
-  DDA_TRY_HIP(hipMemcpyAsync(op->pos_dev, pos, pb, hipMemcpyHostToDevice, st));
+  if (like)
+    DDA_TRY_HIP(hipMemcpyAsync(op->pos_dev, like->pos_dev, pb, hipMemcpyDeviceToDevice, st));
+  else
+    DDA_TRY_HIP(hipMemcpyAsync(op->pos_dev, pos, pb, hipMemcpyHostToDevice, st));
   if (op->nmat > 1)
     DDA_TRY_HIP(hipMemcpyAsync(op->mat_dev, op->mat.data(), d.nv, hipMemcpyHostToDevice, st));
   else
     DDA_TRY_HIP(hipMemsetAsync(op->mat_dev, 0, d.nv, st));
   int* flags = (int*)op->a1;
   uint32_t* occupied = (uint32_t*)op->a1 + 64;
+  uint32_t* active = occupied + d.nrows;
   const int blocks = (int)std::min<size_t>(2048, (std::max<size_t>(ncell, d.nv) + 255) / 256);
   hipLaunchKernelGGL(k_cells_clear, dim3(blocks), dim3(256), 0, st, op->cell, (long long)ncell, occupied, d.nrows, flags);
   hipLaunchKernelGGL(k_cells, dim3(blocks), dim3(256), 0, st, (const uint32_t*)op->pos_dev, d.nv, d.Bx, d.By, d.Bz,
                      op->cell, occupied, flags);
-  hipLaunchKernelGGL(k_row_list, dim3(1), dim3(1024), 0, st, occupied, d.nrows, op->row_list, flags);
+  hipLaunchKernelGGL(k_row_ranges, dim3(d.Bz), dim3(64), 0, st, occupied, d.By, ranges ? 0 : 1, op->yrange, active);
+  hipLaunchKernelGGL(k_row_list, dim3(1), dim3(1024), 0, st, occupied, d.nrows, op->row_list, flags + 1);
+  hipLaunchKernelGGL(k_row_list, dim3(1), dim3(1024), 0, st, active, d.nrows, op->active_list, flags + 2);
   DDA_TRY_HIP(hipGetLastError());
-  int h[2] = {0, 0};
+  int h[3] = {0, 0, 0};
   DDA_TRY_HIP(copy_sync(h, flags, sizeof h, hipMemcpyDeviceToHost, st));
   if (h[0] & 1) {
     set_error(kBadDipole);
     return DDA_INVALID_ARG;
   }
   op->n_nonempty = h[1];
+  op->n_active = h[2];
   if (h[0] & 2) {  // dipoles that share a cell go by the rows' lists
     op->static_x = false;
     op->gen[0] = nullptr;
@@ -2205,6 +2242,8 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
         cp.pstride_in = cp.pstride_out = d.rs;
         cp.bstride_in = inv ? d.p2 : (long long)d.By * d.rs;
         cp.bstride_out = inv ? (long long)d.By * d.rs : d.p2;
+        cp.yr = use_ranges(op, nrhs) ? op->yrange : nullptr;
+        cp.nz = make_fastdiv(d.Bz);
         const void* in = inv ? op->a2 : op->a1;
         void* out = inv ? op->a1 : op->a2;
         // one launch's worth of column batches (a matvec splits larger blocks)

@@ -27,12 +27,19 @@ struct MvView {
 
 // Strided column FFT over T adjacent columns. Column `col` of batch b, point p
 // lives at base[b * bstride + p * pstride + col]; inputs beyond in_len are zero,
-// only the first out_len points are stored.
+// only the first out_len points are stored. With yr (the matvec's Y passes, batch
+// b of plane b mod nz), a forward transform reads and an inverse one stores the
+// plane's occupied range [yr.x, yr.y) alone: the rows outside it are zero before
+// and no dipole's after. A particle that fills 79% of its rows (any ellipsoid)
+// saves a fifth of A1's traffic: two FP32 right-hand sides at 256^3 606 -> 579
+// us, 128 at 128 x 96 x 64 1,657 -> 1,580.
 struct ColParams {
   int ncols;
   int in_len, out_len;
   long long pstride_in, pstride_out;
   long long bstride_in, bstride_out;
+  const int2* yr = nullptr;
+  FastDiv nz = {1, 0, 0};
 };
 
 // ------------------------------------------------------------------------------------
@@ -237,7 +244,8 @@ __attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT, T>::value))) void k_pa
 }
 
 // Pass 1 with a static plan of length N = Gx. A work-group takes LN consecutive
-// lines g = c * nrows + row of the A1 layout (contiguous in A1); thread (l, t),
+// lines g = c * n_list + slot over the rows of row_list (those in the planes'
+// occupied ranges, which pass 2 reads; null: every row); thread (l, t),
 // t = tid mod TPC along the line, reads its first-stage points straight from the
 // vector through the cell map (only x < Bx <= N/2 can hold dipoles) and stores
 // its outputs, TPC consecutive points per line, coalesced.
@@ -247,6 +255,7 @@ __attribute__((amdgpu_waves_per_eu(P3Waves<R, N, PL::PPT, T>::value))) void k_pa
 template <typename R, int N, typename PL, int BS = 256>
 __global__ __launch_bounds__(BS) void k_pass1s(const typename CxT<R>::T* __restrict__ x,
                                                 typename CxT<R>::T* __restrict__ a1,
+                                                const uint32_t* __restrict__ row_list, int n_list,
                                                 const uint32_t* __restrict__ cell, const uint8_t* __restrict__ mat,
                                                 const typename CxT<R>::T* __restrict__ ccs, MvDims d,
                                                 const typename CxT<R>::T* __restrict__ tw, int conj, RhsFlags fl) {
@@ -271,10 +280,11 @@ __global__ __launch_bounds__(BS) void k_pass1s(const typename CxT<R>::T* __restr
   extern __shared__ char smem[];
   C* tile = reinterpret_cast<C*>(smem);
   const int t = threadIdx.x % TPC, l = threadIdx.x / TPC;
-  const int nlines = 3 * d.nrows;
+  const int nlines = 3 * n_list;
   const int g = l < LN ? (int)blockIdx.x * LN + l : nlines;
   const bool ok = g < nlines;
-  const int c = ok ? g / d.nrows : 0, row = ok ? g - c * d.nrows : 0;
+  const int c = ok ? g / n_list : 0, slot = ok ? g - c * n_list : 0;
+  const int row = row_list ? (int)row_list[slot] : slot;
   const uint32_t* cells = cell + (size_t)row * d.Bx;
   x += (size_t)c * d.S;
   uint32_t at[NF];
@@ -294,7 +304,7 @@ __global__ __launch_bounds__(BS) void k_pass1s(const typename CxT<R>::T* __restr
   }
   RunStages<N, TPC, false, 1, C, F, true, P::template twiddles<R>>::run(v, t, tile, lp, l, tw);
   if (ok) {
-    C* dst = a1 + (size_t)g * d.rs;
+    C* dst = a1 + ((size_t)c * d.nrows + row) * d.rs;
 #pragma unroll
     for (int e = 0; e < NO; e++)
       if (first_ok<N, TPC, Out>(t, e)) cstore<true>(dst + first_point<N, TPC, Out>(t, e), v[e]);
@@ -445,17 +455,24 @@ __global__ __launch_bounds__(T * PL::TPC) void k_colfft_s(const typename CxT<R>:
   const bool colok = col < cp.ncols;
   const C* src = in + (long long)blockIdx.y * cp.bstride_in + col;
   C* dst = out + (long long)blockIdx.y * cp.bstride_out + col;
+  int in0 = 0, in1 = cp.in_len, out0 = 0, out1 = cp.out_len;
+  if (cp.yr) {
+    const int2 r = cp.yr[cp.nz.mod(blockIdx.y)];
+    (INV ? out0 : in0) = r.x;
+    (INV ? out1 : in1) = r.y;
+  }
   C v[PPT];
 #pragma unroll
   for (int e = 0; e < NF; e++) {
     const int p = first_point<N, TPC, F>(t, e);
-    v[e] = (!(HIN && upper_half<F>(e)) && first_ok<N, TPC, F>(t, e) && colok && p < cp.in_len) ? src[p * cp.pstride_in] : czero<C>();
+    v[e] = (!(HIN && upper_half<F>(e)) && first_ok<N, TPC, F>(t, e) && colok && p >= in0 && p < in1)
+               ? src[p * cp.pstride_in] : czero<C>();
   }
   RunStages<N, TPC, INV, 1, C, F, HIN, P::template twiddles<R>>::run(v, t, tile, lp, l, tw);
 #pragma unroll
   for (int e = 0; e < NO; e++) {
     const int p = first_point<N, TPC, Out>(t, e);
-    if (!(HOUT && upper_half<Out>(e)) && first_ok<N, TPC, Out>(t, e) && colok && p < cp.out_len)
+    if (!(HOUT && upper_half<Out>(e)) && first_ok<N, TPC, Out>(t, e) && colok && p >= out0 && p < out1)
       cstore<INV>(dst + p * cp.pstride_out, v[e]);
   }
 }
@@ -569,6 +586,16 @@ dda_status launch_col_static(const void* in, void* out, const ColParams& cp, con
   }
   return plan_wide<R>(wide >= 2 ? (wide & 1) : wide) ? launch_col_static_w<R, N, true, INV>(in, out, cp, tw, nbatch, st, done)
                                                     : launch_col_static_w<R, N, false, INV>(in, out, cp, tw, nbatch, st, done);
+}
+
+// Whether the passes of nrhs right-hand sides leave out the rows outside the
+// planes' occupied ranges: where A1 is larger than half of the L2s. In a small
+// one the saved lines cost nothing and the ranges' loads come before the data's:
+// the product of the sphere 40 across (6 MB) 37.6 us with them, 37.0 without;
+// 256^3 (200 MB) 598 and 622.
+inline bool use_ranges(const dda_op_s* op, int nrhs) {
+  const MvDims& d = op->dims;
+  return op->yrange && (size_t)nrhs * 3 * d.nrows * d.rs * (op->prec / 4) > (16u << 20);
 }
 
 inline MvView view_of(const dda_op_s* op, int r0) {
@@ -688,8 +715,10 @@ dda_status launch_x_plan(dda_op_s* op, const MvView& v, bool inverse, const void
   if (!inverse) {
     auto k = k_pass1s<R, N, PL, BS>;
     DDA_TRY(set_lds(k, lds));
-    hipLaunchKernelGGL(k, dim3((3 * d.nrows + LN - 1) / LN, nrhs), dim3(BS), lds, st, (const C*)x, (C*)v.a1,
-                       op->cell, op->mat_dev, (const C*)v.ccs, d, (const C*)op->tw[0], conj, done);
+    const bool part = use_ranges(op, nrhs);
+    const int n = part ? op->n_active : d.nrows;
+    hipLaunchKernelGGL(k, dim3((3 * n + LN - 1) / LN, nrhs), dim3(BS), lds, st, (const C*)x, (C*)v.a1,
+                       part ? op->active_list : nullptr, n, op->cell, op->mat_dev, (const C*)v.ccs, d, (const C*)op->tw[0], conj, done);
   } else {
     auto k = k_pass5s<R, N, PL, BS>;
     DDA_TRY(set_lds(k, lds));

@@ -326,3 +326,28 @@ def test_dipoles_that_share_a_cell(ctx, precision):
     y2 = apply(D.MatVecGpu(twice), twice, np.concatenate([x, x[:, 7:9]], 1))
     tol = FP64_TOL if precision == 64 else FP32_TOL
     assert cases.rel_err(y2, np.concatenate([y1, y1[:, 7:9]], 1)) <= tol
+
+
+@pytest.mark.parametrize("grid", [(16, 16, 16), (32, 48, 32), (18, 512, 20), (20, 540, 16)])
+@pytest.mark.parametrize("precision", [64, 32])
+def test_rows_with_gaps(ctx, grid, precision):
+    """Planes whose occupied rows start late, end early, leave rows out or are
+    missing altogether, after a product of NaNs in the same buffers, planned
+    and (540 points) run-time planned Y passes, against the oracle."""
+    rng = np.random.default_rng(17)
+    box = (7, min(grid[1] // 2, 40), 8)
+    z, y, x = np.meshgrid(*(np.arange(b) for b in box[::-1]), indexing="ij")
+    keep = (rng.random(x.shape) < 0.5) & (y % 5 != 3) & (z != 4) & (y >= z) & ((y < 7) | (z != 2))
+    g = P.DipoleGeometry(np.stack([a[keep] for a in (x, y, z)], 1), None, [1.5 + 0.1j], 0.5e-6)
+    params = P.DDAParams(g, 6e-6, grid)
+    cs = P.couple_constants(params, *P.beam_pols((0.3, -0.2, 0.8))[:2])[1]
+    bad = _ops(ctx, g, params, cs, precision)
+    D.MatVecGpu(bad).apply(np.full(params.vec_size, np.nan + 0j))
+    bad.close()
+    orc = cases.oracle_problem(g, params, cs, dmat_precision=64)
+    v = P.random_dipole_vector(params, seed=4)
+    op = _ops(ctx, g, params, cs, precision)
+    for conj in (False, True):
+        yy = D.MatVecGpu(op).apply(v, conj=conj)
+        assert cases.rel_err(yy, orc.matvec(v, conj=conj, precision=64)) <= (FP64_TOL if precision == 64 else FP32_TOL)
+    op.close()
