@@ -37,6 +37,10 @@ constexpr int kRedThreads = 256;
 constexpr int kMaxRedBlocks = 1024;
 constexpr int kChunk = 16;  // most iterations enqueued between state reads
 
+// Partial sums of a pass 5 that QMR-CS's next vector kernel adds in each of its
+// work-groups instead of waiting for a scalar step (two loads a thread).
+constexpr int kOwnSums = 512;
+
 // Work-groups per right-hand side for vectors of n complex values: two values a
 // thread until that fills kMaxRedBlocks work-groups. (Eight a thread left short
 // vectors on few CUs, each thread's loads in series: at 33,552 dipoles, FP64,
@@ -249,17 +253,35 @@ __global__ __launch_bounds__(kRedThreads) void k_lincomb(typename CxT<R>::T* out
 
 // QMR-CS: vtilda = [vtilda * mBeta] + v * mAlpha + Av, with partials of
 // vtilda.vtilda (quantities 0, 1) and |vtilda|^2 (2). QmrCs.cpp:96-104.
+// part5 (nullable): alpha = v.Av is not in the state yet but in these nb5 partial
+// sums of the matvec's pass 5, which every work-group adds for itself.
 template <typename R>
 __global__ __launch_bounds__(kRedThreads) void k_qmr_vt(typename CxT<R>::T* vt, const typename CxT<R>::T* __restrict__ v,
                                                         const typename CxT<R>::T* __restrict__ av, int first,
-                                                        const SolverState* st, long long n, double* part) {
+                                                        SolverState* st, long long n, double* part,
+                                                        const double* __restrict__ part5, int nb5) {
   typedef typename CxT<R>::T C;
   DDA_RHS_PROLOGUE(st)
   if (s_->done) return;
+  double2 mal = s_->mAlpha;
+  if (part5) {
+    part5 += (long long)rhs_ * 4 * nb5;
+    double a0 = 0, a1 = 0;
+    for (int i = threadIdx.x; i < nb5; i += kRedThreads) {
+      a0 += part5[i];
+      a1 += part5[nb5 + i];
+    }
+    const double al = block_sum(a0), ali = block_sum(a1);
+    mal = make_double2(-al, -ali);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      st[rhs_].alpha = make_double2(al, ali);
+      st[rhs_].mAlpha = mal;
+    }
+  }
   vt += off_;
   v += off_;
   av += off_;
-  const C mb = coef<C>(&s_->mBeta), ma = coef<C>(&s_->mAlpha);
+  const C mb = coef<C>(&s_->mBeta), ma = cmake<C>(mal.x, mal.y);
   double s0 = 0, s1 = 0, s2 = 0;
   DDA_GRID_LOOP(i) {
     C o = cadd(cmul(v[i], ma), av[i]);
@@ -422,13 +444,12 @@ enum Step {
   S_QMR_INIT = 10,
   S_QMR_ALPHA = 11,
   S_QMR_GIVENS = 12,
-  S_END_ITER = 13,   // LoopUpdate + loop head (all solvers)
+  S_END_ITER = 13,   // LoopUpdate + loop head (all solvers); BiCGStab: the next iteration's S_BS_RO too
   S_BS_RO = 20,
   S_BS_ALPHA = 21,
   S_BS_S = 22,
   S_BS_OMEGA = 23,
   S_BS_END = 24,
-  S_BS_RO1 = 25,     // S_BS_RO with r.conj(rtilda) from the previous x/r update (partials 1, 2)
   S_CG_RO = 30,
   S_CG_ALPHA = 31,
   S_BI_RO = 40,
@@ -467,6 +488,26 @@ __device__ inline void loop_head(SolverState* st, int kind) {
   st->skip = st->done;
 }
 
+// The start of a BiCGStab iteration, from rho = r.conj(rtilda) (BicgStab.cpp:66-78).
+__device__ inline void bicgstab_rho(SolverState* st, double2 rho) {
+  st->ro_new = rho;
+  const double dtmp = dabs(st->ro_new) / st->inprodR;
+  if (!(dtmp >= 1e-16)) {
+    finish(st, DDA_BREAKDOWN);
+    return;
+  }
+  if (st->count > 0) {
+    const double2 ro_new_alpha = dmul(st->ro_new, st->alpha);
+    const double2 ro_old_omega = dmul(st->ro_old, st->omega);
+    if (!(dabs(ro_old_omega) / dabs(ro_new_alpha) >= 10e-10)) {
+      finish(st, DDA_BREAKDOWN);
+      return;
+    }
+    st->bbeta = ddiv(ro_new_alpha, ro_old_omega);
+    st->mbo = dneg(dmul(st->bbeta, st->omega));
+  }
+}
+
 __global__ __launch_bounds__(kScalarThreads) void k_scalar(SolverState* st_all, const double* part_all, int nb, int step,
                                                         int kind, double* hist_all) {
   const int rhs = blockIdx.x;
@@ -480,7 +521,6 @@ __global__ __launch_bounds__(kScalarThreads) void k_scalar(SolverState* st_all, 
     case S_INIT_TEMP:
     case S_INIT_R:
     case S_INIT_START:
-    case S_END_ITER:
     case S_CG_RO:
     case S_CG_ALPHA:
     case S_BS_S:
@@ -496,8 +536,10 @@ __global__ __launch_bounds__(kScalarThreads) void k_scalar(SolverState* st_all, 
       break;
     case S_QMR_GIVENS:
     case S_BS_OMEGA:
-    case S_BS_RO1:
       nq = 3;
+      break;
+    case S_END_ITER:
+      nq = kind == DDA_SOLVER_BICGSTAB ? 3 : 1;
       break;
     default:
       break;
@@ -625,29 +667,14 @@ __global__ __launch_bounds__(kScalarThreads) void k_scalar(SolverState* st_all, 
           }
         }
       }
+      // r.conj(rtilda) of the x/r update, for the next iteration
+      if (kind == DDA_SOLVER_BICGSTAB && !st->done) bicgstab_rho(st, make_double2(q1, q2));
       break;
     }
     // ---- BiCGStab, BicgStab.cpp:66-112 ----
     case S_BS_RO:
-    case S_BS_RO1: {
-      st->ro_new = step == S_BS_RO1 ? make_double2(q1, q2) : make_double2(q0, q1);
-      const double dtmp = dabs(st->ro_new) / st->inprodR;
-      if (!(dtmp >= 1e-16)) {
-        finish(st, DDA_BREAKDOWN);
-        break;
-      }
-      if (st->count > 0) {
-        const double2 ro_new_alpha = dmul(st->ro_new, st->alpha);
-        const double2 ro_old_omega = dmul(st->ro_old, st->omega);
-        if (!(dabs(ro_old_omega) / dabs(ro_new_alpha) >= 10e-10)) {
-          finish(st, DDA_BREAKDOWN);
-          break;
-        }
-        st->bbeta = ddiv(ro_new_alpha, ro_old_omega);
-        st->mbo = dneg(dmul(st->bbeta, st->omega));
-      }
+      bicgstab_rho(st, make_double2(q0, q1));
       break;
-    }
     case S_BS_ALPHA:
       st->alpha = ddiv(st->ro_new, make_double2(q0, q1));
       st->mAlpha = dneg(st->alpha);
@@ -1100,8 +1127,19 @@ struct Core {
         case DDA_SOLVER_QMR_CS: {
           C* vv = v[iv];
           C* vt = v[ivt];
-          DDA_TRY(matvec_sums(vv, av, 0, DONE, DOT_U, S_QMR_ALPHA));  // alpha = v.Av
-          hipLaunchKernelGGL(k_qmr_vt<R>, g(), b(), 0, st, vt, vv, av, nr == 0 ? 1 : 0, dst, n, part);
+          // alpha = v.Av; few partial sums are added by k_qmr_vt itself
+          bool own = false;
+          if (fused) {
+            DDA_TRY(launch_matvec<R>(op, vv, av, 0, st, flag(DONE), nrhs, kStateInts, part5, DOT_U));
+            own = op->p5_blocks <= kOwnSums;
+            if (!own)
+              hipLaunchKernelGGL(k_scalar, dim3(nrhs), dim3(kScalarThreads), 0, st, dst, part5, op->p5_blocks,
+                                 S_QMR_ALPHA, kind, hist);
+          } else {
+            DDA_TRY(matvec_sums(vv, av, 0, DONE, DOT_U, S_QMR_ALPHA));
+          }
+          hipLaunchKernelGGL(k_qmr_vt<R>, g(), b(), 0, st, vt, vv, av, nr == 0 ? 1 : 0, dst, n, part,
+                             own ? part5 : nullptr, op->p5_blocks);
           scalar(S_QMR_GIVENS);
           const int mode = nr == 0 ? 0 : (nr == 1 ? 1 : 2);
           hipLaunchKernelGGL(k_qmr_upd<R>, g(), b(), 0, st, v[ipo], v[ipn], vv, vt, x, r, mode, dst, n, part);
@@ -1115,11 +1153,9 @@ struct Core {
           C* vv = v[5];
           C* sv = v[6];
           C* rt = v[7];
-          if (nr == 0) {
+          if (nr == 0) {  // later: at the end of the iteration before
             reduce(RED_DOTC, r, rt, DONE);
             scalar(S_BS_RO);
-          } else {
-            scalar(S_BS_RO1);  // rho from the previous x/r update's partials
           }
           hipLaunchKernelGGL(k_bs_p<R>, g(), b(), 0, st, p, vv, r, nr == 0 ? 1 : 0, dst, n);
           DDA_TRY(matvec(p, vv, 0, DONE));
