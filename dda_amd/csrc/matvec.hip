@@ -557,22 +557,37 @@ inline bool has_static_plan(int n) {
   }
 }
 
-// The static Z pass (k_pass3s) addresses A2 and each component of the tensor
-// octant with 32-bit byte offsets from uniform bases: a tensor component spans
-// (Gx/2+1)(Gy/2+1)(Gz/2+1) elements, and one buffer range of A2 at most
-// Gz/8 planes of Gy*Gx elements (its plans have at least 8 points per
-// thread). Grids beyond that run the run-time planned Z pass, whose addressing
-// is 64-bit.
-inline bool z_offsets_fit(int Gx, int Gy, int Gz, size_t csz) {
-  const uint64_t lim = 1ull << 32;
-  const uint64_t oct = (uint64_t)(Gx / 2 + 1) * (Gy / 2 + 1) * (Gz / 2 + 1);
-  // (a general plan of a short length holds fewer points, at most 28 threads
-  // or an eighth of the length per column)
-  const uint64_t span = (uint64_t)std::max(Gz / 8 + 1, std::min(Gz, 28)) * (Gy + 1) * row_stride(Gx, csz == sizeof(double2) ? 64 : 32);
-  return oct * csz < lim && span * csz < lim;
+// Threads per column of the tuned Z plans at length n, at most (variants differ);
+// 0: no such plan.
+inline int static_z_threads(int n) {
+  switch (n) {
+#define X(N) \
+  case N:    \
+    return std::max(StaticPlan<N, false>::TPC, StaticPlan<N, true>::TPC);
+    DDA_STATIC_SIZES(X)
+#undef X
+    default:
+      return 0;
+  }
 }
-inline bool static_z_fits(int Gx, int Gy, int Gz, size_t csz) {
-  return has_static_plan(Gz) && z_offsets_fit(Gx, Gy, Gz, csz);
+
+// The compile-time planned Z pass (k_pass3s) addresses A2 and each component of
+// the tensor octant with 32-bit byte offsets from uniform bases: a component
+// spans (Gx/2+1)(Gy/2+1)(Gz/2+1) elements, and thread t of a column addresses
+// plane t from a base, so the offsets of a plan of `threads` threads span as many
+// planes of A2. Also of the threads that a stage has no butterfly for: only the
+// end of the buffer's range keeps those from storing, and an offset that wraps
+// past 4 GiB is inside it again. Grids beyond that run the run-time planned Z
+// pass, whose addressing is 64-bit.
+inline bool z_offsets_fit(int Gx, int Gy, int Gz, int prec, int threads) {
+  const uint64_t lim = 1ull << 32, csz = prec == 64 ? sizeof(double2) : sizeof(float2);
+  const uint64_t oct = (uint64_t)(Gx / 2 + 1) * (Gy / 2 + 1) * (Gz / 2 + 1);
+  const uint64_t plane = (uint64_t)Gy * row_stride(Gx, prec) + line_elems(prec);
+  return oct * csz < lim && threads * plane * csz < lim;
+}
+inline bool static_z_fits(int Gx, int Gy, int Gz, int prec) {
+  const int threads = static_z_threads(Gz);
+  return threads && z_offsets_fit(Gx, Gy, Gz, prec, threads);
 }
 
 template <typename R, bool INV>
@@ -1182,10 +1197,18 @@ extern "C" dda_status dda_grid_plan(const uint32_t grid[3], int precision, int* 
     set_error("dda_grid_plan: null grid or precision not 32/64");
     return DDA_INVALID_ARG;
   }
-  const size_t csz = precision == 64 ? sizeof(double2) : sizeof(float2);
   if (static_x) *static_x = has_static_plan((int)grid[0]) ? 1 : 0;
-  if (static_z) *static_z = static_z_fits((int)grid[0], (int)grid[1], (int)grid[2], csz) ? 1 : 0;
+  if (static_z) *static_z = static_z_fits((int)grid[0], (int)grid[1], (int)grid[2], precision) ? 1 : 0;
   return DDA_OK;
+}
+
+// For the tests, not in the header: threads per column of the compile-time planned
+// Z pass that an operator on `grid` runs, 0 where it runs the run-time planned one.
+extern "C" int dda_z_pass_threads(const uint32_t grid[3], int precision) {
+  const int gx = (int)grid[0], gy = (int)grid[1], gz = (int)grid[2];
+  const AxisOps* gen = axis_ops(gz, precision);
+  const int threads = gen ? gen->z_threads : static_z_threads(gz);
+  return threads && z_offsets_fit(gx, gy, gz, precision, threads) ? threads : 0;
 }
 
 extern "C" uint32_t dda_fft_fit_static(uint32_t x) {
@@ -1537,8 +1560,8 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
   const size_t csz = precision == 64 ? sizeof(double2) : sizeof(float2);
   if (!std::getenv("DDA_GENERIC_FFT")) {
     for (int a = 0; a < 3; a++) op->gen[a] = axis_ops(grid[a], precision);
-    if (!z_offsets_fit(d.Gx, d.Gy, d.Gz, csz)) op->gen[2] = nullptr;
-    op->static_z = op->gen[2] || static_z_fits(d.Gx, d.Gy, d.Gz, csz);
+    op->static_z = dda_z_pass_threads(grid, precision) != 0;
+    if (!op->static_z) op->gen[2] = nullptr;
     op->static_x = op->gen[0] || has_static_plan(d.Gx);
   }
   op->split_rhs = std::getenv("DDA_SPLIT") && std::atoi(std::getenv("DDA_SPLIT")) != 0;

@@ -113,8 +113,8 @@ template <typename R, int N, int PPT, int T> struct P3Waves {
 // first stage (K_e a compile-time constant per register e), so one lane offset
 // t * Gy * Gx + l addresses all of them from per-(component, e) uniform bases;
 // each such buffer's range ends at z = Bz (points at and beyond it read as zero
-// and are not stored) and spans at most TPC planes (it stays below 4 GiB up
-// to 1024^3). The tensor is read through one buffer per component with a lane
+// and are not stored) and spans at most TPC planes, which have to stay below 4 GiB
+// (z_offsets_fit). The tensor is read through one buffer per component with a lane
 // offset per point.
 // PL is the plan (StaticPlan<N, W>, a PlanOf variant or a GenPlan, whose idle
 // threads the ranges and, for the tensor, first_ok leave out).
@@ -808,6 +808,7 @@ struct AxisOps {
   dda_status (*z)(dda_op_s* op, const MvView& v, hipStream_t st, RhsFlags done, int nrhs);
   dda_status (*x)(dda_op_s* op, const MvView& v, bool inverse, const void* x, void* y, int conj, hipStream_t st,
                   RhsFlags done, int nrhs, const PassDotReq& dr);
+  int z_threads;  // threads per column of the Z pass
 };
 
 // The column passes of the interaction tensor's generation: nb batches of ncols

@@ -31,7 +31,7 @@ template <int N, typename PL, typename PZ>
 const AxisOps* ops_of() {
   static const AxisOps ops = {launch_gen_col<Real, N, PL>,
                               launch_pass3_plan<Real, N, PZ, gen_cols<Real, N, PZ::TPC>(16)>,
-                              launch_x_plan<Real, N, PL>};
+                              launch_x_plan<Real, N, PL>, PZ::TPC};
   return &ops;
 }
 

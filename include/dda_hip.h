@@ -87,8 +87,9 @@ uint32_t dda_fft_fit_static(uint32_t x);
  * counterpart in the reference, whose FFT plans are chosen at run time,
  * DDA/GpuFFTPlans.cpp:34-61): static_x for the X passes (Gx has a static
  * plan), static_z for the Z pass with the tensor product (Gz has one and every
- * byte offset of that pass fits 32 bits: the tensor octant's components and
- * Gz/8 planes of the grid each below 4 GiB). Other grids use the run-time
+ * byte offset of that pass fits 32 bits: the tensor octant's components, and as
+ * many planes of the grid as the pass has threads per column, Gz/8 at most, each
+ * below 4 GiB). Other grids use the run-time
  * planned kernels. Host-only. */
 dda_status dda_grid_plan(const uint32_t grid[3], int precision, int* static_x, int* static_z);
 
