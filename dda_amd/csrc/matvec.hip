@@ -2008,6 +2008,10 @@ static dda_status ensure_rhs_capacity(dda_op_s* op, int nrhs) {
   return DDA_OK;
 }
 
+// For the tests, not in the header: whether a product of nrhs right-hand sides
+// leaves out the rows outside the planes' occupied ranges.
+extern "C" int dda_op_row_ranges(dda_op_t op, int nrhs) { return use_ranges(op, nrhs) ? 1 : 0; }
+
 // Uploads sqrt(cc) for RHS first .. first+nrhs-1 ([nrhs][nmat][3] complex double,
 // m^(3/2)), d^(-3/2) scaled into the operator's precision.
 static dda_status upload_ccs(dda_op_s* op, const double* cc_sqrt, int first, int nrhs) {
