@@ -237,9 +237,13 @@ __device__ inline void jones_frame(const FarGrid& g, int i, int f, double n[3], 
     pa[a] = -st * g.prop[a] + ct * (cp * X + sp * Y);
   }
 }
+// Component a of a slot's direction in dirs (64-bit: 2^30 slots are accepted).
+__host__ __device__ constexpr size_t dir_index(int slot, int a) { return 3 * (size_t)slot + a; }
+static_assert(dir_index((1 << 30) - 1, 2) == 3221225471u, "direction index");
+
 __device__ inline void far_direction(const FarDirs& f, int slot, double n[3]) {
   if (f.dirs) {
-    for (int a = 0; a < 3; a++) n[a] = f.dirs[3 * slot + a];
+    for (int a = 0; a < 3; a++) n[a] = f.dirs[dir_index(slot, a)];
   } else {
     double pe[3], pa[3];
     if (f.g.symmetric)
@@ -899,7 +903,7 @@ extern "C" dda_status dda_far_field(dda_op_t op, const void* pol_dev, int nrhs, 
       std::vector<int> hi(slots + slots / 64, -1);
       for (int i = 0; i < nq; i++) {
         const int r = rhs ? rhs[i] : 0, s = fill[r]++;
-        for (int a = 0; a < 3; a++) hd[3 * (size_t)s + a] = dirs[3 * (size_t)i + a];
+        for (int a = 0; a < 3; a++) hd[dir_index(s, a)] = dirs[dir_index(i, a)];
         hi[s] = i;
         hi[slots + s / 64] = r;
       }
@@ -937,8 +941,8 @@ extern "C" dda_status dda_far_field(dda_op_t op, const void* pol_dev, int nrhs, 
   double* od = part + 6ull * nchunk * nq;
   std::vector<double> hq(4ull * nq);
   for (int i = 0; i < nq; i++) {
-    hq[4 * i] = rhs ? rhs[i] : 0;
-    for (int a = 0; a < 3; a++) hq[4 * i + 1 + a] = dirs[3 * i + a];
+    hq[4ull * i] = rhs ? rhs[i] : 0;
+    for (int a = 0; a < 3; a++) hq[4ull * i + 1 + a] = dirs[dir_index(i, a)];
   }
   hipStream_t st = op->ctx->stream;
   DDA_TRY_HIP(hipMemcpyAsync(qd, hq.data(), qbytes, hipMemcpyHostToDevice, st));
