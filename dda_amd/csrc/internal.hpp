@@ -230,7 +230,8 @@ struct dda_op_s {
     int npos = 0, nchunk = 0;
     const void *segs = nullptr, *wave_seg = nullptr;
   } far;
-  void* far_dev = nullptr;
+  void* far_dev = nullptr;      // used on the context's stream alone
+  size_t far_bytes = 0;
   void* obs_scratch = nullptr;  // observables' work space
   size_t obs_bytes = 0;  // dda_op_tune ran (an FP32 twin of a tuned operator is tuned too)
   bool static_x = false;  // X passes with a compile-time plan (Gx has one)

@@ -1293,13 +1293,14 @@ static void free_op(dda_op_s* op) {
   }
   if (op->pack.dhat_tab) (void)hipFree(op->pack.dhat_tab);
   if (op->pack.member_dev) (void)hipFree(op->pack.member_dev);
-  void* bufs[] = {op->cell, op->active_list, op->yrange, op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->tw[0], op->stage_x, op->stage_y, op->pos_dev, op->far_dev,
-                  op->obs_scratch};
+  void* bufs[] = {op->cell, op->active_list, op->yrange, op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->tw[0], op->stage_x, op->stage_y, op->pos_dev};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
   release_large(op, op->a1, op->a1_bytes);
   release_large(op, op->a2, op->a2_bytes);
   release_large(op, op->dhat, op->dhat_bytes);
+  ctx_free(op->ctx, op->far_dev, op->far_bytes);
+  ctx_free(op->ctx, op->obs_scratch, op->obs_bytes);
   delete op;
 }
 

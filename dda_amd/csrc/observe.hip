@@ -9,7 +9,6 @@
 // go through one two-stage reduction, many directions as a matrix product.
 #include <cmath>
 #include <complex>
-#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -479,89 +478,239 @@ dda_status positions_on_device(dda_op_s* op) {
   return DDA_OK;
 }
 
-// Device scratch of at least `bytes`, kept by the operator between calls.
+// Device scratch of at least `bytes`, kept by the operator between calls (a
+// hipMalloc of some megabytes takes 300 us: the context's spare buffers serve a
+// new operator's first call).
 dda_status obs_scratch(dda_op_s* op, size_t bytes, void** out) {
   if (op->obs_bytes < bytes) {
     if (op->obs_scratch) {
       DDA_TRY_HIP(hipStreamSynchronize(op->ctx->stream));
-      (void)hipFree(op->obs_scratch);
+      ctx_free(op->ctx, op->obs_scratch, op->obs_bytes);
       op->device_bytes -= op->obs_bytes;
       op->obs_scratch = nullptr;
       op->obs_bytes = 0;
     }
-    DDA_TRY_HIP(hipMalloc(&op->obs_scratch, bytes));
-    op->obs_bytes = bytes;
-    op->device_bytes += bytes;
+    size_t got = 0;
+    DDA_TRY_HIP(ctx_alloc(op->ctx, &op->obs_scratch, bytes, &got));
+    op->obs_bytes = got;
+    op->device_bytes += got;
   }
   *out = op->obs_scratch;
   return DDA_OK;
 }
 
+// ------------------------------------------------------------------------------------
 // The operator's positions as k_far_rows takes them, made on first use: the
 // folded halves of the occupied rows, each from its innermost to its outermost
 // dipole, in segments of at most 32 steps, dealt to the waves in equal numbers of
-// steps. far.npos stays 0 where the rows are mostly holes (four positions and
-// more per dipole) or two dipoles share a position: those go by k_far_partial.
+// steps. Formed on the device from the cell map (or the run-time planned X passes'
+// row lists), one wave per row, and four launches and one wait in all: on the host
+// (a copy of the positions and two passes over them) the first call on an
+// operator of 33,552 dipoles took 470 us more than later ones, of 8.8 million
+// 61 ms, which is more than many calls take altogether.
+// ------------------------------------------------------------------------------------
+
+// Chunks for npos positions: 64 steps a wave, at most 64 work-groups' worth of waves.
+__host__ __device__ inline int far_chunks(int npos) {
+  const int per = 128 * kFarWaves, n = (npos + per - 1) / per;
+  return n < 64 ? n : 64;
+}
+
+// What the plan's kernels share. rows: [nocc] inner and outer fold of each
+// occupied row; first: [nocc + 1] its first position and segment; info: positions
+// (-1: too many holes), segments, and whether two dipoles share a position.
+struct FarMake {
+  const uint32_t *row_list, *cell, *row_start, *row_dip, *row_meta;
+  int nocc, Bx, By;
+  long long most;  // positions
+  int2 *rows, *first, *pair, *wave_seg;
+  FarSeg* segs;
+  int* info;
+};
+
+// x of the dipoles at +u (side 0) and -u of a row's centre; fold is the way back.
+__device__ inline int far_x(int Bx, int u, int side) { return side ? (Bx - 1) / 2 - u : Bx / 2 + u; }
+__device__ inline int far_fold(int Bx, int x) { return abs(2 * x - (Bx - 1)) / 2; }
+
+__global__ __launch_bounds__(256) void k_far_extent(FarMake m) {
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (i == 0 && lane < 3) m.info[lane] = 0;
+  if (i >= m.nocc) return;
+  const uint32_t row = m.row_list[i];
+  int lo = m.Bx, hi = -1;
+  if (m.cell) {
+    const uint32_t* c = m.cell + (size_t)row * m.Bx;
+    for (int x = lane; x < m.Bx; x += 64)
+      if ((int)c[x] >= 0) {
+        const int u = far_fold(m.Bx, x);
+        lo = min(lo, u);
+        hi = max(hi, u);
+      }
+  } else {
+    for (uint32_t k = m.row_start[row] + lane; k < m.row_start[row + 1]; k += 64) {
+      const int u = far_fold(m.Bx, m.row_meta[k] & 0xffff);
+      lo = min(lo, u);
+      hi = max(hi, u);
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o, 64));
+    hi = max(hi, __shfl_xor(hi, o, 64));
+  }
+  if (lane == 0) m.rows[i] = make_int2(lo, hi);
+}
+
+// One work-group: the rows' first positions (an even number each) and segments.
+__global__ __launch_bounds__(1024) void k_far_scan(FarMake m) {
+  __shared__ long long wp[16];
+  __shared__ int ws[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  long long pos0 = 0;
+  int seg0 = 0;
+  for (int i0 = 0; i0 < m.nocc; i0 += 1024) {
+    const int i = i0 + threadIdx.x;
+    int n = 0;
+    if (i < m.nocc) n = m.rows[i].y - m.rows[i].x + 1;
+    const int np = (n + 1) & ~1, ns = (n + 63) / 64;
+    long long p = np;
+    int s = ns;
+    for (int o = 1; o < 64; o <<= 1) {
+      const long long pp = __shfl_up(p, o, 64);
+      const int ss = __shfl_up(s, o, 64);
+      if (lane >= o) {
+        p += pp;
+        s += ss;
+      }
+    }
+    if (lane == 63) {
+      wp[wave] = p;
+      ws[wave] = s;
+    }
+    __syncthreads();
+    long long pb = pos0;
+    int sb = seg0;
+    for (int w = 0; w < 16; w++) {
+      if (w < wave) {
+        pb += wp[w];
+        sb += ws[w];
+      }
+      pos0 += wp[w];
+      seg0 += ws[w];
+    }
+    if (i < m.nocc) m.first[i] = make_int2((int)(pb + p - np), sb + s - ns);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    m.first[m.nocc] = make_int2((int)pos0, seg0);
+    m.info[0] = pos0 > m.most ? -1 : (int)pos0;
+    m.info[1] = seg0;
+  }
+}
+
+// Segments and pairs of each row; the last work-group: where each wave starts,
+// the first segment that ends at or after its share of the steps.
+__global__ __launch_bounds__(256) void k_far_fill(FarMake m) {
+  const int npos = m.info[0];
+  if (npos < 0) return;
+  if (blockIdx.x == gridDim.x - 1) {
+    const long long steps = npos / 2;
+    const int nw = far_chunks(npos) * kFarWaves;
+    for (int w = threadIdx.x; w <= nw; w += 256) {
+      const long long t = steps * w / nw;
+      // the row i in which step t lies: it starts before t (row 0: t = 0)
+      int a = 0, b = m.nocc;
+      while (b - a > 1) {
+        const int c = (a + b) / 2;
+        (m.first[c].x / 2 < t ? a : b) = c;
+      }
+      const int2 f = m.first[a], e = m.first[a + 1];
+      const int j = (int)((t - f.x / 2 + 31) / 32);
+      m.wave_seg[w] = make_int2(f.y + j, min(f.x + 64 * j, e.x));
+    }
+    return;
+  }
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (i >= m.nocc) return;
+  const uint32_t row = m.row_list[i];
+  const int lo = m.rows[i].x, hi = m.rows[i].y;
+  const int2 f = m.first[i], e = m.first[i + 1];
+  for (int q = f.y + lane; q < e.y; q += 64) {
+    const int u = lo + 64 * (q - f.y);
+    m.segs[q] = {u, min(32, (hi - u + 2) / 2), (int)(row % m.By), (int)(row / m.By)};
+  }
+  if (m.cell) {
+    const uint32_t* c = m.cell + (size_t)row * m.Bx;
+    for (int p = lane; p < e.x - f.x; p += 64) {
+      const int u = lo + p, xa = far_x(m.Bx, u, 0), xb = far_x(m.Bx, u, 1);
+      m.pair[f.x + p] = make_int2(u <= hi && xa < m.Bx ? (int)c[xa] : -1, u <= hi && xb >= 0 && xb != xa ? (int)c[xb] : -1);
+    }
+    return;
+  }
+  for (int p = lane; p < e.x - f.x; p += 64) m.pair[f.x + p] = make_int2(-1, -1);
+  __threadfence();  // before the row's own dipoles, which other lanes of the wave write
+  for (uint32_t k = m.row_start[row] + lane; k < m.row_start[row + 1]; k += 64) {
+    const int x = m.row_meta[k] & 0xffff, u = far_fold(m.Bx, x);
+    int2* q = &m.pair[f.x + u - lo];
+    if (atomicExch(x == far_x(m.Bx, u, 0) ? &q->x : &q->y, (int)m.row_dip[k]) >= 0) m.info[2] = 1;
+  }
+}
+
+// far.npos stays 0 where the rows are mostly holes (four positions and more per
+// dipole) or two dipoles share a position: those go by k_far_partial.
 dda_status far_segments(dda_op_s* op) {
   dda_op_s::Far& far = op->far;
   if (far.made) return DDA_OK;
-  DDA_TRY(host_positions(op));
   const MvDims& d = op->dims;
-  const int nrows = d.nrows, c2 = d.Bx - 1;  // twice the centre
-  auto fold = [&](int x) { return std::abs(2 * x - c2) / 2; };
-  std::vector<int> lo(nrows, d.Bx), hi(nrows, -1), first(nrows);
-  for (int i = 0; i < d.nv; i++) {
-    const uint32_t* p = &op->pos[3 * (size_t)i];
-    const int r = p[2] * d.By + p[1], u = fold(p[0]);
-    lo[r] = std::min(lo[r], u);
-    hi[r] = std::max(hi[r], u);
-  }
-  std::vector<FarSeg> segs;
-  long long npos = 0;
-  for (int r = 0; r < nrows; r++) {
-    first[r] = (int)std::min<long long>(npos, INT32_MAX);
-    for (int u = lo[r]; u <= hi[r]; u += 64) {
-      FarSeg sg = {u, std::min(32, (hi[r] - u + 2) / 2), r % d.By, r / d.By};
-      segs.push_back(sg);
-      npos += 2 * sg.steps;
-    }
+  hipStream_t st = op->ctx->stream;
+  const int nocc = op->n_nonempty, half = (d.Bx + 1) / 2;
+  FarMake m;
+  m.row_list = op->row_list;
+  m.cell = op->cell;
+  m.row_start = op->row_start;
+  m.row_dip = op->row_dip;
+  m.row_meta = op->row_meta;
+  m.nocc = nocc;
+  m.Bx = d.Bx;
+  m.By = d.By;
+  m.most = std::min<long long>(4ll * d.nv + 64, 1 << 26);
+  const size_t npos = std::min<long long>(m.most, (long long)nocc * (half + 1));
+  const size_t bytes[6] = {npos * sizeof(int2),
+                           (size_t)nocc * ((half + 63) / 64) * sizeof(FarSeg),
+                           (far_chunks((int)npos) * kFarWaves + 1ull) * sizeof(int2),
+                           nocc * sizeof(int2), (nocc + 1ull) * sizeof(int2), 3 * sizeof(int)};
+  size_t off[7] = {0};
+  for (int i = 0; i < 6; i++) off[i + 1] = off[i] + (bytes[i] + 127) / 128 * 128;
+  DDA_TRY_HIP(ctx_alloc(op->ctx, &op->far_dev, off[6], &op->far_bytes));
+  op->device_bytes += op->far_bytes;
+  char* dev = (char*)op->far_dev;
+  m.pair = (int2*)dev;
+  m.segs = (FarSeg*)(dev + off[1]);
+  m.wave_seg = (int2*)(dev + off[2]);
+  m.rows = (int2*)(dev + off[3]);
+  m.first = (int2*)(dev + off[4]);
+  m.info = (int*)(dev + off[5]);
+  const int nb = (nocc + 3) / 4;
+  hipLaunchKernelGGL(k_far_extent, dim3(nb), dim3(256), 0, st, m);
+  hipLaunchKernelGGL(k_far_scan, dim3(1), dim3(1024), 0, st, m);
+  hipLaunchKernelGGL(k_far_fill, dim3(nb + 1), dim3(256), 0, st, m);
+  int info[3] = {-1, 0, 0};
+  hipError_t le = hipGetLastError();
+  if (le == hipSuccess) le = hipMemcpyAsync(info, m.info, sizeof info, hipMemcpyDeviceToHost, st);
+  const hipError_t se = hipStreamSynchronize(st);
+  if (le == hipSuccess) le = se;
+  if (le != hipSuccess || info[0] <= 0 || info[2]) {
+    ctx_free(op->ctx, op->far_dev, op->far_bytes);
+    op->device_bytes -= op->far_bytes;
+    op->far_dev = nullptr;
+    far.made = le == hipSuccess;
+    DDA_TRY_HIP(le);
+    return DDA_OK;
   }
   far.made = true;
-  if (npos > 4ll * d.nv + 64 || npos > (1 << 26)) return DDA_OK;
-  std::vector<int2> pair(npos, make_int2(-1, -1));
-  for (int i = 0; i < d.nv; i++) {
-    const uint32_t* p = &op->pos[3 * (size_t)i];
-    const int r = p[2] * d.By + p[1], x = p[0];
-    int2& q = pair[first[r] + fold(x) - lo[r]];
-    int& at = 2 * x >= c2 ? q.x : q.y;
-    if (at >= 0) return DDA_OK;
-    at = i;
-  }
-  const long long steps = npos / 2;
-  // 64 steps a wave, at most 64 work-groups' worth of waves
-  far.nchunk = (int)std::min<long long>(64, (steps + 64 * kFarWaves - 1) / (64 * kFarWaves));
-  const int nw = far.nchunk * kFarWaves;
-  std::vector<int2> ws(nw + 1);
-  long long at = 0;
-  size_t q = 0;
-  for (int w = 0; w <= nw; w++) {
-    while (q < segs.size() && at < steps * w / nw) at += segs[q++].steps;
-    ws[w] = make_int2((int)q, (int)(2 * at));
-  }
-  // (records are read three steps ahead, from one position buffer per batch)
-  const size_t pb = (pair.size() * sizeof(int2) + 15) / 16 * 16, sb = segs.size() * sizeof(FarSeg);
-  const size_t wb = ws.size() * sizeof(int2);
-  DDA_TRY_HIP(hipMalloc(&op->far_dev, pb + sb + wb));
-  op->device_bytes += pb + sb + wb;
-  char* dev = (char*)op->far_dev;
-  hipStream_t st = op->ctx->stream;
-  DDA_TRY_HIP(hipMemcpyAsync(dev, pair.data(), pair.size() * sizeof(int2), hipMemcpyHostToDevice, st));
-  DDA_TRY_HIP(hipMemcpyAsync(dev + pb, segs.data(), sb, hipMemcpyHostToDevice, st));
-  DDA_TRY_HIP(hipMemcpyAsync(dev + pb + sb, ws.data(), wb, hipMemcpyHostToDevice, st));
-  DDA_TRY_HIP(hipStreamSynchronize(st));
-  far.segs = dev + pb;
-  far.wave_seg = dev + pb + sb;
-  far.npos = (int)npos;
+  far.segs = m.segs;
+  far.wave_seg = m.wave_seg;
+  far.nchunk = far_chunks(info[0]);
+  far.npos = info[0];
   return DDA_OK;
 }
 
@@ -635,20 +784,111 @@ dda_status far_batches(dda_op_s* op, const double2* pol, const FarDirs& f, const
   return DDA_OK;
 }
 
-// Whether nq field evaluations, of `slots` 64-padded slots, go by k_far_rows. Its
-// launches and tables cost what some hundred evaluations by k_far_partial do: the
-// two meet at 64 evaluations of 217,160 dipoles (113 against 118 us), 128 of
-// 94,296 (92 and 93), about 200 of 33,552 (81) and 4,096 of 280 (77 and 78), so
-// the line lies at 8 million dipole phases. A work-group's 64 directions take the
-// time of ten by k_far_partial, however many of them are in use. (4,096 of
-// 217,160 dipoles: 582 against 3,434 us.) An angle grid's directions and Jones
-// matrices are formed on the device too, which pays from 1,000 evaluations on at
-// any size (11,102 of 280 dipoles: 70 against 434 us).
-dda_status many_directions(dda_op_s* op, bool angle_grid, long long nq, long long slots, bool* many) {
-  *many = ((double)nq * op->dims.nv >= 8e6 || (angle_grid && nq >= 1000)) && 6 * nq >= slots && slots < (1ll << 30);
-  if (!*many) return DDA_OK;
+// Whether nq field evaluations of `used` right-hand sides go by k_far_rows. Its
+// launches and tables cost what some hundred evaluations by k_far_partial do, the
+// records of a right-hand side and 64 directions what 38 do in large particles.
+// The two, on an operator that has made the segments and on a new one (whose first
+// call of k_far_partial is that much longer too), in us:
+//   33,552 dipoles, 256 evaluations        83 and 121   against  90 and  97
+//   217,160 dipoles, 48                   116 and 160   against 116 and 121
+//   1,099,136 dipoles, 16, 48 and 64      311, 310 and 312   against 198, 339 and 407
+//   8,783,848 dipoles, 32, 48 and 256     2,783, 2,789 and 2,598   against 2,411, 3,160
+//                                         and 11,907; new, 256: 3,015 against 12,876
+// so the line lies at 8 million dipole phases and 48 evaluations of each
+// right-hand side. An angle grid's directions and Jones matrices are formed on the
+// device too, which pays from 1,000 evaluations on at any size (11,102 of 280
+// dipoles: 72 against 426 us). k_far_partial's grid has no room for more than
+// kFarDirect.
+constexpr int kFarDirect = 4 * 65535;
+bool many_directions(const dda_op_s* op, bool angle_grid, long long nq, int used) {
+  return nq > kFarDirect || (angle_grid && nq >= 1000) ||
+         ((double)nq * op->dims.nv >= 8e6 && nq >= 48ll * used);
+}
+
+// dda_far_field of many directions; DDA_NOT_SUPPORTED where k_far_partial takes them.
+dda_status far_field_many(dda_op_s* op, const double2* pol, int nrhs, const int* rhs, const double* dirs, int nq,
+                          double* out) {
+  // slots by right-hand side, each's filled up to 64
+  std::vector<int> fill(nrhs + 1, 0);
+  for (int i = 0; i < nq; i++) fill[(rhs ? rhs[i] : 0) + 1]++;
+  long long slots = 0;
+  int used = 0;
+  for (int r = 0; r < nrhs; r++) {
+    const int n = fill[r + 1];
+    fill[r] = (int)slots;
+    slots += (n + 63) / 64 * 64;
+    used += n > 0;
+  }
+  if (!many_directions(op, false, nq, used) || slots >= (1ll << 30)) return DDA_NOT_SUPPORTED;
   DDA_TRY(far_segments(op));
-  *many = op->far.npos > 0;
+  if (op->far.npos == 0) return DDA_NOT_SUPPORTED;
+  const FarPlan plan = far_plan(op, (int)slots, 1, nrhs);
+  const size_t dbytes = 3ull * slots * sizeof(double), ibytes = (slots + slots / 64 + 3) / 4 * 16;
+  void* buf = nullptr;
+  DDA_TRY(obs_scratch(op, plan.bytes + dbytes + ibytes + 6ull * nq * sizeof(double), &buf));
+  std::vector<double> hd(3 * slots, 0.0);
+  std::vector<int> hi(slots + slots / 64, -1);
+  for (int i = 0; i < nq; i++) {
+    const int r = rhs ? rhs[i] : 0, s = fill[r]++;
+    for (int a = 0; a < 3; a++) hd[dir_index(s, a)] = dirs[dir_index(i, a)];
+    hi[s] = i;
+    hi[slots + s / 64] = r;
+  }
+  for (long long t = 0; t < slots / 64; t++) hi[slots + t] = std::max(0, hi[slots + t]);
+  double* dd = (double*)((char*)buf + plan.bytes);
+  int* id = (int*)((char*)dd + dbytes);
+  double* od = (double*)((char*)id + ibytes);
+  hipStream_t st = op->ctx->stream;
+  DDA_TRY_HIP(hipMemcpyAsync(dd, hd.data(), dbytes, hipMemcpyHostToDevice, st));
+  DDA_TRY_HIP(hipMemcpyAsync(id, hi.data(), hi.size() * sizeof(int), hipMemcpyHostToDevice, st));
+  FarDirs f;
+  std::memset(&f, 0, sizeof f);
+  f.dirs = dd;
+  f.count = (int)slots;
+  DDA_TRY(far_batches<1>(op, pol, f, plan, hi.data() + slots, id + slots, id, od, buf));
+  DDA_TRY_HIP(hipMemcpyAsync(out, od, 6ull * nq * sizeof(double), hipMemcpyDeviceToHost, st));
+  DDA_TRY_HIP(hipStreamSynchronize(st));
+  return DDA_OK;
+}
+
+// dda_jones of many angles; DDA_NOT_SUPPORTED where dda_far_field takes them.
+dda_status jones_many(dda_op_s* op, const double2* pol, int symmetric, const double prop[3], const double pol1[3],
+                      const double pol2[3], uint32_t ntheta, double theta0, double dtheta, uint32_t nphi, double phi0,
+                      double dphi, double* out) {
+  const size_t count = (size_t)ntheta * nphi, slots = symmetric ? 2 * count : count;
+  if (!many_directions(op, true, 2 * (long long)count, 1) || slots >= (1ll << 30)) return DDA_NOT_SUPPORTED;
+  DDA_TRY(far_segments(op));
+  if (op->far.npos == 0) return DDA_NOT_SUPPORTED;
+  const FarPlan plan = far_plan(op, (int)slots, symmetric ? 1 : 2, 1);
+  const size_t tbytes = 2 * ((size_t)ntheta + nphi) * sizeof(double);
+  void* buf = nullptr;
+  DDA_TRY(obs_scratch(op, plan.bytes + tbytes + 8 * count * sizeof(double), &buf));
+  std::vector<double> trig(2 * ((size_t)ntheta + nphi));
+  for (size_t i = 0; i < (size_t)ntheta + nphi; i++) {
+    const double a = i < ntheta ? theta0 + (double)i * dtheta : phi0 + (double)(i - ntheta) * dphi;
+    trig[2 * i] = std::sin(a);
+    trig[2 * i + 1] = std::cos(a);
+  }
+  double* td = (double*)((char*)buf + plan.bytes);
+  double* od = (double*)((char*)td + tbytes);
+  hipStream_t st = op->ctx->stream;
+  DDA_TRY_HIP(hipMemcpyAsync(td, trig.data(), tbytes, hipMemcpyHostToDevice, st));
+  FarDirs f;
+  std::memset(&f, 0, sizeof f);
+  f.g.trig = td;
+  f.g.ntheta = (int)ntheta;
+  f.g.nphi = (int)nphi;
+  f.g.symmetric = symmetric;
+  for (int a = 0; a < 3; a++) {
+    f.g.prop[a] = prop[a];
+    f.g.pol1[a] = pol1[a];
+    f.g.pol2[a] = pol2[a];
+  }
+  f.count = (int)slots;
+  DDA_TRY(symmetric ? far_batches<1>(op, pol, f, plan, nullptr, nullptr, nullptr, od, buf)
+                    : far_batches<2>(op, pol, f, plan, nullptr, nullptr, nullptr, od, buf));
+  DDA_TRY_HIP(hipMemcpyAsync(out, od, 8 * count * sizeof(double), hipMemcpyDeviceToHost, st));
+  DDA_TRY_HIP(hipStreamSynchronize(st));
   return DDA_OK;
 }
 
@@ -886,47 +1126,9 @@ extern "C" dda_status dda_far_field(dda_op_t op, const void* pol_dev, int nrhs, 
       set_error("dda_far_field: right-hand side index out of range");
       return DDA_INVALID_ARG;
     }
-  {
-    // many directions: slots by right-hand side, each's filled up to 64
-    std::vector<int> fill(nrhs + 1, 0);
-    for (int i = 0; i < nq; i++) fill[(rhs ? rhs[i] : 0) + 1]++;
-    long long slots = 0;
-    for (int r = 0; r < nrhs; r++) {
-      const int n = fill[r + 1];
-      fill[r] = (int)slots;
-      slots += (n + 63) / 64 * 64;
-    }
-    bool many = false;
-    DDA_TRY(many_directions(op, false, nq, slots, &many));
-    if (many) {
-      std::vector<double> hd(3 * slots, 0.0);
-      std::vector<int> hi(slots + slots / 64, -1);
-      for (int i = 0; i < nq; i++) {
-        const int r = rhs ? rhs[i] : 0, s = fill[r]++;
-        for (int a = 0; a < 3; a++) hd[dir_index(s, a)] = dirs[dir_index(i, a)];
-        hi[s] = i;
-        hi[slots + s / 64] = r;
-      }
-      for (long long t = 0; t < slots / 64; t++) hi[slots + t] = std::max(0, hi[slots + t]);
-      const FarPlan plan = far_plan(op, (int)slots, 1, nrhs);
-      const size_t dbytes = hd.size() * sizeof(double), ibytes = (hi.size() + 3) / 4 * 16;
-      void* buf = nullptr;
-      DDA_TRY(obs_scratch(op, plan.bytes + dbytes + ibytes + 6ull * nq * sizeof(double), &buf));
-      double* dd = (double*)((char*)buf + plan.bytes);
-      int* id = (int*)((char*)dd + dbytes);
-      double* od = (double*)((char*)id + ibytes);
-      hipStream_t st = op->ctx->stream;
-      DDA_TRY_HIP(hipMemcpyAsync(dd, hd.data(), dbytes, hipMemcpyHostToDevice, st));
-      DDA_TRY_HIP(hipMemcpyAsync(id, hi.data(), hi.size() * sizeof(int), hipMemcpyHostToDevice, st));
-      FarDirs f;
-      std::memset(&f, 0, sizeof f);
-      f.dirs = dd;
-      f.count = (int)slots;
-      DDA_TRY(far_batches<1>(op, (const double2*)pol_dev, f, plan, hi.data() + slots, id + slots, id, od, buf));
-      DDA_TRY_HIP(hipMemcpyAsync(out, od, 6ull * nq * sizeof(double), hipMemcpyDeviceToHost, st));
-      DDA_TRY_HIP(hipStreamSynchronize(st));
-      return DDA_OK;
-    }
+  if (many_directions(op, false, nq, 1)) {
+    const dda_status rc = far_field_many(op, (const double2*)pol_dev, nrhs, rhs, dirs, nq, out);
+    if (rc != DDA_NOT_SUPPORTED) return rc;
   }
   DDA_TRY(positions_on_device(op));
   const MvDims& d = op->dims;
@@ -966,43 +1168,11 @@ extern "C" dda_status dda_jones(dda_op_t op, const void* pol_dev, int symmetric,
   }
   DDA_TRY(one_wave_number(op, "dda_jones"));
   const size_t count = (size_t)ntheta * nphi;
-  const size_t slots = symmetric ? 2 * count : count;
   DDA_TRY(bind_device(op->ctx));
-  bool many = false;
-  DDA_TRY(many_directions(op, true, 2 * (long long)count, (long long)slots, &many));
-  if (many) {
-    std::vector<double> trig(2 * ((size_t)ntheta + nphi));
-    for (size_t i = 0; i < (size_t)ntheta + nphi; i++) {
-      const double a = i < ntheta ? theta0 + (double)i * dtheta : phi0 + (double)(i - ntheta) * dphi;
-      trig[2 * i] = std::sin(a);
-      trig[2 * i + 1] = std::cos(a);
-    }
-    const FarPlan plan = far_plan(op, (int)slots, symmetric ? 1 : 2, 1);
-    const size_t tbytes = trig.size() * sizeof(double);
-    void* buf = nullptr;
-    DDA_TRY(obs_scratch(op, plan.bytes + tbytes + 8 * count * sizeof(double), &buf));
-    double* td = (double*)((char*)buf + plan.bytes);
-    double* od = (double*)((char*)td + tbytes);
-    hipStream_t st = op->ctx->stream;
-    DDA_TRY_HIP(hipMemcpyAsync(td, trig.data(), tbytes, hipMemcpyHostToDevice, st));
-    FarDirs f;
-    std::memset(&f, 0, sizeof f);
-    f.g.trig = td;
-    f.g.ntheta = (int)ntheta;
-    f.g.nphi = (int)nphi;
-    f.g.symmetric = symmetric;
-    for (int a = 0; a < 3; a++) {
-      f.g.prop[a] = prop[a];
-      f.g.pol1[a] = pol1[a];
-      f.g.pol2[a] = pol2[a];
-    }
-    f.count = (int)slots;
-    const double2* pol = (const double2*)pol_dev;
-    DDA_TRY(symmetric ? far_batches<1>(op, pol, f, plan, nullptr, nullptr, nullptr, od, buf)
-                      : far_batches<2>(op, pol, f, plan, nullptr, nullptr, nullptr, od, buf));
-    DDA_TRY_HIP(hipMemcpyAsync(out, od, 8 * count * sizeof(double), hipMemcpyDeviceToHost, st));
-    DDA_TRY_HIP(hipStreamSynchronize(st));
-    return DDA_OK;
+  {
+    const dda_status rc = jones_many(op, (const double2*)pol_dev, symmetric, prop, pol1, pol2, ntheta, theta0, dtheta,
+                                     nphi, phi0, dphi, out);
+    if (rc != DDA_NOT_SUPPORTED) return rc;
   }
   // two field evaluations per angle: (p1; X = pol2, Y = pol1) and
   // (p2; X = pol2, Y = pol1) or, for a symmetric target, (p1; X = pol1, Y = -pol2)
