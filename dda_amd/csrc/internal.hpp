@@ -229,6 +229,7 @@ struct dda_op_s {
     bool made = false;
     int npos = 0, nchunk = 0;
     const void *segs = nullptr, *wave_seg = nullptr;
+    std::vector<int2> start;  // copy of wave_seg where the records are made in groups
   } far;
   void* far_dev = nullptr;      // used on the context's stream alone
   size_t far_bytes = 0;

@@ -316,9 +316,10 @@ typedef double far4 __attribute__((ext_vector_type(4)));
 // wave_seg[w] .. wave_seg[w + 1], w = 8 b + wave; their records are a stream,
 // read three steps ahead. Four tiles of 16 directions share each record; their
 // cos and sin come from LDS (LDSX) or, for boxes too long for it, from L2.
-// Records: those of right-hand side rhs[tile] - r0, or (rhs null) of the only one.
+// Records: those of positions pos0 .. pos0 + npos - 1 (where the launch's chunks
+// lie) of right-hand side rhs[tile] - r0, or (rhs null) of the only one.
 template <int NR, bool LDSX>
-__global__ __launch_bounds__(64 * kFarWaves) void k_far_rows(const double* __restrict__ rec, int npos,
+__global__ __launch_bounds__(64 * kFarWaves) void k_far_rows(const double* __restrict__ rec, int pos0, int npos,
                                                              const FarSeg* __restrict__ segs,
                                                              const int2* __restrict__ wave_seg,
                                                              const double* __restrict__ cs,
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(64 * kFarWaves) void k_far_rows(const double* __res
   ct += (g >> 1) * 128 + (g & 1) * 16 + j;
   if (rhs) rec += (long long)(rhs[blockIdx.x] - r0) * npos * 32;
   const int2 ws = wave_seg[blockIdx.y * kFarWaves + wave], we = wave_seg[blockIdx.y * kFarWaves + wave + 1];
-  const double* r = rec + (long long)ws.y * 32 + lane;
+  const double* r = rec + (long long)(ws.y - pos0) * 32 + lane;
   double acc_r[4][NR], acc_i[4][NR];
 #pragma unroll
   for (int t = 0; t < 4; t++)
@@ -510,10 +511,15 @@ dda_status obs_scratch(dda_op_s* op, size_t bytes, void** out) {
 // 61 ms, which is more than many calls take altogether.
 // ------------------------------------------------------------------------------------
 
-// Chunks for npos positions: 64 steps a wave, at most 64 work-groups' worth of waves.
+// Positions of which the records of one right-hand side take 256 MB.
+constexpr int kFarGroup = 1 << 20;
+
+// Chunks for npos positions: 64 steps a wave, at most 64 work-groups' worth of
+// waves in each group of positions.
+__host__ __device__ inline int far_groups(int npos) { return (npos + kFarGroup - 1) / kFarGroup; }
 __host__ __device__ inline int far_chunks(int npos) {
-  const int per = 128 * kFarWaves, n = (npos + per - 1) / per;
-  return n < 64 ? n : 64;
+  const int per = 128 * kFarWaves, n = (npos + per - 1) / per, g = far_groups(npos);
+  return g > 1 ? 64 * g : n < 64 ? n : 64;
 }
 
 // What the plan's kernels share. rows: [nocc] inner and outer fold of each
@@ -656,7 +662,8 @@ __global__ __launch_bounds__(256) void k_far_fill(FarMake m) {
 }
 
 // far.npos stays 0 where the rows are mostly holes (four positions and more per
-// dipole) or two dipoles share a position: those go by k_far_partial.
+// dipole), two dipoles share a position or the memory cannot be had: those go by
+// k_far_partial.
 dda_status far_segments(dda_op_s* op) {
   dda_op_s::Far& far = op->far;
   if (far.made) return DDA_OK;
@@ -680,7 +687,12 @@ dda_status far_segments(dda_op_s* op) {
                            nocc * sizeof(int2), (nocc + 1ull) * sizeof(int2), 3 * sizeof(int)};
   size_t off[7] = {0};
   for (int i = 0; i < 6; i++) off[i + 1] = off[i] + (bytes[i] + 127) / 128 * 128;
-  DDA_TRY_HIP(ctx_alloc(op->ctx, &op->far_dev, off[6], &op->far_bytes));
+  const hipError_t e = ctx_alloc(op->ctx, &op->far_dev, off[6], &op->far_bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return DDA_OK;
+  }
+  DDA_TRY_HIP(e);
   op->device_bytes += op->far_bytes;
   char* dev = (char*)op->far_dev;
   m.pair = (int2*)dev;
@@ -698,6 +710,11 @@ dda_status far_segments(dda_op_s* op) {
   if (le == hipSuccess) le = hipMemcpyAsync(info, m.info, sizeof info, hipMemcpyDeviceToHost, st);
   const hipError_t se = hipStreamSynchronize(st);
   if (le == hipSuccess) le = se;
+  if (le == hipSuccess && info[0] > 0 && !info[2] && far_groups(info[0]) > 1) {
+    far.start.resize(far_chunks(info[0]) * kFarWaves + 1);
+    le = hipMemcpyAsync(far.start.data(), m.wave_seg, far.start.size() * sizeof(int2), hipMemcpyDeviceToHost, st);
+    if (le == hipSuccess) le = hipStreamSynchronize(st);
+  }
   if (le != hipSuccess || info[0] <= 0 || info[2]) {
     ctx_free(op->ctx, op->far_dev, op->far_bytes);
     op->device_bytes -= op->far_bytes;
@@ -715,22 +732,32 @@ dda_status far_segments(dda_op_s* op) {
 }
 
 // Work space of far_batches: the batches' tables, partial sums and records,
-// each batch's tables and sums and its records below 256 MB where they can be.
+// each batch's tables and sums and its records below 256 MB. The records of more
+// than kFarGroup positions are made and used group by group.
 struct FarPlan {
   int nu;         // positions of the folded x axis, one more for the step's second
   int per_batch;  // slots per batch, a multiple of 64
+  int groups;     // of positions
   int recs;       // right-hand sides (NR = 2: pairs) per batch
   size_t cs, yz, parts, bytes;
 };
+// First position of a group's records, and the end of the last's.
+int group_start(const dda_op_s::Far& far, int groups, int g) {
+  return groups == 1 ? g * far.npos : far.start[(size_t)g * (far.nchunk / groups) * kFarWaves].y;
+}
 FarPlan far_plan(const dda_op_s* op, int slots, int nr, int nrec) {
   const MvDims& d = op->dims;
   const size_t most = 256ull << 20;
   FarPlan p;
   p.nu = (d.Bx + 1) / 2 + 1;
   const size_t cs = 16ull * p.nu, yz = 16ull * (d.By + d.Bz), part = 48ull * nr * op->far.nchunk;
-  const size_t rec = 256ull * op->far.npos;
+  p.groups = far_groups(op->far.npos);
+  int npos = 0;
+  for (int g = 0; g < p.groups; g++)
+    npos = std::max(npos, group_start(op->far, p.groups, g + 1) - group_start(op->far, p.groups, g));
+  const size_t rec = 256ull * npos;
   p.per_batch = (int)std::min<size_t>(std::max<size_t>(1, most / (64 * (cs + yz + part))), (slots + 63) / 64) * 64;
-  p.recs = (int)std::min<size_t>(std::max<size_t>(1, most / rec), std::min(nrec, 65535));
+  p.recs = p.groups > 1 ? 1 : (int)std::min<size_t>(std::max<size_t>(1, most / rec), std::min(nrec, 65535));
   p.cs = cs * p.per_batch;
   p.yz = yz * p.per_batch;
   p.parts = part * p.per_batch;
@@ -765,18 +792,23 @@ dda_status far_batches(dda_op_s* op, const double2* pol, const FarDirs& f, const
     const int r0 = rhs_host ? rhs_host[t0] : 0;
     for (t1 = t0; t1 < tiles && (t1 - t0) * 64 < p.per_batch && (rhs_host ? rhs_host[t1] : 0) < r0 + p.recs;) t1++;
     const int r1 = (rhs_host ? rhs_host[t1 - 1] : 0) + 1;
-    if (r0 < have0 || r1 > have1) {
-      have0 = r0;
-      have1 = r1;
-      hipLaunchKernelGGL(k_far_pack<NR>, dim3(std::min(1024, (16 * far.npos + 255) / 256), r1 - r0), dim3(256), 0, st,
-                         pol + (size_t)r0 * 3 * NR * d.S, (const int2*)op->far_dev, far.npos, d.S, rec);
-    }
     const int s0 = t0 * 64, ns = (t1 - t0) * 64;
     hipLaunchKernelGGL(k_far_tables, dim3(t1 - t0, std::min(p.nu + d.By + d.Bz, 64)), dim3(64), 0, st, f, s0, ns, p.nu,
                        d.Bx & 1 ? 0.0 : 0.5, d.By, d.Bz, op->wave_num * op->grid_unit, cs, yz);
-    hipLaunchKernelGGL(k, dim3(t1 - t0, far.nchunk), dim3(64 * kFarWaves), lds, st, rec, far.npos,
-                       (const FarSeg*)far.segs, (const int2*)far.wave_seg, cs, yz, p.nu, d.By, ns,
-                       rhs ? rhs + t0 : nullptr, have0, part);
+    const int chunks = far.nchunk / p.groups;
+    for (int gr = 0; gr < p.groups; gr++) {
+      const int pos0 = group_start(far, p.groups, gr), np = group_start(far, p.groups, gr + 1) - pos0;
+      if (p.groups > 1 || r0 < have0 || r1 > have1) {
+        have0 = r0;
+        have1 = r1;
+        hipLaunchKernelGGL(k_far_pack<NR>, dim3(std::min(1024, (16 * np + 255) / 256), r1 - r0), dim3(256), 0, st,
+                           pol + (size_t)r0 * 3 * NR * d.S, (const int2*)op->far_dev + pos0, np, d.S, rec);
+      }
+      hipLaunchKernelGGL(k, dim3(t1 - t0, chunks), dim3(64 * kFarWaves), lds, st, rec, pos0, np,
+                         (const FarSeg*)far.segs, (const int2*)far.wave_seg + (size_t)gr * chunks * kFarWaves, cs, yz,
+                         p.nu, d.By, ns, rhs ? rhs + t0 : nullptr, have0,
+                         part + (size_t)gr * chunks * 6 * NR * ns);
+    }
     hipLaunchKernelGGL(k_far_last<NR>, dim3(t1 - t0), dim3(384 * NR), 0, st, part, f, s0, ns, far.nchunk, op->wave_num,
                        query, out_dev);
     DDA_TRY_HIP(hipGetLastError());
@@ -805,6 +837,15 @@ bool many_directions(const dda_op_s* op, bool angle_grid, long long nq, int used
          ((double)nq * op->dims.nv >= 8e6 && nq >= 48ll * used);
 }
 
+// Scratch for k_far_rows and what is beside it: DDA_NOT_SUPPORTED where it cannot
+// be had, and k_far_partial, which needs less, has to do.
+dda_status far_scratch(dda_op_s* op, size_t bytes, void** out) {
+  const dda_status rc = obs_scratch(op, bytes, out);
+  if (rc != DDA_OUT_OF_MEMORY) return rc;
+  (void)hipGetLastError();
+  return DDA_NOT_SUPPORTED;
+}
+
 // dda_far_field of many directions; DDA_NOT_SUPPORTED where k_far_partial takes them.
 dda_status far_field_many(dda_op_s* op, const double2* pol, int nrhs, const int* rhs, const double* dirs, int nq,
                           double* out) {
@@ -825,7 +866,7 @@ dda_status far_field_many(dda_op_s* op, const double2* pol, int nrhs, const int*
   const FarPlan plan = far_plan(op, (int)slots, 1, nrhs);
   const size_t dbytes = 3ull * slots * sizeof(double), ibytes = (slots + slots / 64 + 3) / 4 * 16;
   void* buf = nullptr;
-  DDA_TRY(obs_scratch(op, plan.bytes + dbytes + ibytes + 6ull * nq * sizeof(double), &buf));
+  DDA_TRY(far_scratch(op, plan.bytes + dbytes + ibytes + 6ull * nq * sizeof(double), &buf));
   std::vector<double> hd(3 * slots, 0.0);
   std::vector<int> hi(slots + slots / 64, -1);
   for (int i = 0; i < nq; i++) {
@@ -862,7 +903,7 @@ dda_status jones_many(dda_op_s* op, const double2* pol, int symmetric, const dou
   const FarPlan plan = far_plan(op, (int)slots, symmetric ? 1 : 2, 1);
   const size_t tbytes = 2 * ((size_t)ntheta + nphi) * sizeof(double);
   void* buf = nullptr;
-  DDA_TRY(obs_scratch(op, plan.bytes + tbytes + 8 * count * sizeof(double), &buf));
+  DDA_TRY(far_scratch(op, plan.bytes + tbytes + 8 * count * sizeof(double), &buf));
   std::vector<double> trig(2 * ((size_t)ntheta + nphi));
   for (size_t i = 0; i < (size_t)ntheta + nphi; i++) {
     const double a = i < ntheta ? theta0 + (double)i * dtheta : phi0 + (double)(i - ntheta) * dphi;

@@ -1,6 +1,8 @@
 """Far fields of many directions: the plan of the positions on an operator that
-runs the row lists, dipoles that share a position, and what the first call on a
-new operator costs. Each against a few directions at a time."""
+runs the row lists, positions beyond one group of records, dipoles that share a
+position, device memory that leaves no room for the records, and what the first
+call on a new operator costs. Each against a few directions at a time."""
+import ctypes
 import time
 
 import numpy as np
@@ -73,6 +75,37 @@ def test_shared_positions(ctx):
     assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
     op.close()
     pol.close()
+
+
+def _all_but(ctx, leave):
+    """A device allocation that leaves `leave` bytes of the GPU's memory."""
+    p, free, total = ctypes.c_void_p(), ctypes.c_size_t(), ctypes.c_size_t()
+    assert D.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    assert D.lib().dda_malloc(ctx.handle, ctypes.c_size_t(free.value - leave), ctypes.byref(p)) == D.OK
+    return p
+
+
+def test_groups_of_positions_and_no_room_for_records(ctx):
+    """2.9 million dipoles, 1.5 million folded positions: two groups of records.
+    Then the same call with 150 MB of device memory left, which its records do
+    not fit: accepted all the same."""
+    own = D.Context(0)  # without spare buffers of other tests
+    box = (160, 136, 134)
+    pos = _box(box)
+    op = _operator(own, pos, box)
+    pol = _random_pol(own, op, 2, 4)
+    dirs = _dirs(200)
+    rhs = np.arange(200) // 100
+    ref = _few(op, pol, 2, dirs, rhs)
+    fill = _all_but(own, 150 << 20)
+    try:
+        short = D.far_field(op, pol, 2, dirs, rhs)
+    finally:
+        D.lib().dda_free(own.handle, fill)
+    assert np.abs(short - ref).max() <= TOL * np.abs(ref).max()
+    got = D.far_field(op, pol, 2, dirs, rhs)
+    assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
+    own.close()
 
 
 def test_first_call_on_a_new_operator(ctx):
