@@ -1,4 +1,5 @@
 // Context, error reporting and plain memory helpers of the C ABI.
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -15,6 +16,10 @@ void set_error(const std::string& msg) { g_last_error = msg; }
 using namespace dda;
 
 extern "C" const char* dda_last_error(void) { return g_last_error.c_str(); }
+
+// The contexts alive, for dev_malloc (locked before a context's spare_mu).
+static std::mutex g_ctx_mu;
+static std::vector<dda_ctx_s*> g_ctx;
 
 extern "C" dda_status dda_ctx_create(int device, dda_ctx_t* out) {
   if (!out) {
@@ -44,6 +49,10 @@ extern "C" dda_status dda_ctx_create(int device, dda_ctx_t* out) {
     delete c;
     return rs;
   }
+  {
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    g_ctx.push_back(c);
+  }
   *out = c;
   return DDA_OK;
 }
@@ -52,31 +61,55 @@ extern "C" dda_status dda_ctx_create(int device, dda_ctx_t* out) {
 // and hipFree of a buffer of some ten megabytes takes 100 us and more (the three
 // of a 96 x 72 x 60 box 590 us, allocating them anew 100). Up to kSpareBytes of a
 // context's freed buffers wait for its next operators; work on its stream orders
-// old and new use.
+// old and new use. Any allocation of the library that finds the memory short gives
+// them back first, those of the other contexts on the device too.
 constexpr size_t kSpareBytes = 1ull << 30;
 
-hipError_t dda::ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, size_t* got) {
+static bool free_spares(dda_ctx_s* c) {
   std::lock_guard<std::mutex> lk(c->spare_mu);
-  auto best = c->spare.end();
-  for (auto it = c->spare.begin(); it != c->spare.end(); ++it)
-    if (it->bytes >= bytes && it->bytes <= bytes + bytes / 2 && (best == c->spare.end() || it->bytes < best->bytes))
-      best = it;
-  if (best != c->spare.end()) {
-    *p = best->ptr;
-    *got = best->bytes;
-    c->spare.erase(best);
-    return hipSuccess;
-  }
+  for (auto& s : c->spare) (void)hipFree(s.ptr);
+  const bool any = !c->spare.empty();
+  c->spare.clear();
+  return any;
+}
+
+hipError_t dda::dev_malloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
-  if (e == hipErrorOutOfMemory && !c->spare.empty()) {
+  if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
-    for (auto& s : c->spare) (void)hipFree(s.ptr);
-    c->spare.clear();
-    e = hipMalloc(p, bytes);
+    int device = -1;
+    (void)hipGetDevice(&device);
+    bool any = false;
+    {
+      std::lock_guard<std::mutex> lk(g_ctx_mu);
+      for (dda_ctx_s* c : g_ctx)
+        if (c->device == device) any = free_spares(c) || any;
+    }
+    if (any) e = hipMalloc(p, bytes);
   }
-  if (e != hipSuccess) *p = nullptr;
-  *got = bytes;
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // (the next launch's check is not to find it)
+    *p = nullptr;
+  }
   return e;
+}
+
+hipError_t dda::ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, size_t* got) {
+  {
+    std::lock_guard<std::mutex> lk(c->spare_mu);
+    auto best = c->spare.end();
+    for (auto it = c->spare.begin(); it != c->spare.end(); ++it)
+      if (it->bytes >= bytes && it->bytes <= bytes + bytes / 2 && (best == c->spare.end() || it->bytes < best->bytes))
+        best = it;
+    if (best != c->spare.end()) {
+      *p = best->ptr;
+      *got = best->bytes;
+      c->spare.erase(best);
+      return hipSuccess;
+    }
+  }
+  *got = bytes;
+  return dev_malloc(p, bytes);
 }
 
 void dda::ctx_free(dda_ctx_s* c, void* p, size_t bytes) {
@@ -97,8 +130,12 @@ void dda::ctx_free(dda_ctx_s* c, void* p, size_t bytes) {
 
 extern "C" dda_status dda_ctx_destroy(dda_ctx_t ctx) {
   if (!ctx) return DDA_OK;
+  {
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    g_ctx.erase(std::find(g_ctx.begin(), g_ctx.end(), ctx));
+  }
   (void)hipStreamSynchronize(ctx->stream);
-  for (auto& s : ctx->spare) (void)hipFree(s.ptr);
+  free_spares(ctx);
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return DDA_OK;
@@ -134,7 +171,7 @@ extern "C" dda_status dda_malloc(dda_ctx_t ctx, size_t bytes, void** out) {
     return DDA_INVALID_ARG;
   }
   DDA_TRY_HIP(hipSetDevice(ctx->device));
-  DDA_TRY_HIP(hipMalloc(out, bytes ? bytes : 1));
+  DDA_TRY_HIP(dev_malloc(out, bytes ? bytes : 1));
   return DDA_OK;
 }
 

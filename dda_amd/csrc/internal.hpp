@@ -140,10 +140,19 @@ inline dda_status bind_device(const dda_ctx_s* c) {
   return DDA_OK;
 }
 
+// hipMalloc on the current device; where memory is short, the spare buffers of the
+// contexts on it are freed first.
+hipError_t dev_malloc(void** p, size_t bytes);
+template <typename T> hipError_t dev_malloc(T** p, size_t bytes) {
+  void* v = nullptr;
+  const hipError_t e = dev_malloc(&v, bytes);
+  *p = (T*)v;
+  return e;
+}
+
 // Large device buffers of a context's operators: a spare one of the size, else
-// hipMalloc (after giving the spare ones back where memory is short). *got is the
-// buffer's size, which ctx_free takes. ctx_free's caller has waited for all work
-// on the buffer but that on the context's stream.
+// dev_malloc. *got is the buffer's size, which ctx_free takes. ctx_free's caller
+// has waited for all work on the buffer but that on the context's stream.
 hipError_t ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, size_t* got);
 void ctx_free(dda_ctx_s* c, void* p, size_t bytes);
 }  // namespace dda

@@ -1018,13 +1018,13 @@ struct Core {
     max_iter = mi;
     max_res_increase = mri;
     hist_cap = std::min<uint64_t>(mi + 1, 1u << 16);
-    DDA_TRY_HIP(hipMalloc(&dst, cap * sizeof(SolverState)));
+    DDA_TRY_HIP(dev_malloc(&dst, cap * sizeof(SolverState)));
     DDA_TRY_HIP(hipHostMalloc((void**)&host2, 2 * cap * sizeof(SolverState), hipHostMallocDefault));
-    DDA_TRY_HIP(hipMalloc(&part, (size_t)cap * 4 * nb * sizeof(double)));
+    DDA_TRY_HIP(dev_malloc(&part, (size_t)cap * 4 * nb * sizeof(double)));
     if (o->static_x)
-      DDA_TRY_HIP(hipMalloc(&part5, (size_t)cap * 4 * std::max(1, 3 * o->n_nonempty) * sizeof(double)));
-    DDA_TRY_HIP(hipMalloc(&hist, (size_t)cap * hist_cap * sizeof(double)));
-    for (int i = 0; i < 8; i++) DDA_TRY_HIP(hipMalloc(&v[i], (size_t)cap * n * sizeof(C)));
+      DDA_TRY_HIP(dev_malloc(&part5, (size_t)cap * 4 * std::max(1, 3 * o->n_nonempty) * sizeof(double)));
+    DDA_TRY_HIP(dev_malloc(&hist, (size_t)cap * hist_cap * sizeof(double)));
+    for (int i = 0; i < 8; i++) DDA_TRY_HIP(dev_malloc(&v[i], (size_t)cap * n * sizeof(C)));
     return DDA_OK;
   }
   void drop_graph() {
@@ -1395,17 +1395,17 @@ dda_status alloc_buffers(dda_solver_s* s, int k) {
   s->mask = nullptr;
   const int nb = red_blocks(s->n);
   const size_t vb = (size_t)k * s->n * sizeof(double2);
-  DDA_TRY_HIP(hipMalloc(&s->io, 2 * vb));
+  DDA_TRY_HIP(dev_malloc(&s->io, 2 * vb));
   if (s->mode != DDA_MODE_FP32) {
-    DDA_TRY_HIP(hipMalloc(&s->t64, vb));
-    DDA_TRY_HIP(hipMalloc(&s->r64, vb));
+    DDA_TRY_HIP(dev_malloc(&s->t64, vb));
+    DDA_TRY_HIP(dev_malloc(&s->r64, vb));
   }
-  DDA_TRY_HIP(hipMalloc(&s->part64, (size_t)k * 4 * nb * sizeof(double)));
-  DDA_TRY_HIP(hipMalloc(&s->scale, k * sizeof(double)));
-  DDA_TRY_HIP(hipMalloc(&s->mask, k * sizeof(int)));
+  DDA_TRY_HIP(dev_malloc(&s->part64, (size_t)k * 4 * nb * sizeof(double)));
+  DDA_TRY_HIP(dev_malloc(&s->scale, k * sizeof(double)));
+  DDA_TRY_HIP(dev_malloc(&s->mask, k * sizeof(int)));
   if (s->mode == DDA_MODE_MIXED) {
-    DDA_TRY_HIP(hipMalloc(&s->x64, vb));
-    DDA_TRY_HIP(hipMalloc(&s->b64, vb));
+    DDA_TRY_HIP(dev_malloc(&s->x64, vb));
+    DDA_TRY_HIP(dev_malloc(&s->b64, vb));
     DDA_TRY(s->c32.alloc(s->op32, s->kind, s->max_iter, s->max_res_increase, k));
   } else if (s->mode == DDA_MODE_FP32) {
     DDA_TRY(s->c32.alloc(op_fp32(s), s->kind, s->max_iter, s->max_res_increase, k));

@@ -456,7 +456,7 @@ dda_status make_twiddles(const int n[3], int prec, void* out[3], hipStream_t st)
       if (t) set(n[a] - t, (double)c, t * 2 == n[a] ? (double)s : -(double)s);
     }
   }
-  DDA_TRY_HIP(hipMalloc(&out[0], h.size()));
+  DDA_TRY_HIP(dev_malloc(&out[0], h.size()));
   for (int a = 1; a < 3; a++) out[a] = (char*)out[0] + off[a];
   DDA_TRY_HIP(copy_sync(out[0], h.data(), h.size(), hipMemcpyHostToDevice, st));
   return DDA_OK;
@@ -939,7 +939,7 @@ static dda_status generate_dhat(dda_op_s* op, int cx, int cy, int cz, void* dst)
   // the double-precision tensor is formed where it stays
   double2* w = oct && op->prec == 64 ? (double2*)dst : nullptr;
   const bool own = w == nullptr;
-  if (own) DDA_TRY_HIP(hipMalloc(&w, (oct ? 6 * cz * plane : total) * sizeof(double2)));
+  if (own) DDA_TRY_HIP(dev_malloc(&w, (oct ? 6 * cz * plane : total) * sizeof(double2)));
   void* tw64[3] = {nullptr, nullptr, nullptr};
   dda_status rc = DDA_OK;
   if (op->prec == 64)
@@ -1096,7 +1096,7 @@ static dda_status cache_get(dda_dhat_cache_s* c, dda_op_s* op, void** out) {
   lk.unlock();
   dda_status rc = DDA_OK;
   void* ptr = nullptr;
-  hipError_t e = hipMalloc(&ptr, bytes);
+  hipError_t e = dev_malloc(&ptr, bytes);
   if (e != hipSuccess) {
     set_error(std::string("tensor cache: hipMalloc failed: ") + hipGetErrorString(e));
     rc = e == hipErrorOutOfMemory ? DDA_OUT_OF_MEMORY : DDA_HIP_ERROR;
@@ -1400,7 +1400,7 @@ static dda_status build_rows(dda_op_s* op) {
   auto upload = [&](uint32_t*& p, const std::vector<uint32_t>& v) -> dda_status {
     if (p) (void)hipFree(p);
     p = nullptr;
-    DDA_TRY_HIP(hipMalloc(&p, std::max<size_t>(1, v.size()) * 4));
+    DDA_TRY_HIP(dev_malloc(&p, std::max<size_t>(1, v.size()) * 4));
     op->device_bytes += v.size() * 4;
     if (!v.empty()) DDA_TRY_HIP(copy_sync(p, v.data(), v.size() * 4, hipMemcpyHostToDevice, st));
     return DDA_OK;
@@ -1419,7 +1419,7 @@ static dda_status build_index(dda_op_s* op, const uint32_t* pos, const dda_op_s*
   hipStream_t st = op->ctx->stream;
   const size_t pb = 12ull * d.nv, ncell = (size_t)d.nrows * d.Bx;
   auto dmalloc = [&](void* p, size_t bytes) -> dda_status {
-    DDA_TRY_HIP(hipMalloc((void**)p, bytes));
+    DDA_TRY_HIP(dev_malloc((void**)p, bytes));
     op->device_bytes += bytes;
     return DDA_OK;
   };
@@ -1579,7 +1579,7 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
   }
 
   auto dmalloc = [&](void** p, size_t bytes) -> dda_status {
-    hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = dev_malloc(p, bytes);
     if (e != hipSuccess) {
       set_error(std::string("dda_op_create: hipMalloc failed: ") + hipGetErrorString(e));
       return e == hipErrorOutOfMemory ? DDA_OUT_OF_MEMORY : DDA_HIP_ERROR;
@@ -1730,7 +1730,7 @@ static dda_status pack_extend(dda_op_s* op, const std::vector<uint8_t>& mats, co
         op->pack.dhat[m] = op->pack.dhat[same];
         continue;
       }
-      DDA_TRY_HIP(hipMalloc(&op->pack.dhat[m], dn * csz));
+      DDA_TRY_HIP(dev_malloc(&op->pack.dhat[m], dn * csz));
       op->device_bytes += dn * csz;
       if (src) {
         hipLaunchKernelGGL(k_narrow, dim3(1024), dim3(256), 0, st, (const double2*)src->pack.dhat[m],
@@ -1749,7 +1749,7 @@ static dda_status pack_extend(dda_op_s* op, const std::vector<uint8_t>& mats, co
   // materials of every member ([nm][nv]) and, for the run-time planned X passes,
   // row metadata; the union is in (z, y, x) order, so row k holds dipole k
   uint8_t* mat_dev = nullptr;
-  DDA_TRY_HIP(hipMalloc(&mat_dev, mats.size()));
+  DDA_TRY_HIP(dev_malloc(&mat_dev, mats.size()));
   (void)hipFree(op->mat_dev);
   op->mat_dev = mat_dev;
   op->device_bytes += (size_t)(nm - 1) * d.nv;
@@ -1760,16 +1760,16 @@ static dda_status pack_extend(dda_op_s* op, const std::vector<uint8_t>& mats, co
       for (int k = 0; k < d.nv; k++)
         meta[(size_t)m * d.nv + k] = op->pos[3 * (size_t)k] | ((uint32_t)mats[(size_t)m * d.nv + k] << 16);
     uint32_t* row_meta = nullptr;
-    DDA_TRY_HIP(hipMalloc(&row_meta, meta.size() * 4));
+    DDA_TRY_HIP(dev_malloc(&row_meta, meta.size() * 4));
     (void)hipFree(op->row_meta);
     op->row_meta = row_meta;
     op->device_bytes += (size_t)(nm - 1) * d.nv * 4;
     DDA_TRY_HIP(copy_sync(row_meta, meta.data(), meta.size() * 4, hipMemcpyHostToDevice, st));
   }
-  DDA_TRY_HIP(hipMalloc(&op->pack.dhat_tab, nm * sizeof(void*)));
+  DDA_TRY_HIP(dev_malloc(&op->pack.dhat_tab, nm * sizeof(void*)));
   DDA_TRY_HIP(copy_sync(op->pack.dhat_tab, op->pack.dhat.data(), nm * sizeof(void*), hipMemcpyHostToDevice, st));
   op->pack.member_host.assign(op->cap_rhs, 0);
-  DDA_TRY_HIP(hipMalloc(&op->pack.member_dev, op->cap_rhs * sizeof(int)));
+  DDA_TRY_HIP(dev_malloc(&op->pack.member_dev, op->cap_rhs * sizeof(int)));
   DDA_TRY_HIP(copy_sync(op->pack.member_dev, op->pack.member_host.data(), op->cap_rhs * sizeof(int),
                         hipMemcpyHostToDevice, st));
   d.member = op->pack.member_dev;
@@ -1976,7 +1976,7 @@ static dda_status ensure_rhs_capacity(dda_op_s* op, int nrhs) {
   size_t b1 = 0, b2 = 0;
   hipError_t e = ctx_alloc(op->ctx, &a1, a1n * csz * nrhs, &b1);
   if (e == hipSuccess) e = ctx_alloc(op->ctx, &a2, a2n * csz * nrhs, &b2);
-  if (e == hipSuccess) e = hipMalloc(&ccs, 3ull * d.nmat * csz * nrhs);
+  if (e == hipSuccess) e = dev_malloc(&ccs, 3ull * d.nmat * csz * nrhs);
   if (e == hipSuccess)
     e = copy_sync(ccs, op->ccs, 3ull * d.nmat * csz * op->cap_rhs, hipMemcpyDeviceToDevice, op->ctx->stream);
   if (e != hipSuccess) {
@@ -1997,7 +1997,7 @@ static dda_status ensure_rhs_capacity(dda_op_s* op, int nrhs) {
   op->ccs = ccs;
   if (op->pack.nmember) {
     int* mem = nullptr;
-    DDA_TRY_HIP(hipMalloc(&mem, nrhs * sizeof(int)));
+    DDA_TRY_HIP(dev_malloc(&mem, nrhs * sizeof(int)));
     op->pack.member_host.resize(nrhs, 0);
     DDA_TRY_HIP(copy_sync(mem, op->pack.member_host.data(), nrhs * sizeof(int), hipMemcpyHostToDevice,
                           op->ctx->stream));
@@ -2096,8 +2096,8 @@ extern "C" dda_status dda_op_apply_host(dda_op_t op, const double* x, double* y,
   const size_t n = 3ull * op->dims.S;
   const size_t csz = op->prec == 64 ? sizeof(double2) : sizeof(float2);
   if (!op->stage_x) {
-    DDA_TRY_HIP(hipMalloc(&op->stage_x, n * csz));
-    DDA_TRY_HIP(hipMalloc(&op->stage_y, n * csz));
+    DDA_TRY_HIP(dev_malloc(&op->stage_x, n * csz));
+    DDA_TRY_HIP(dev_malloc(&op->stage_y, n * csz));
     op->device_bytes += 2 * n * csz;
   }
   hipStream_t st = op->ctx->stream;
@@ -2213,7 +2213,7 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
   dda_op_s::Tune best = op->tune;
   void* xv = nullptr;  // dipole vectors for the X passes
   if (op->static_x) {
-    DDA_TRY_HIP(hipMalloc(&xv, 2 * 3ull * d.S * csz * nrhs));
+    DDA_TRY_HIP(dev_malloc(&xv, 2 * 3ull * d.S * csz * nrhs));
     const hipError_t e = hipMemsetAsync(xv, 0, 2 * 3ull * d.S * csz * nrhs, st);
     if (e != hipSuccess) {
       (void)hipFree(xv);
@@ -2327,7 +2327,7 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
   // two halves on two streams (on the grid buffers as input and output)
   if (nrhs >= 2 && !op->prof) {
     void* xy = nullptr;
-    DDA_TRY_HIP(hipMalloc(&xy, 2 * 3ull * d.S * csz * nrhs));
+    DDA_TRY_HIP(dev_malloc(&xy, 2 * 3ull * d.S * csz * nrhs));
     hipError_t e = hipMemsetAsync(xy, 0, 2 * 3ull * d.S * csz * nrhs, st);
     double ts[2] = {0, 0};
     dda_status rc = e == hipSuccess ? DDA_OK : DDA_HIP_ERROR;

@@ -472,7 +472,7 @@ Frame frame_of(const dda_op_s* op) {
 dda_status positions_on_device(dda_op_s* op) {
   if (op->pos_dev) return DDA_OK;
   const size_t b = op->pos.size() * sizeof(uint32_t);
-  DDA_TRY_HIP(hipMalloc(&op->pos_dev, b));
+  DDA_TRY_HIP(dev_malloc(&op->pos_dev, b));
   op->device_bytes += b;
   DDA_TRY_HIP(hipMemcpyAsync(op->pos_dev, op->pos.data(), b, hipMemcpyHostToDevice, op->ctx->stream));
   DDA_TRY_HIP(hipStreamSynchronize(op->ctx->stream));
@@ -688,10 +688,7 @@ dda_status far_segments(dda_op_s* op) {
   size_t off[7] = {0};
   for (int i = 0; i < 6; i++) off[i + 1] = off[i] + (bytes[i] + 127) / 128 * 128;
   const hipError_t e = ctx_alloc(op->ctx, &op->far_dev, off[6], &op->far_bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    return DDA_OK;
-  }
+  if (e == hipErrorOutOfMemory) return DDA_OK;
   DDA_TRY_HIP(e);
   op->device_bytes += op->far_bytes;
   char* dev = (char*)op->far_dev;
@@ -841,9 +838,7 @@ bool many_directions(const dda_op_s* op, bool angle_grid, long long nq, int used
 // be had, and k_far_partial, which needs less, has to do.
 dda_status far_scratch(dda_op_s* op, size_t bytes, void** out) {
   const dda_status rc = obs_scratch(op, bytes, out);
-  if (rc != DDA_OUT_OF_MEMORY) return rc;
-  (void)hipGetLastError();
-  return DDA_NOT_SUPPORTED;
+  return rc == DDA_OUT_OF_MEMORY ? DDA_NOT_SUPPORTED : rc;
 }
 
 // dda_far_field of many directions; DDA_NOT_SUPPORTED where k_far_partial takes them.
