@@ -17,6 +17,15 @@ using namespace dda;
 
 extern "C" const char* dda_last_error(void) { return g_last_error.c_str(); }
 
+// A stream of different particles makes and destroys operators of similar sizes,
+// and hipFree of a buffer of some ten megabytes takes 100 us and more (the three
+// of a 96 x 72 x 60 box 590 us, allocating them anew 100). Up to kSpareBytes of a
+// context's freed buffers wait for its next operators; work on its stream orders
+// old and new use. Any allocation of the library that finds the memory short gives
+// them back first, those of the other contexts on the device too.
+constexpr size_t kSpareBytes = 1ull << 30;
+constexpr size_t kSpareCount = 64;  // (the list is searched from end to end)
+
 // The contexts alive, for dev_malloc (locked before a context's spare_mu).
 static std::mutex g_ctx_mu;
 static std::vector<dda_ctx_s*> g_ctx;
@@ -36,6 +45,7 @@ extern "C" dda_status dda_ctx_create(int device, dda_ctx_t* out) {
   DDA_TRY_HIP(hipSetDevice(device));
   dda_ctx_s* c = new dda_ctx_s();
   c->device = device;
+  c->spare_limit = kSpareBytes;
   hipError_t e = hipGetDeviceProperties(&c->prop, device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -56,14 +66,6 @@ extern "C" dda_status dda_ctx_create(int device, dda_ctx_t* out) {
   *out = c;
   return DDA_OK;
 }
-
-// A stream of different particles makes and destroys operators of similar sizes,
-// and hipFree of a buffer of some ten megabytes takes 100 us and more (the three
-// of a 96 x 72 x 60 box 590 us, allocating them anew 100). Up to kSpareBytes of a
-// context's freed buffers wait for its next operators; work on its stream orders
-// old and new use. Any allocation of the library that finds the memory short gives
-// them back first, those of the other contexts on the device too.
-constexpr size_t kSpareBytes = 1ull << 30;
 
 static bool free_spares(dda_ctx_s* c) {
   std::lock_guard<std::mutex> lk(c->spare_mu);
@@ -94,7 +96,7 @@ hipError_t dda::dev_malloc(void** p, size_t bytes) {
   return e;
 }
 
-hipError_t dda::ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, size_t* got) {
+hipError_t dda::ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, Held* h) {
   {
     std::lock_guard<std::mutex> lk(c->spare_mu);
     auto best = c->spare.end();
@@ -103,29 +105,37 @@ hipError_t dda::ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, size_t* got) {
         best = it;
     if (best != c->spare.end()) {
       *p = best->ptr;
-      *got = best->bytes;
+      *h = {best->bytes, bytes};
+      c->surplus += h->got - bytes;
       c->spare.erase(best);
       return hipSuccess;
     }
   }
-  *got = bytes;
+  *h = {bytes, bytes};
   return dev_malloc(p, bytes);
 }
 
-void dda::ctx_free(dda_ctx_s* c, void* p, size_t bytes) {
+void dda::ctx_free(dda_ctx_s* c, void* p, const Held& h) {
   if (!p) return;
   std::lock_guard<std::mutex> lk(c->spare_mu);
-  size_t total = bytes;
+  c->surplus -= h.got - h.want;
+  if (h.got + c->surplus > c->spare_limit) {
+    (void)hipFree(p);
+    return;
+  }
+  c->spare.push_back({p, h.got});
+  size_t total = c->surplus;
   for (auto& s : c->spare) total += s.bytes;
-  while (total > kSpareBytes && !c->spare.empty()) {
+  while (total > c->spare_limit || c->spare.size() > kSpareCount) {
     total -= c->spare.front().bytes;
     (void)hipFree(c->spare.front().ptr);
     c->spare.erase(c->spare.begin());
   }
-  if (total > kSpareBytes)
-    (void)hipFree(p);
-  else
-    c->spare.push_back({p, bytes});
+}
+
+void dda::ctx_limit_spare(dda_ctx_s* c, size_t bytes) {
+  std::lock_guard<std::mutex> lk(c->spare_mu);
+  c->spare_limit = std::min(bytes, kSpareBytes);
 }
 
 extern "C" dda_status dda_ctx_destroy(dda_ctx_t ctx) {

@@ -115,17 +115,24 @@ struct dda_ctx_s {
   int device = 0;
   hipStream_t stream = nullptr;
   hipDeviceProp_t prop;
-  // Grid buffers and tensors of destroyed operators, oldest first, for the
-  // context's next ones (ctx_alloc, ctx_free).
+  // Large buffers of destroyed operators, oldest first, for the context's next ones
+  // (ctx_alloc, ctx_free). These and what the buffers in use are larger than asked
+  // for (surplus) stay within spare_limit bytes together.
   struct Spare {
     void* ptr;
     size_t bytes;
   };
   std::mutex spare_mu;
   std::vector<Spare> spare;
+  size_t surplus = 0, spare_limit = 0;
 };
 
 namespace dda {
+// The size of a buffer from ctx_alloc, and the size that was asked for.
+struct Held {
+  size_t got = 0, want = 0;
+};
+
 // Makes the context's device current on the calling thread (handles may be
 // used from any thread, one at a time).
 inline dda_status bind_device(const dda_ctx_s* c) {
@@ -150,11 +157,13 @@ template <typename T> hipError_t dev_malloc(T** p, size_t bytes) {
   return e;
 }
 
-// Large device buffers of a context's operators: a spare one of the size, else
-// dev_malloc. *got is the buffer's size, which ctx_free takes. ctx_free's caller
-// has waited for all work on the buffer but that on the context's stream.
-hipError_t ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, size_t* got);
-void ctx_free(dda_ctx_s* c, void* p, size_t bytes);
+// Large device buffers of a context's operators: a spare one of the size or up to
+// half as large again, else dev_malloc. ctx_free's caller has waited for all work
+// on the buffer but that on the context's stream.
+hipError_t ctx_alloc(dda_ctx_s* c, void** p, size_t bytes, Held* h);
+void ctx_free(dda_ctx_s* c, void* p, const Held& h);
+// At most `bytes` of spare buffers from now on (1 GB at most and by default).
+void ctx_limit_spare(dda_ctx_s* c, size_t bytes);
 }  // namespace dda
 
 struct dda_op_s {
@@ -186,7 +195,7 @@ struct dda_op_s {
   void* dhat = nullptr;           // octant [6][Gz/2+1][Gy/2+1][Gx/2+1] complex R, d^3 scaled
   void* a1 = nullptr;             // [3][Bz][By][Gx]
   void* a2 = nullptr;             // [3][Bz][Gy][Gx]
-  size_t a1_bytes = 0, a2_bytes = 0, dhat_bytes = 0;  // as ctx_alloc gave them
+  dda::Held a1_held, a2_held, dhat_held;  // as ctx_alloc gave them
   bool foreign = false;           // products were launched on streams other than the context's
   void* tw[3] = {nullptr, nullptr, nullptr};
   dda::FftPlan plan[3];
@@ -213,7 +222,7 @@ struct dda_op_s {
     int x_wide[2] = {-1, -1};    // X passes (scatter + forward, inverse + gather)
     int split = -1;              // a block as two half-blocks on two streams: -1 default (off), 0 off, 1 on
   } tune;
-  bool tuned = false;
+  bool tuned = false;  // dda_op_tune ran (an FP32 twin of a tuned operator is tuned too)
   // the tuning for blocks of kBlockTuneRhs or more right-hand sides (used when
   // tuned_blk; else `tune` serves every block size)
   Tune tune_blk;
@@ -241,9 +250,9 @@ struct dda_op_s {
     std::vector<int2> start;  // copy of wave_seg where the records are made in groups
   } far;
   void* far_dev = nullptr;      // used on the context's stream alone
-  size_t far_bytes = 0;
+  dda::Held far_held;
   void* obs_scratch = nullptr;  // observables' work space
-  size_t obs_bytes = 0;  // dda_op_tune ran (an FP32 twin of a tuned operator is tuned too)
+  dda::Held obs_held;
   bool static_x = false;  // X passes with a compile-time plan (Gx has one)
   const dda::AxisOps* gen[3] = {nullptr, nullptr, nullptr};  // the axes whose length has a general plan
   int cap_rhs = 1;   // right-hand sides the grid buffers hold

@@ -1257,12 +1257,10 @@ dda_status dda::host_positions(dda_op_s* op) {
 }
 
 // Buffers that other streams may still use are freed, which waits for them.
-static void release_large(dda_op_s* op, void* p, size_t bytes) {
+static void release_large(dda_op_s* op, void* p, const Held& h) {
   if (!p) return;
-  if (op->foreign)
-    (void)hipFree(p);
-  else
-    ctx_free(op->ctx, p, bytes);
+  if (op->foreign) (void)hipDeviceSynchronize();
+  ctx_free(op->ctx, p, h);
 }
 
 static void free_op(dda_op_s* op) {
@@ -1296,11 +1294,11 @@ static void free_op(dda_op_s* op) {
   void* bufs[] = {op->cell, op->active_list, op->yrange, op->row_start, op->row_dip, op->row_meta, op->row_list, op->mat_dev, op->ccs, op->tw[0], op->stage_x, op->stage_y, op->pos_dev};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
-  release_large(op, op->a1, op->a1_bytes);
-  release_large(op, op->a2, op->a2_bytes);
-  release_large(op, op->dhat, op->dhat_bytes);
-  ctx_free(op->ctx, op->far_dev, op->far_bytes);
-  ctx_free(op->ctx, op->obs_scratch, op->obs_bytes);
+  release_large(op, op->a1, op->a1_held);
+  release_large(op, op->a2, op->a2_held);
+  release_large(op, op->dhat, op->dhat_held);
+  ctx_free(op->ctx, op->far_dev, op->far_held);
+  ctx_free(op->ctx, op->obs_scratch, op->obs_held);
   delete op;
 }
 
@@ -1587,13 +1585,13 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
     op->device_bytes += bytes;
     return DDA_OK;
   };
-  auto large = [&](void** p, size_t bytes, size_t* got) -> dda_status {
-    const hipError_t e = ctx_alloc(ctx, p, bytes, got);
+  auto large = [&](void** p, size_t bytes, Held* h) -> dda_status {
+    const hipError_t e = ctx_alloc(ctx, p, bytes, h);
     if (e != hipSuccess) {
       set_error(std::string("dda_op_create: hipMalloc failed: ") + hipGetErrorString(e));
       return e == hipErrorOutOfMemory ? DDA_OUT_OF_MEMORY : DDA_HIP_ERROR;
     }
-    op->device_bytes += bytes;
+    op->device_bytes += h->got;
     return DDA_OK;
   };
   const size_t a1n = 3ull * d.Bz * d.By * d.rs;
@@ -1601,9 +1599,9 @@ static dda_status create_op(dda_ctx_t ctx, const dda_op_desc* desc, int precisio
   const size_t dn = 6ull * (d.Gx / 2 + 1) * (d.Gy / 2 + 1) * (d.Gz / 2 + 1);
   dda_status rc = DDA_OK;
   if (rc == DDA_OK) rc = dmalloc(&op->ccs, 3ull * ds.nmat * csz);
-  if (rc == DDA_OK && (ds.dmatrix || !cache)) rc = large(&op->dhat, dn * csz, &op->dhat_bytes);
-  if (rc == DDA_OK) rc = large(&op->a1, a1n * csz, &op->a1_bytes);
-  if (rc == DDA_OK) rc = large(&op->a2, a2n * csz, &op->a2_bytes);
+  if (rc == DDA_OK && (ds.dmatrix || !cache)) rc = large(&op->dhat, dn * csz, &op->dhat_held);
+  if (rc == DDA_OK) rc = large(&op->a1, a1n * csz, &op->a1_held);
+  if (rc == DDA_OK) rc = large(&op->a2, a2n * csz, &op->a2_held);
   if (rc == DDA_OK) {
     const int n[3] = {d.Gx, d.Gy, d.Gz};
     rc = make_twiddles(n, precision, op->tw, ctx->stream);
@@ -1973,7 +1971,7 @@ static dda_status ensure_rhs_capacity(dda_op_s* op, int nrhs) {
   const size_t csz = op->prec == 64 ? sizeof(double2) : sizeof(float2);
   const size_t a1n = 3ull * d.Bz * d.By * d.rs, a2n = 3ull * d.Bz * d.p2;
   void *a1 = nullptr, *a2 = nullptr, *ccs = nullptr;
-  size_t b1 = 0, b2 = 0;
+  Held b1, b2;
   hipError_t e = ctx_alloc(op->ctx, &a1, a1n * csz * nrhs, &b1);
   if (e == hipSuccess) e = ctx_alloc(op->ctx, &a2, a2n * csz * nrhs, &b2);
   if (e == hipSuccess) e = dev_malloc(&ccs, 3ull * d.nmat * csz * nrhs);
@@ -1986,14 +1984,14 @@ static dda_status ensure_rhs_capacity(dda_op_s* op, int nrhs) {
     set_error(std::string("grid buffers for a batch: ") + hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? DDA_OUT_OF_MEMORY : DDA_HIP_ERROR;
   }
-  op->device_bytes += (a1n + a2n + 3ull * d.nmat) * csz * (nrhs - op->cap_rhs);
-  release_large(op, op->a1, op->a1_bytes);
-  release_large(op, op->a2, op->a2_bytes);
+  op->device_bytes += b1.got + b2.got - op->a1_held.got - op->a2_held.got + 3ull * d.nmat * csz * (nrhs - op->cap_rhs);
+  release_large(op, op->a1, op->a1_held);
+  release_large(op, op->a2, op->a2_held);
   (void)hipFree(op->ccs);
   op->a1 = a1;
   op->a2 = a2;
-  op->a1_bytes = b1;
-  op->a2_bytes = b2;
+  op->a1_held = b1;
+  op->a2_held = b2;
   op->ccs = ccs;
   if (op->pack.nmember) {
     int* mem = nullptr;

@@ -483,18 +483,18 @@ dda_status positions_on_device(dda_op_s* op) {
 // hipMalloc of some megabytes takes 300 us: the context's spare buffers serve a
 // new operator's first call).
 dda_status obs_scratch(dda_op_s* op, size_t bytes, void** out) {
-  if (op->obs_bytes < bytes) {
+  if (op->obs_held.got < bytes) {
     if (op->obs_scratch) {
       DDA_TRY_HIP(hipStreamSynchronize(op->ctx->stream));
-      ctx_free(op->ctx, op->obs_scratch, op->obs_bytes);
-      op->device_bytes -= op->obs_bytes;
+      ctx_free(op->ctx, op->obs_scratch, op->obs_held);
+      op->device_bytes -= op->obs_held.got;
       op->obs_scratch = nullptr;
-      op->obs_bytes = 0;
+      op->obs_held = Held();
     }
-    size_t got = 0;
-    DDA_TRY_HIP(ctx_alloc(op->ctx, &op->obs_scratch, bytes, &got));
-    op->obs_bytes = got;
-    op->device_bytes += got;
+    Held h;
+    DDA_TRY_HIP(ctx_alloc(op->ctx, &op->obs_scratch, bytes, &h));
+    op->obs_held = h;
+    op->device_bytes += h.got;
   }
   *out = op->obs_scratch;
   return DDA_OK;
@@ -687,10 +687,10 @@ dda_status far_segments(dda_op_s* op) {
                            nocc * sizeof(int2), (nocc + 1ull) * sizeof(int2), 3 * sizeof(int)};
   size_t off[7] = {0};
   for (int i = 0; i < 6; i++) off[i + 1] = off[i] + (bytes[i] + 127) / 128 * 128;
-  const hipError_t e = ctx_alloc(op->ctx, &op->far_dev, off[6], &op->far_bytes);
+  const hipError_t e = ctx_alloc(op->ctx, &op->far_dev, off[6], &op->far_held);
   if (e == hipErrorOutOfMemory) return DDA_OK;
   DDA_TRY_HIP(e);
-  op->device_bytes += op->far_bytes;
+  op->device_bytes += op->far_held.got;
   char* dev = (char*)op->far_dev;
   m.pair = (int2*)dev;
   m.segs = (FarSeg*)(dev + off[1]);
@@ -713,8 +713,8 @@ dda_status far_segments(dda_op_s* op) {
     if (le == hipSuccess) le = hipStreamSynchronize(st);
   }
   if (le != hipSuccess || info[0] <= 0 || info[2]) {
-    ctx_free(op->ctx, op->far_dev, op->far_bytes);
-    op->device_bytes -= op->far_bytes;
+    ctx_free(op->ctx, op->far_dev, op->far_held);
+    op->device_bytes -= op->far_held.got;
     op->far_dev = nullptr;
     far.made = le == hipSuccess;
     DDA_TRY_HIP(le);

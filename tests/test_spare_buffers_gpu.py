@@ -160,3 +160,48 @@ def test_products_on_a_callers_stream():
     for v in x + y:
         v.close()
     own.close()
+
+
+def _device_bytes(op):
+    n = ctypes.c_size_t()
+    assert D.lib().dda_op_info(op.handle, None, None, ctypes.byref(n)) == D.OK
+    return n.value
+
+
+def _free():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert D.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_a_larger_buffer_counts_as_it_is():
+    fresh, own = D.Context(0), D.Context(0)
+    op, _ = _operator(fresh, (96, 96, 80))
+    alone = _device_bytes(op)
+    op.close()
+    _operator(own, BOX)[0].close()  # its buffers are a fifth larger
+    op, _ = _operator(own, (96, 96, 80))
+    assert 1.15 * alone <= _device_bytes(op) <= 1.25 * alone
+    op.close()
+    own.close()
+    fresh.close()
+
+
+def test_spare_buffers_stay_within_a_gigabyte():
+    """One operator of more than that, then eight of 340 MB that are destroyed
+    together; all of it is given back with the context."""
+    own = D.Context(0)
+    before = _free()
+    small, _ = _operator(own, (40, 40, 40))
+    small.close()
+    kept = _free()
+    big, _ = _operator(own, (128, 128, 128), nrhs=2)  # grid buffers of 1.2 GB and 600 MB
+    big.close()
+    assert before - _free() <= (1 << 30) + (64 << 20)
+    ops = [_operator(own, BOX)[0] for _ in range(8)]
+    assert before - _free() >= 8 * (300 << 20)
+    for op in ops:
+        op.close()
+    assert before - _free() <= (1 << 30) + (64 << 20)
+    own.close()
+    assert _free() >= kept - (64 << 20)
