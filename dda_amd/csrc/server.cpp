@@ -26,6 +26,7 @@
 namespace dda {
 void set_error(const std::string& msg);  // api.hip: the message dda_last_error returns
 bool last_tensor_cache_hit();            // matvec.hip: this thread's last cached-tensor lookup hit
+void ctx_limit_spare(dda_ctx_s* c, size_t bytes);  // api.hip: spare buffers a context may keep
 double tensor_cache_seconds();           // matvec.hip: this thread's seconds in tensor-cache lookups
 }
 
@@ -82,6 +83,7 @@ struct dda_server_s {
   std::chrono::steady_clock::time_point t0;
   std::mutex mu;
   std::condition_variable cv_work, cv_done;
+  size_t slot_spare = 0;  // bytes of spare buffers that a slot's context may keep
   std::deque<Job*> queue;
   std::map<uint64_t, std::unique_ptr<Job>> jobs;
   uint64_t next_id = 1, submitted = 0, completed = 0;
@@ -91,19 +93,31 @@ struct dda_server_s {
 
   double now() const { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); }
 
+  // Device bytes of an operator of this geometry with k right-hand sides: the
+  // grid buffers, whose rows are whole 128-byte lines with one line more to a plane
+  // of the second, twiddles and couple constants, and the index arrays (positions,
+  // materials, cell map, two lists of rows and the planes' ranges; the dipoles
+  // by row where some share a cell). The tensor is counted by the cache.
+  static size_t op_bytes(const Job& j, int prec, int k) {
+    const size_t csz = prec / 4, line = 128 / csz;
+    const size_t rows = (size_t)j.box[1] * j.box[2], rs = (j.grid[0] + line - 1) / line * line;
+    const size_t a = 3 * rows * rs + 3ull * j.box[2] * (j.grid[1] * rs + line);
+    const size_t tw = ((size_t)j.grid[0] + j.grid[1] + j.grid[2]) * csz + 384;
+    return k * (a + 3ull * j.nmat) * csz + tw + 21ull * j.nv + 4ull * j.box[0] * rows + 12 * rows + 4 + 8ull * j.box[2];
+  }
+
   // Device bytes a block solve of k right-hand sides of this geometry holds
-  // (grid buffers of the operator and its FP32 twin, Krylov vectors, FP64
-  // refinement vectors, index arrays); the tensor is counted by the cache.
+  // (the operator and its FP32 twin, Krylov vectors and the partial sums of their
+  // products, FP64 refinement vectors).
   size_t footprint(const Job& j, int k) const {
-    const size_t n = 3ull * j.stride;
-    const size_t a = 3ull * j.box[2] * j.box[1] * j.grid[0] + 3ull * j.box[2] * j.grid[1] * j.grid[0];
+    const size_t n = 3ull * j.stride, sums = 96ull * j.box[1] * j.box[2];
     const bool lanczos = cfg.solver_kind == DDA_SOLVER_QMR_CS || cfg.solver_kind == DDA_SOLVER_BICG_CS;
-    size_t b = 13ull * j.nv + 4ull * j.box[1] * j.box[2] + (size_t)k * a * 16;
+    size_t b = op_bytes(j, 64, k);
     if (cfg.mode == DDA_MODE_MIXED) {
-      b += (size_t)k * (a * 8 + 8 * n * 8 + 6 * n * 16);
-      if (lanczos) b += (size_t)k * 8 * n * 16;  // FP64 inner fallback
+      b += op_bytes(j, 32, k) + (size_t)k * (8 * n * 8 + 6 * n * 16 + sums);
+      if (lanczos) b += (size_t)k * (8 * n * 16 + sums);  // FP64 inner fallback
     } else {
-      b += (size_t)k * (8 * n * 16 + 4 * n * 16);
+      b += (size_t)k * (8 * n * 16 + 4 * n * 16 + sums);
     }
     return b;
   }
@@ -119,6 +133,7 @@ struct dda_server_s {
         u.grid[a] = p->grid[a];
       }
       u.nv += p->nv;
+      u.nmat = std::max(u.nmat, p->nmat + 1);
     }
     u.stride = (u.nv + 15) / 16 * 16;
     return footprint(u, k) + parts.size() * 5 * u.nv;
@@ -303,6 +318,7 @@ void dda_server_s::worker(int slot) {
   (void)slot;
   dda_ctx_t ctx = nullptr;  // each slot: its own stream, its device bound on this thread
   if (dda_ctx_create(cfg.device, &ctx) != DDA_OK) ctx = nullptr;
+  if (ctx) dda::ctx_limit_spare(ctx, slot_spare);
   for (;;) {
     std::vector<Job*> pack;
     size_t foot = 0;
@@ -401,6 +417,9 @@ extern "C" dda_status dda_server_create(const dda_server_config* cfg, dda_server
   const size_t budget = cfg->hbm_budget ? cfg->hbm_budget : hbm / 10 * 9;
   const size_t cache_bytes = cfg->cache_bytes ? cfg->cache_bytes : budget / 4;
   s->job_budget = budget > cache_bytes ? budget - cache_bytes : budget / 2;
+  // what the slots' contexts keep between jobs is part of the budget
+  s->slot_spare = std::min<size_t>(1ull << 30, s->job_budget / 8 / cfg->slots);
+  s->job_budget -= s->slot_spare * cfg->slots;
   rc = dda_dhat_cache_create(s->ctx0, cache_bytes, &s->cache);
   if (rc != DDA_OK) {
     dda_ctx_destroy(s->ctx0);

@@ -59,7 +59,10 @@ typedef struct dda_dhat_cache_s* dda_dhat_cache_t;
 /* Message of the last failed call on this thread ("" if none). */
 const char* dda_last_error(void);
 
-/* Context: one GPU and one in-order stream (DDA/DDAMain.cpp:556-575). */
+/* Context: one GPU and one in-order stream (DDA/DDAMain.cpp:556-575). It keeps up
+ * to 1 GB of its destroyed operators' buffers for the next ones (the job server's
+ * contexts: less, within hbm_budget) until an allocation of the library finds the
+ * GPU's memory short or the context is destroyed. */
 dda_status dda_ctx_create(int device, dda_ctx_t* out);
 dda_status dda_ctx_destroy(dda_ctx_t ctx);
 dda_status dda_ctx_synchronize(dda_ctx_t ctx);
@@ -405,7 +408,8 @@ typedef struct dda_server_s* dda_server_t;
 typedef struct dda_server_config {
   int device;          /* GPU */
   int slots;           /* concurrent block solves, 1..16, each on its own stream */
-  size_t hbm_budget;   /* bytes for admitted jobs plus the tensor cache (0 = 90% of HBM) */
+  size_t hbm_budget;   /* bytes for admitted jobs, the tensor cache and what the slots' contexts
+                          keep between jobs (0 = 90% of HBM) */
   size_t cache_bytes;  /* tensor cache limit, part of hbm_budget (0 = a quarter of it) */
   int solver_kind;     /* dda_solver_kind */
   int mode;            /* dda_solver_mode */
