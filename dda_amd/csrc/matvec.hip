@@ -2286,14 +2286,17 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
       }
       t[w] = it < nvar ? tt : std::min(t[w], tt);
     }
-    // the precision's default unless another variant is faster by more than
-    // 2% (closer timings change places between runs)
-    // (the X passes default to the narrow plan in both precisions)
-    const int def = pass == 1 && d.Gz >= 512 && sizeof(R) == 4 ? 2 : pass < 3 && sizeof(R) == 4 ? 1 : 0;
+    // the untuned rule's variant unless another is faster by more than 2% (closer
+    // timings change places between runs): -1, so that the rule goes on to
+    // decide for each block size that these choices serve
+    const int nb = 3 * d.Bz * std::min(nrhs, 65535 / (3 * d.Bz));
+    const int def = pass == 1                                ? default_p3_variant(d, op->prec, nrhs)
+                    : pass >= 3 || op->prec == 64            ? 0
+                                                             : default_col_variant(d.Gy, d.Gx, nb);
     int fastest = 0;
     for (int w = 1; w < nvar; w++)
       if (t[w] < t[fastest]) fastest = w;
-    const int pick = t[fastest] < 0.98 * t[def] ? fastest : def;
+    const int pick = t[fastest] < 0.98 * t[def] ? fastest : -1;
     if (pass == 1)
       best.p3_wide = pick;
     else if (pass >= 3)
@@ -2312,7 +2315,7 @@ dda_status tune_impl(dda_op_s* op, int nrhs, std::string* report) {
       std::snprintf(buf, sizeof buf, ", %s %.1f us", vnames[w], t[w]);
       *report += buf;
     }
-    std::snprintf(buf, sizeof buf, " -> %s", vnames[pick]);
+    std::snprintf(buf, sizeof buf, " -> %s", vnames[pick < 0 ? def : pick]);
     *report += buf;
     op->tune = best;
   }

@@ -562,11 +562,10 @@ dda_status launch_col_static_w(const void* in, void* out, const ColParams& cp, c
 // work-groups 16 columns are as fast or faster, at 192 and 256 points always (by
 // up to 7%). At 512 points the narrow plan, which has three stages like the wide
 // one and half its registers: 442 and 418 us against 476 and 435 at 512^3.
-template <int N>
-inline int default_col_variant(int ncols, int nbatch) {
-  if (N == 512) return 0;
-  if (N > 128 || ncols % 64 || (long long)(ncols / 64) * nbatch < 6144) return 1;
-  return N >= 48 ? 5 : 3;
+inline int default_col_variant(int n, int ncols, int nbatch) {
+  if (n == 512) return 0;
+  if (n > 128 || ncols % 64 || (long long)(ncols / 64) * nbatch < 6144) return 1;
+  return n >= 48 ? 5 : 3;
 }
 
 // wide: -1 the precision's default plan, 0 narrow, 1 wide; FP32 also 2 and 3,
@@ -576,7 +575,7 @@ template <typename R, int N, bool INV>
 dda_status launch_col_static(const void* in, void* out, const ColParams& cp, const void* tw, int nbatch, hipStream_t st,
                              RhsFlags done, int wide) {
   if constexpr (sizeof(R) == 4) {
-    if (wide < 0) wide = default_col_variant<N>(cp.ncols, nbatch);
+    if (wide < 0) wide = default_col_variant(N, cp.ncols, nbatch);
     if (wide >= 4)
       return (wide & 1) ? launch_col_static_w<R, N, true, INV, 2>(in, out, cp, tw, nbatch, st, done)
                         : launch_col_static_w<R, N, false, INV, 2>(in, out, cp, tw, nbatch, st, done);
@@ -686,21 +685,26 @@ template <> struct Plan32<512> : PlanOf<512, 32, RadixList<32, 16>, TW_SPLIT> {}
 // FP32 below 1024 points: 2 and 3 are the narrow and wide plans with the
 // other tile (other_cols_z).
 inline int p3_variants(int n, int prec) { return prec == 32 ? 4 : 2; }
+// The variant of an untuned Z pass.
+inline int default_p3_variant(const MvDims& d, int prec, int nrhs) {
+  if (prec == 64) return 0;
+  return d.Gz >= 512 ? 2 : d.Gz <= 64 && wide_z_tile(d, nrhs) ? 3 : 1;
+}
 
 template <typename R, int N>
 dda_status launch_pass3_static(dda_op_s* op, const MvView& v, hipStream_t st, RhsFlags done, int nrhs,
                                const dda_op_s::Tune& tn) {
-  const int var = tn.p3_wide;
+  const int var = tn.p3_wide < 0 ? default_p3_variant(v.d, 8 * (int)sizeof(R), nrhs) : tn.p3_wide;
   if constexpr (N >= 512 && sizeof(R) == 4) {
-    if (var == 2 || var < 0) return launch_pass3_plan<R, N, Plan32<N>, 16>(op, v, st, done, nrhs);
+    if (var == 2) return launch_pass3_plan<R, N, Plan32<N>, 16>(op, v, st, done, nrhs);
     if (var == 3) return launch_pass3_plan<R, N, Plan32<N>, 8>(op, v, st, done, nrhs);
   } else if constexpr (sizeof(R) == 4) {
-    if (var >= 2 || (N <= 64 && var < 0 && wide_z_tile(v.d, nrhs)))
+    if (var >= 2)
       return (var & 1) ? launch_pass3_static_w<R, N, true, true>(op, v, st, done, nrhs)
                        : launch_pass3_static_w<R, N, false, true>(op, v, st, done, nrhs);
   }
-  return plan_wide<R>(var >= 2 ? (var & 1) : var) ? launch_pass3_static_w<R, N, true>(op, v, st, done, nrhs)
-                           : launch_pass3_static_w<R, N, false>(op, v, st, done, nrhs);
+  return (var & 1) ? launch_pass3_static_w<R, N, true>(op, v, st, done, nrhs)
+                   : launch_pass3_static_w<R, N, false>(op, v, st, done, nrhs);
 }
 
 template <typename R, int N, typename PL, int BS = 256>

@@ -183,13 +183,14 @@ dda_status dda_op_apply_batch(dda_op_t op, const void* x_dev, void* y_dev, int n
 /* Autotuner (no counterpart in the reference, whose FFT plans are fixed per
  * length): times each variant of the column passes (plan width: 8 or 16
  * points per thread; in FP32 every pass also with another tile, i.e.
- * another number of columns or lines per work-group, and 1024-point Z columns
- * with the 32 x 32 plan over 16 or 8 columns) on this operator's own buffers for nrhs
- * right-hand sides, each twice (the faster timing counts), and keeps per pass
- * the fastest where it beats the precision's default by more than 2% (the
- * default otherwise). nrhs >= 2 tunes a separate set for blocks of right-hand
- * sides (matvecs of blocks use it; single right-hand sides, the set of
- * nrhs = 1). The choices are cached for the process by (grid, box,
+ * another number of columns or lines per work-group, and Z columns of 512 and
+ * 1024 points with plans of 32 points per thread over 16 or 8 columns; axes of
+ * other lengths have one plan) on this operator's own buffers for nrhs right-hand
+ * sides, each twice (the faster timing counts), and keeps per pass the fastest
+ * where it beats the one that an untuned operator runs by more than 2% (else the
+ * pass stays at -1, the untuned rule). nrhs >= 2 tunes a separate set for blocks
+ * of right-hand sides (matvecs of blocks use it; single right-hand sides, the
+ * set of nrhs = 1). The choices are cached for the process by (grid, box,
  * precision, block or not), so later operators of that shape start tuned. A
  * solver over a tuned operator tunes the operator its iterations run on (the
  * FP32 twin in the mixed and FP32 modes) for one right-hand side at creation
@@ -199,14 +200,12 @@ dda_status dda_op_apply_batch(dda_op_t op, const void* x_dev, void* y_dev, int n
  * `report` (nullable) receives a one-line summary of the timings. */
 dda_status dda_op_tune(dda_op_t op, int nrhs, char* report, size_t report_len);
 /* The kernel variant of each pass, in the tuner's order: Y forward, Z with
- * the tensor product, Y inverse, X forward, X inverse; -1 = the precision's
- * default, 0 = narrow plan, 1 = wide plan; in FP32 every pass also takes 2
- * and 3 (narrow and wide with the other tile), except the Z pass of a
- * 1024-point grid, where 2 and 3 are the 32 x 32 plan over 16 or 8 columns;
- * the Y passes also 4 and 5 (a third tile, four times the default columns
- * where they fit).
- * Entry 5:
- * a block of right-hand sides as two half-blocks on two streams (-1 default
+ * the tensor product, Y inverse, X forward, X inverse; -1 = the default for the
+ * precision, the grid and the block size, 0 = narrow plan, 1 = wide plan; in FP32
+ * every pass also takes 2 and 3 (narrow and wide with the other tile), except the
+ * Z pass of a 512- or 1024-point grid, where 2 and 3 are plans of 32 points per
+ * thread over 16 or 8 columns; the Y passes also 4 and 5 (a third tile, four times
+ * the default columns where they fit). Entry 5: a block of right-hand sides as two half-blocks on two streams (-1 default
  * = off, 0 off, 1 on). Getting reads the set used for single right-hand sides;
  * setting pins the variants for every block size (e.g. a stored tuning, or a
  * parity test of one variant); values a pass does not have run as its
