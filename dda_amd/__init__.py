@@ -204,7 +204,8 @@ def fft_fit(x, override=0, support_non_pot=True):
 
 def grid_plan(grid, precision):
     """(static_x, static_z): whether an operator on `grid` runs the X passes and
-    the Z pass on compile-time planned kernels (host-only query)."""
+    the Z pass on kernels with tuned variants (host-only query; the other even
+    7-smooth lengths from 8 to 512 have one compile-time plan each)."""
     g = (ctypes.c_uint32 * 3)(*[int(v) for v in grid])
     sx, sz = ctypes.c_int(), ctypes.c_int()
     _check(lib().dda_grid_plan(g, int(precision), ctypes.byref(sx), ctypes.byref(sz)), "dda_grid_plan")

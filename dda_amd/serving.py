@@ -89,7 +89,7 @@ def make_stream(n, seed, rate=None, label=None):
 
 def submit(server, job, grid=(0, 0, 0)):
     """Submits a job; grid 0 lets the server pick per axis the smallest length
-    with compile-time planned kernels (dda_fft_fit_static)."""
+    whose kernels have tuned variants (dda_fft_fit_static)."""
     g = job.geometry
     return server.submit(g.pos, g.mat, g.box, g.grid_unit, job.params.wave_num, job.einc, job.cc_sqrt,
                          nmat=len(g.materials), grid=grid)

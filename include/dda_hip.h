@@ -79,21 +79,25 @@ dda_status dda_memcpy_d2d(dda_ctx_t ctx, void* dst, const void* src, size_t byte
 /* FFT grid size for a box extent of x dipoles: fftFit, DDA/DDAParams.cpp:45-90.
  * x is 2*box; override != 0 returns override (0 if it is smaller than x). */
 uint32_t dda_fft_fit(uint32_t x, uint32_t override_, int support_non_pot);
-/* The smallest length >= x that has compile-time planned kernels (32, 48, 64,
- * 96, 128, 192, 256, 512, 1024), else dda_fft_fit's smooth rule: the faster
- * grid for a box extent of x/2 (any grid of at least twice the box gives the
- * same product, to rounding). The job server uses it for jobs without a grid;
- * the reference's GPU path likewise rounds to powers of two. */
+/* The smallest length >= x whose kernels have tuned variants (32, 48, 64, 96,
+ * 128, 192, 256, 512, 1024), else dda_fft_fit's smooth rule. The job server uses it
+ * for jobs without a grid, so that particles of near sizes share a grid and its
+ * tensor. Any grid of at least twice the box gives the same product, to rounding,
+ * and every even length of the smooth rule from 8 to 512 has compile-time planned
+ * kernels, so the smooth rule's grid, being smaller, is the faster one: two FP32
+ * right-hand sides take 39 us on 70^3 and 49 on 96^3, 111 us on 140^3 and 183 on
+ * 192^3, 1.09 ms on 270^3 and 3.83 on 512^3. */
 uint32_t dda_fft_fit_static(uint32_t x);
 
-/* Which passes of an operator on `grid` run compile-time planned kernels (no
+/* Which passes of an operator on `grid` run kernels with tuned variants (no
  * counterpart in the reference, whose FFT plans are chosen at run time,
- * DDA/GpuFFTPlans.cpp:34-61): static_x for the X passes (Gx has a static
- * plan), static_z for the Z pass with the tensor product (Gz has one and every
+ * DDA/GpuFFTPlans.cpp:34-61): static_x for the X passes (Gx is one of the lengths
+ * above), static_z for the Z pass with the tensor product (Gz is one and every
  * byte offset of that pass fits 32 bits: the tensor octant's components, and as
  * many planes of the grid as the pass has threads per column, Gz/8 at most, each
- * below 4 GiB). Other grids use the run-time
- * planned kernels. Host-only. */
+ * below 4 GiB). The other even lengths 2^a 3^b 5^c 7^d from 8 to 512 have one
+ * compile-time plan each, under the same condition in the Z pass, and lengths
+ * beyond, or whose offsets do not fit, the run-time planned kernels. Host-only. */
 dda_status dda_grid_plan(const uint32_t grid[3], int precision, int* static_x, int* static_z);
 
 /* Operator description: the parts of DDAParams/DipoleGeometry the matvec reads
