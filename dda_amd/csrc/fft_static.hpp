@@ -20,26 +20,48 @@
 namespace dda {
 
 // ------------------------------------------------------------------------------------
-// Compile-time cos/sin(2 pi v / M) by exact octant reduction of v/M and a Taylor
-// series on [0, pi/4].
+// The roots of unity of the in-register DFTs, at compile time: cos and sin(2 pi t / n)
+// by exact octant reduction of t / n and Taylor series on [0, pi / 4], in sums of
+// two doubles (the error-free sum and product of Knuth and Dekker), so that each is
+// the closest double. (In plain double half of them came out a unit or two in the
+// last place off, cos(2 pi / 3) among them, which made the FP64 products at
+// lengths of the factors 3 and 4 up to 1.4 times as far from the exact ones.)
 // ------------------------------------------------------------------------------------
-constexpr double kPiD = 3.14159265358979323846264338327950288;
-
-constexpr double taylor_sin(double x) {
-  double term = x, sum = x;
-  for (int n = 1; n < 14; n++) {
-    term *= -x * x / ((2 * n) * (2 * n + 1));
-    sum += term;
-  }
-  return sum;
+struct TwoDoubles {
+  double hi, lo;
+};
+constexpr TwoDoubles two_sum(double a, double b) {
+  const double s = a + b, t = s - a;
+  return {s, (a - (s - t)) + (b - t)};
 }
-constexpr double taylor_cos(double x) {
-  double term = 1, sum = 1;
-  for (int n = 1; n < 14; n++) {
-    term *= -x * x / ((2 * n - 1) * (2 * n));
-    sum += term;
+constexpr TwoDoubles two_prod(double a, double b) {
+  const double k = 134217729.0;  // 2^27 + 1
+  const double p = a * b, ca = k * a, cb = k * b;
+  const double ah = ca - (ca - a), al = a - ah, bh = cb - (cb - b), bl = b - bh;
+  return {p, ((ah * bh - p) + ah * bl + al * bh) + al * bl};
+}
+constexpr TwoDoubles add2(TwoDoubles a, TwoDoubles b) {
+  const TwoDoubles s = two_sum(a.hi, b.hi);
+  return two_sum(s.hi, s.lo + a.lo + b.lo);
+}
+constexpr TwoDoubles mul2(TwoDoubles a, TwoDoubles b) {
+  const TwoDoubles p = two_prod(a.hi, b.hi);
+  return two_sum(p.hi, p.lo + a.hi * b.lo + a.lo * b.hi);
+}
+constexpr TwoDoubles div2(TwoDoubles a, double d) {
+  const double q = a.hi / d;
+  const TwoDoubles p = two_prod(q, d);
+  return two_sum(q, ((a.hi - p.hi) - p.lo + a.lo) / d);
+}
+// cos x (first = 0) or sin x (first = 1): x^m / m!, m = first, first + 2, ..
+constexpr double taylor(TwoDoubles x, int first) {
+  TwoDoubles term = first ? x : TwoDoubles{1, 0}, sum = term;
+  const TwoDoubles x2 = mul2(x, x);
+  for (int m = first + 2; m < 30; m += 2) {
+    term = div2(mul2(term, x2), -(double)(m * (m - 1)));
+    sum = add2(sum, term);
   }
-  return sum;
+  return sum.hi;
 }
 // cos(2 pi t / n) (which = 0) or sin(2 pi t / n) (which = 1)
 constexpr double cexpr_trig(long long t, long long n, int which) {
@@ -59,15 +81,26 @@ constexpr double cexpr_trig(long long t, long long n, int which) {
     v = M / 4 - v;
     swap = true;
   }
-  const double x = 2 * kPiD * (double)v / (double)M;
-  double s = taylor_sin(x), c = taylor_cos(x);
-  if (swap) {
-    double tmp = s;
-    s = c;
-    c = tmp;
-  }
+  const TwoDoubles pi = {3.141592653589793116, 1.2246467991473531772e-16};
+  const TwoDoubles x = div2(mul2(pi, {(double)(2 * v), 0}), (double)M);
+  const double s = taylor(x, swap ? 0 : 1), c = taylor(x, swap ? 1 : 0);
   return which ? sgn_s * s : sgn_c * c;
 }
+template <int N> struct RootsOfUnity {
+  double cos[N] = {}, sin[N] = {};
+  constexpr RootsOfUnity() {
+    for (int t = 0; t < N; t++) {
+      cos[t] = cexpr_trig(t, N, 0);
+      sin[t] = cexpr_trig(t, N, 1);
+    }
+  }
+};
+template <int N> constexpr RootsOfUnity<N> kRoots{};
+static_assert(kRoots<3>.cos[1] == -0.5 && kRoots<12>.sin[1] == 0.5 && kRoots<3>.sin[1] == 0.86602540378443864676 &&
+                  kRoots<8>.cos[1] == 0.70710678118654752440 && kRoots<7>.cos[1] == 0.62348980185873353053 &&
+                  kRoots<9>.sin[2] == 0.98480775301220805937 && kRoots<16>.cos[3] == 0.38268343236508977173 &&
+                  kRoots<27>.sin[13] == 0.11609291412523022967 && kRoots<25>.cos[12] == -0.99211470131447783105,
+              "roots of unity to the last place");
 
 // ------------------------------------------------------------------------------------
 // In-register DFT of length R (forward exp(-2 pi i jk/R) unless INV).
@@ -87,16 +120,16 @@ template <int R, bool INV, typename C> struct RDft;
 // a * W_R^k (W_R = exp(-2 pi i / R), conjugated when INV). k and R are
 // constants once the calling loops are unrolled, so the branches fold away and
 // multiples of a quarter turn become swaps and sign changes.
-template <bool INV, typename C>
-__device__ __forceinline__ C cmul_w(C a, int k, int R) {
+template <int R, bool INV, typename C>
+__device__ __forceinline__ C cmul_w(C a, int k) {
   typedef decltype(C().x) F;
-  k = ((k % R) + R) % R;
+  k = k % R;
   if (k == 0) return a;
   if (2 * k == R) return cmake<C>(-a.x, -a.y);
   if (4 * k == R) return INV ? cmul_pi(a) : cmul_mi(a);
   if (4 * k == 3 * R) return INV ? cmul_mi(a) : cmul_pi(a);
-  const F c = (F)cexpr_trig(k, R, 0);
-  const F s = (F)cexpr_trig(k, R, 1);
+  const F c = (F)kRoots<R>.cos[k];
+  const F s = (F)kRoots<R>.sin[k];
   return cmul(a, cmake<C>(c, INV ? s : -s));
 }
 
@@ -142,8 +175,8 @@ template <int R, bool INV, typename C> struct RDftOdd {
       C sn = czero<C>();
 #pragma unroll
       for (int m = 1; m <= H; m++) {
-        const F cv = (F)cexpr_trig(m * k, R, 0);
-        const F sv = (F)cexpr_trig(m * k, R, 1);
+        const F cv = (F)kRoots<R>.cos[m * k % R];
+        const F sv = (F)kRoots<R>.sin[m * k % R];
         cs.x += cv * s[m].x;
         cs.y += cv * s[m].y;
         sn.x += sv * d[m].x;
@@ -178,7 +211,7 @@ template <int R, bool INV, typename C> struct RDft {
       for (int p = 0; p < P; p++) t[p] = a[q + Q * p];
       RDft<P, INV, C>::run(t);
 #pragma unroll
-      for (int k1 = 0; k1 < P; k1++) b[q + Q * k1] = cmul_w<INV>(t[k1], q * k1, R);
+      for (int k1 = 0; k1 < P; k1++) b[q + Q * k1] = cmul_w<R, INV>(t[k1], q * k1);
     }
 #pragma unroll
     for (int k1 = 0; k1 < P; k1++) {
@@ -202,7 +235,7 @@ template <int R, bool INV, typename C> struct RDftHalfIn {
 #pragma unroll
     for (int m = 0; m < H; m++) {
       e[m] = a[m];
-      o[m] = cmul_w<INV>(a[m], m, R);
+      o[m] = cmul_w<R, INV>(a[m], m);
     }
     RDft<H, INV, C>::run(e);
     RDft<H, INV, C>::run(o);
