@@ -258,8 +258,8 @@ template <int R, bool INV, typename C> struct RDftHalfIn {
 // General plans take TW_SPLIT: their radices go up to 28, whose chained powers
 // made the FP64 product at 80^3 2.1e-16 and the FP32 one at 96 x 70 x 120 9.9e-8
 // from the exact one, against 1.6e-16 and 8.1e-8 with run-time planned radices up
-// to 8; with TW_SPLIT it is 1.7e-16 and 6.5e-8, over 22 boxes of 8 to 250 cells
-// a side 0.97 (FP64) and 0.87 (FP32) of the run-time planned kernels' error.
+// to 8; with TW_SPLIT it is 1.5e-16 and 6.5e-8, over 150 grids of all general
+// lengths 0.93 (FP64) and 0.82 (FP32) of the run-time planned kernels' error.
 // Loading every power (FP64) gave no smaller error and took 22% longer at
 // 180 x 144 x 120. TW_SPLIT in the plans of the powers of two halves the FP32
 // error at 512^3 but makes their products 2 to 9% slower.
