@@ -119,13 +119,15 @@ void dda::ctx_free(dda_ctx_s* c, void* p, const Held& h) {
   if (!p) return;
   std::lock_guard<std::mutex> lk(c->spare_mu);
   c->surplus -= h.got - h.want;
-  if (h.got + c->surplus > c->spare_limit) {
+  size_t total = c->surplus + h.got;
+  for (auto& s : c->spare) total += s.bytes;
+  // beyond the limit a buffer that was too large for its use goes before those
+  // that fit theirs
+  if (h.got + c->surplus > c->spare_limit || (total > c->spare_limit && h.got > h.want)) {
     (void)hipFree(p);
     return;
   }
   c->spare.push_back({p, h.got});
-  size_t total = c->surplus;
-  for (auto& s : c->spare) total += s.bytes;
   while (total > c->spare_limit || c->spare.size() > kSpareCount) {
     total -= c->spare.front().bytes;
     (void)hipFree(c->spare.front().ptr);

@@ -205,3 +205,24 @@ def test_spare_buffers_stay_within_a_gigabyte():
     assert before - _free() <= (1 << 30) + (64 << 20)
     own.close()
     assert _free() >= kept - (64 << 20)
+
+
+def test_buffers_that_fit_outlast_those_too_large():
+    """A large block's buffers first serve smaller operators, whose own set then
+    fits the limit: once it is made, destroying and making such an operator again
+    frees nothing (a hipFree of the buffers takes most of a millisecond)."""
+    own = D.Context(0)
+    op, _ = _operator(own, (64, 48, 32), 32, nrhs=128)  # grid buffers of 300 and 600 MB
+    op.close()
+    for _ in range(3):
+        op, _ = _operator(own, (128, 128, 128), 32, nrhs=2)  # 100, 200, 200, 400 and 100 MB
+        op.close()
+    kept = _free()
+    for _ in range(3):
+        op, _ = _operator(own, (128, 128, 128), 32, nrhs=2)
+        # positions, materials and cell map, 17 bytes a cell of the full box, in pages of
+        # 2 MB, and small arrays: no grid buffer (100 MB and more) was taken anew
+        assert kept - _free() <= 17 * op.nv + (16 << 20)
+        op.close()
+        assert abs(kept - _free()) <= 16 << 20
+    own.close()
